@@ -161,3 +161,47 @@ def tolerance(case):
     if "bf16" in (case["out"], case["dtype"] if case["path"] in ("layer", "scan") else ""):
         return {"rel": 7e-3}
     return {"rel": 1e-3 if case["out"] == "fp16" else 1e-5}
+
+
+def exact(case, seed):
+    """What run returns, computed chunk by chunk in 64 bits."""
+    s = prepare(case, seed)
+    b, L, H, P, N, G, Q = (case[k] for k in "bLHPNGQ")
+    C, dev = -(-L // Q), s["x"].device
+    A, seq = s["A"].double(), s["seq"]
+    if case["path"] == "layer":
+        raw = s["dt_raw"].double() + s["bias"].double()
+        dt = torch.nn.functional.pad(torch.nn.functional.softplus(raw, threshold=1e9), (0, 0, 0, C * Q - L))
+        dt = dt.view(b, C, Q, H).permute(0, 3, 1, 2).contiguous()
+        dA = torch.cumsum(dt * A.view(1, H, 1, 1), dim=-1)
+    else:
+        dt, dA = s["dt"].double(), s["dA"].double()
+    heads = lambda t: t.double().repeat_interleave(H // G, dim=2).transpose(1, 2).contiguous()  # noqa: E731  (b,k,G,N) -> (b,H,k,N)
+    state = torch.zeros(b, H, P, N, device=dev, dtype=torch.float64) if s["init"] is None else s["init"].double()
+    states = torch.empty(b, C, H, P, N, device=dev, dtype=torch.float64) if case["path"] == "unfused" else None
+    out = torch.empty(b, C, H, P, N, device=dev, dtype=torch.float64) if case["path"] != "scan" else None
+    y = torch.empty(b, L, H, P, device=dev, dtype=torch.float64) if "C" in s else None
+    before = torch.zeros(b, device=dev, dtype=torch.int32)          # sequence of the token in front of the chunk
+    for c in range(C):
+        t0, t1 = c * Q, min((c + 1) * Q, L)
+        ids = torch.zeros(b, t1 - t0, device=dev, dtype=torch.int32) if seq is None else seq[:, t0:t1]
+        last = ids[:, -1]
+        w = torch.exp(torch.clamp(dA[:, :, c, -1:] - dA[:, :, c, :t1 - t0], max=0.0)) * dt[:, :, c, :t1 - t0]
+        w = w * (ids == last[:, None])[:, None]
+        xw = (s["x"][:, t0:t1].double().permute(0, 2, 3, 1) * w[:, :, None]).contiguous()
+        chunk = torch.matmul(xw, heads(s["B"][:, t0:t1]))
+        if out is not None:
+            out[:, c] = state
+        if states is not None:
+            states[:, c] = chunk
+        if y is not None:
+            scale = torch.exp(dA[:, :, c, :t1 - t0]) * (ids == before[:, None])[:, None]
+            cy = torch.matmul(heads(s["C"][:, t0:t1]), state.transpose(-1, -2).contiguous())
+            y[:, t0:t1] = (cy * scale[..., None]).transpose(1, 2)
+        keep = torch.exp(dA[:, :, c, -1]) * (last == before)[:, None]
+        state, before = keep[..., None, None] * state + chunk, last
+    if case["path"] == "layer":
+        return dA, dt, out, state, y
+    if case["path"] == "unfused":
+        return states, out.flatten(-2), state.flatten(-2)
+    return (state, y) if case["path"] == "scan" else (out, state)
