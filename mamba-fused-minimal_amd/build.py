@@ -10,6 +10,7 @@ import sys
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "libssd_gfx950.so")
+HOST = os.path.join(HERE, "_ssd_host.so")
 OBJ_DIR = os.path.join(HERE, "build")
 SOURCES = ["ssd_capi.hip", "ssd_mfma.hip", "ssd_quad.hip", "ssd_chain.hip", "ssd_generic.hip", "ssd_state_passing.hip", "ssd_chunk_cumsum.hip", "ssd_chunk_scan_states.hip", "ssd_mover.hip", "ssd_chain_scan.hip"]
 FLAGS = [
@@ -56,6 +57,23 @@ def _resource_usage(asm_text):
                             "Dynamic Stack": "True" if f.get("uses_dynamic_stack") == "true" else "False",
                             "Occupancy [waves/SIMD]": occupancy.get(f["name"], 0)}
     return usage
+
+
+def build_host():
+    """Compiles the Python extension module that hands tensors to the library (host code only, no GPU code in it)."""
+    import sysconfig
+    import torch
+    torch_dir = os.path.dirname(torch.__file__)
+    cxx = shutil.which("g++") or shutil.which("c++")
+    if cxx is None:
+        raise RuntimeError("no C++ compiler found")
+    cmd = [cxx, "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+           "-isystem", os.path.join(torch_dir, "include"), "-isystem", os.path.join(torch_dir, "include", "torch", "csrc", "api", "include"),
+           "-I", sysconfig.get_paths()["include"], os.path.join(CSRC, "ssd_host.cpp"), "-o", HOST,
+           f"-L{HERE}", "-l:libssd_gfx950.so", "-Wl,-rpath,$ORIGIN",
+           f"-L{os.path.join(torch_dir, 'lib')}", "-ltorch_python", "-ltorch_cpu", "-lc10", f"-Wl,-rpath,{os.path.join(torch_dir, 'lib')}"]
+    _run(cmd)
+    return HOST
 
 
 def build_library(verbose=False, extra_flags=(), jobs=None):
@@ -109,6 +127,7 @@ def build_library(verbose=False, extra_flags=(), jobs=None):
         raise RuntimeError(f"the compiler moved operands that inline assembly is still loading in {sorted(bad)} "
                            f"({sum(len(v) for v in bad.values())} places, e.g. {first}); see {ISA_CHECK}")
     out = _run([hipcc(), "--offload-arch=gfx950", "-shared", "-fPIC", *[o for o, _ in results], "-o", LIB])
+    build_host()
     for src, (_, text) in zip(SOURCES, results):
         if verbose and text.strip():
             print(text)

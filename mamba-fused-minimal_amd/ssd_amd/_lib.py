@@ -2,12 +2,14 @@
 
 There is no fallback: if the library is missing, or the tensors are not on a gfx950 device, the calls raise."""
 import ctypes
+import importlib.util
 import os
 
 import torch
 
 _PKG_ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 LIB_PATH = os.path.join(_PKG_ROOT, "libssd_gfx950.so")
+HOST_PATH = os.path.join(_PKG_ROOT, "_ssd_host.so")
 
 SSD_F32, SSD_BF16, SSD_F16 = 0, 1, 2
 _DTYPES = {torch.float32: SSD_F32, torch.bfloat16: SSD_BF16, torch.float16: SSD_F16}
@@ -109,6 +111,23 @@ def load():
     lib.ssd_set_segment_chunks.argtypes = [ctypes.c_int]
     _lib = lib
     return lib
+
+
+_host = None
+
+
+def host():
+    """The extension module that hands tensors to the library's entry points (csrc/ssd_host.cpp), loaded once."""
+    global _host
+    if _host is None:
+        load()
+        if not os.path.exists(HOST_PATH):
+            raise ImportError(f"{HOST_PATH} is missing: build it with `python {os.path.join(_PKG_ROOT, 'build.py')}`")
+        spec = importlib.util.spec_from_file_location("_ssd_host", HOST_PATH)
+        module = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(module)
+        _host = module
+    return _host
 
 
 def tensor_arg(t):

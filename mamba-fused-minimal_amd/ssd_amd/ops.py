@@ -8,6 +8,7 @@ Same names, positional order, defaults, shape asserts and output shapes/dtypes a
 of the reference.  The wrappers own allocation and argument checking; the arithmetic runs in the gfx950 HIP
 kernels behind the C ABI of libssd_gfx950.so, asynchronously on the current torch stream."""
 import ctypes
+import functools
 import math
 import threading
 
@@ -18,6 +19,20 @@ from . import _lib
 
 def _stream(t):
     return ctypes.c_void_p(torch.cuda.current_stream(t.device).cuda_stream)
+
+
+# The current stream's handle without a torch.cuda.Stream object around it, and no device guard where the tensors' device
+# is the current one: together a quarter of what a wrapper costs.
+_raw_stream = torch._C._cuda_getCurrentRawStream
+
+
+def _on_device(t, call, *args):
+    """call(*args, stream handle) with t's device current."""
+    index = t.device.index
+    if index == torch.cuda.current_device():
+        return call(*args, _raw_stream(index))
+    with torch.cuda.device(index):
+        return call(*args, _raw_stream(index))
 
 
 # Workspaces of the ticket / flag-chain kernel that the wrappers keep to themselves: one per (device, stream), grown on
@@ -69,13 +84,29 @@ def _workspace_key(device, stream=None):
     return (device.index if device.index is not None else torch.cuda.current_device(), stream.cuda_stream)
 
 
+@functools.lru_cache(maxsize=1024)
+def _fused_workspace_need(device, sizes, out_code, chunks_per_item, pairs_only):
+    """Bytes of workspace for a fused call of these sizes: a question about sizes only, asked once.  0 = that kernel is not
+    offered for these arguments, its plain workspace then."""
+    lib = _lib.load()
+    dims = _lib.dims_arg(*sizes)
+    nbytes = 0 if pairs_only else int(lib.ssd_fused_workspace_bytes_for(dims, out_code, chunks_per_item))
+    return nbytes or int(lib.ssd_fused_workspace_bytes(dims))
+
+
+@functools.lru_cache(maxsize=1024)
+def _fused_scan_workspace_need(device, sizes, with_out, chunks_per_item):
+    return int(_lib.load().ssd_fused_scan_workspace_bytes(_lib.dims_arg(*sizes), with_out, chunks_per_item))
+
+
 def _own_workspace(x, nbytes):
     """-> the _Kept of x's device and current stream, holding at least nbytes (None under stream capture)."""
     if torch.cuda.is_current_stream_capturing():
         # a captured launch is replayed with the same arguments: the same epoch again and again would take the flags of
         # the replay before for its own.  Epoch 0 (clear every time) is what a graph needs.
         return None
-    key = _workspace_key(x.device)
+    index = x.device.index
+    key = (index, _raw_stream(index))
     with _WORKSPACES_LOCK:
         ent = _WORKSPACES.get(key)
         if ent is None or ent.tensor.numel() * 4 < nbytes:
@@ -92,17 +123,17 @@ def release_workspaces():
         _WORKSPACES.clear()
 
 
-def _launch_on_own_workspace(x, nbytes, launch, used, pairs):
-    """Runs launch(workspace, epoch) -> status on the wrappers' workspace for x's device and stream.  pairs: the
+def _launch_on_own_workspace(x, nbytes, launch, pairs):
+    """Runs launch(workspace, epoch) -> (status, used) on the wrappers' workspace for x's device and stream.  pairs: the
     (state tile, chunk) pairs of the call, i.e. the flags it looks at.  Only launches on the same device and stream
     wait for each other here."""
     ent = _own_workspace(x, nbytes)
     if ent is None:
-        return launch(torch.empty(((nbytes + 3) // 4,), device=x.device, dtype=torch.int32), 0)
+        return launch(torch.empty(((nbytes + 3) // 4,), device=x.device, dtype=torch.int32), 0)[0]
     with ent.lock:
         epoch = ent.epochs.next(pairs)
-        rc = launch(ent.tensor, epoch)
-        ent.epochs.done(epoch, rc, used.value, pairs)
+        rc, used = launch(ent.tensor, epoch)
+        ent.epochs.done(epoch, rc, used, pairs)
         return rc
 
 
@@ -160,16 +191,11 @@ def _chunk_state_impl(B, x, dt, dA_cumsum, seq_idx, states, states_in_fp32, _cla
     if states is not None:
         assert states.shape == (batch, nchunks, nheads, headdim, dstate)
     _lib.require_device(x, "_chunk_state_fwd")
-    lib = _lib.load()
     if states is None:
         states_dtype = torch.float32 if states_in_fp32 else B.dtype
         states = torch.empty((batch, nchunks, nheads, headdim, dstate), device=x.device, dtype=states_dtype)
     B, x, dt, dA_cumsum, seq_idx = _prep_inputs(B, x, dt, dA_cumsum, seq_idx)
-    dims = _lib.dims_arg(batch, seqlen, nheads, headdim, dstate, ngroups, chunk_size, nchunks)
-    with torch.cuda.device(x.device):
-        rc = lib.ssd_chunk_state_fwd(_lib.tensor_arg(x), _lib.tensor_arg(B), _lib.tensor_arg(dt),
-                                     _lib.tensor_arg(dA_cumsum), _lib.tensor_arg(seq_idx), _lib.tensor_arg(states),
-                                     dims, 1 if _clamp else 0, _stream(x))
+    rc = _on_device(x, _lib.host().chunk_state, x, B, dt, dA_cumsum, seq_idx, states, 1 if _clamp else 0)
     _lib.check(rc, "ssd_chunk_state_fwd")
     return states
 
@@ -186,7 +212,6 @@ def _state_passing_fwd(states, dA_chunk_cumsum, initial_states=None, seq_idx=Non
         seqlen = seq_idx.shape[-1]
         assert seq_idx.shape == (batch, seqlen)
     _lib.require_device(states, "_state_passing_fwd")
-    lib = _lib.load()
     out_dtype = states.dtype if out_dtype is None else out_dtype
     out = torch.empty((batch, nchunks, nheads, dim), device=states.device, dtype=out_dtype)
     final_states = torch.empty((batch, nheads, dim), device=states.device, dtype=torch.float32)
@@ -198,12 +223,8 @@ def _state_passing_fwd(states, dA_chunk_cumsum, initial_states=None, seq_idx=Non
         initial_states = initial_states.contiguous()
     if seq_idx is not None and seq_idx.dtype != torch.int32:
         seq_idx = seq_idx.to(torch.int32)
-    with torch.cuda.device(states.device):
-        rc = lib.ssd_state_passing_fwd(_lib.tensor_arg(states), _lib.tensor_arg(dA_chunk_cumsum),
-                                       _lib.tensor_arg(initial_states), _lib.tensor_arg(seq_idx),
-                                       _lib.tensor_arg(out), _lib.tensor_arg(final_states),
-                                       batch, nchunks, nheads, dim, seqlen,
-                                       chunk_size if seq_idx is not None else 0, _stream(states))
+    rc = _on_device(states, _lib.host().state_passing, states, dA_chunk_cumsum, initial_states, seq_idx, out, final_states, seqlen,
+                    chunk_size if seq_idx is not None else 0)
     _lib.check(rc, "ssd_state_passing_fwd")
     return out, final_states
 
@@ -244,37 +265,26 @@ def _fused_chunk_state_state_passing_fwd(B, x, dt, dA_cumsum, out_dtype, initial
         assert initial_states.shape == (batch, nheads, headdim, dstate)
     assert chunk_size is not None
     _lib.require_device(x, "_fused_chunk_state_state_passing_fwd")
-    lib = _lib.load()
     out_dtype = states_dtype if out_dtype is None else out_dtype
     out = torch.empty((batch, nchunks, nheads, headdim, dstate), device=x.device, dtype=out_dtype)
     final_states = torch.empty((batch, nheads, headdim, dstate), device=x.device, dtype=torch.float32)
     B, x, dt, dA_cumsum, seq_idx = _prep_inputs(B, x, dt, dA_cumsum, seq_idx)
     if initial_states is not None and initial_states.stride(-1) != 1:
         initial_states = initial_states.contiguous()
-    dims = _lib.dims_arg(batch, seqlen, nheads, headdim, dstate, ngroups, chunk_size, nchunks)
-
-    used = ctypes.c_int32(0)
 
     def launch(workspace, epoch):
-        opts = _lib.SsdFusedOpts(workspace.data_ptr(), workspace.numel() * 4, int(_spin_limit), int(_kernel),
-                                 int(_chunks_per_item), int(epoch), ctypes.pointer(used))
-        with torch.cuda.device(x.device):
-            return lib.ssd_fused_chunk_state_passing_fwd_ws(
-                _lib.tensor_arg(x), _lib.tensor_arg(B), _lib.tensor_arg(dt), _lib.tensor_arg(dA_cumsum),
-                _lib.tensor_arg(seq_idx), _lib.tensor_arg(initial_states), _lib.tensor_arg(states),
-                _lib.tensor_arg(out), _lib.tensor_arg(final_states), dims, 1 if _clamp else 0, ctypes.byref(opts),
-                _stream(x))
+        return _on_device(x, _lib.host().fused, x, B, dt, dA_cumsum, seq_idx, initial_states, states, out, final_states,
+                          1 if _clamp else 0, workspace.data_ptr(), workspace.numel() * 4, int(_spin_limit), int(_kernel),
+                          int(_chunks_per_item), int(epoch))
 
     if _workspace is not None:
-        rc = launch(_workspace, _epoch)
+        rc = launch(_workspace, _epoch)[0]
     else:
         # bf16 passed states: the workspace also takes the fp32 states that cross between work items (a quarter of
-        # an fp32 `out`, as a rule); 0 = that kernel is not offered for these arguments
-        nbytes = 0
-        if states is None:          # with a `states` buffer the call runs on other kernels anyway
-            nbytes = int(lib.ssd_fused_workspace_bytes_for(dims, _lib._DTYPES.get(out_dtype, -1), int(_chunks_per_item)))
-        rc = _launch_on_own_workspace(x, nbytes or int(lib.ssd_fused_workspace_bytes(dims)), launch, used,
-                                      batch * nheads * ((headdim + 31) // 32) * nchunks)
+        # an fp32 `out`, as a rule); with a `states` buffer the call runs on other kernels anyway
+        nbytes = _fused_workspace_need(x.device.index, (batch, seqlen, nheads, headdim, dstate, ngroups, chunk_size, nchunks),
+                                       _lib._DTYPES.get(out_dtype, -1), int(_chunks_per_item), states is not None)
+        rc = _launch_on_own_workspace(x, nbytes, launch, batch * nheads * ((headdim + 31) // 32) * nchunks)
     _lib.check(rc, "ssd_fused_chunk_state_passing_fwd_ws")
     return out, final_states
 
@@ -364,12 +374,8 @@ def _chunk_cumsum_fwd(dt, A, chunk_size, dt_bias=None, dt_softplus=False, dt_lim
     nchunks = math.ceil(seqlen / chunk_size)
     dt_out = torch.empty(batch, nheads, nchunks, chunk_size, device=dt.device, dtype=torch.float32)
     dA_cumsum = torch.empty(batch, nheads, nchunks, chunk_size, device=dt.device, dtype=torch.float32)
-    lib = _lib.load()
-    with torch.cuda.device(dt.device):
-        rc = lib.ssd_chunk_cumsum_fwd(_lib.tensor_arg(dt), _lib.tensor_arg(A), _lib.tensor_arg(dt_bias),
-                                      _lib.tensor_arg(dt_out), _lib.tensor_arg(dA_cumsum), batch, seqlen, nheads,
-                                      int(chunk_size), int(bool(dt_softplus)), float(dt_limit[0]), float(dt_limit[1]),
-                                      _stream(dt))
+    rc = _on_device(dt, _lib.host().chunk_cumsum, dt, A, dt_bias, dt_out, dA_cumsum, int(chunk_size), int(bool(dt_softplus)),
+                    float(dt_limit[0]), float(dt_limit[1]))
     _lib.check(rc, "ssd_chunk_cumsum_fwd")
     return dA_cumsum, dt_out
 
@@ -420,16 +426,17 @@ def _fused_cumsum_chunk_state_state_passing_fwd(B, x, dt, A, chunk_size, out_dty
         opts = _lib.SsdFusedOpts(workspace.data_ptr(), workspace.numel() * 4, 0, int(_kernel), int(_chunks_per_item), int(epoch),
                                  ctypes.pointer(used))
         with torch.cuda.device(x.device):
-            return lib.ssd_fused_cumsum_chunk_state_passing_fwd_ws(
+            rc = lib.ssd_fused_cumsum_chunk_state_passing_fwd_ws(
                 T(x), T(B), T(dt), T(A), T(dt_bias), T(seq_idx), T(initial_states), T(dt_out), T(dA_cumsum), T(out),
                 T(final_states), dims, int(bool(dt_softplus)), float(dt_limit[0]), float(dt_limit[1]), 1 if _clamp else 0,
                 ctypes.byref(opts), _stream(x))
+        return rc, used.value
 
     if _workspace is not None:
-        rc = launch(_workspace, 0)
+        rc = launch(_workspace, 0)[0]
     else:
         nbytes = int(lib.ssd_fused_workspace_bytes_for(dims, _lib._DTYPES.get(out.dtype, -1), int(_chunks_per_item)))
-        rc = _launch_on_own_workspace(x, nbytes or int(lib.ssd_fused_workspace_bytes(dims)), launch, used,
+        rc = _launch_on_own_workspace(x, nbytes or int(lib.ssd_fused_workspace_bytes(dims)), launch,
                                       batch * nheads * ((headdim + 31) // 32) * nchunks)
     _lib.check(rc, "ssd_fused_cumsum_chunk_state_passing_fwd_ws")
     return out, final_states, dA_cumsum, dt_out
@@ -467,11 +474,7 @@ def _chunk_scan_states_fwd(C, prev_states, dA_cumsum, seq_idx=None, out=None, ou
         prev_states = prev_states.contiguous()
     if dA_cumsum.dtype != torch.float32:
         dA_cumsum = dA_cumsum.float()
-    dims = _lib.dims_arg(batch, seqlen, nheads, headdim, dstate, ngroups, chunk_size, nchunks)
-    with torch.cuda.device(C.device):
-        rc = _lib.load().ssd_chunk_scan_states_fwd(_lib.tensor_arg(C), _lib.tensor_arg(prev_states),
-                                                   _lib.tensor_arg(dA_cumsum), _lib.tensor_arg(seq_idx),
-                                                   _lib.tensor_arg(out), dims, int(bool(accumulate)), _stream(C))
+    rc = _on_device(C, _lib.host().chunk_scan_states, C, prev_states, dA_cumsum, seq_idx, out, int(bool(accumulate)))
     _lib.check(rc, "ssd_chunk_scan_states_fwd")
     return out
 
@@ -500,7 +503,6 @@ def _fused_chunk_state_state_passing_scan_fwd(B, x, C, dt, dA_cumsum, out_dtype=
     if initial_states is not None:
         assert initial_states.shape == (batch, nheads, headdim, dstate)
     _lib.require_device(x, "_fused_chunk_state_state_passing_scan_fwd")
-    lib = _lib.load()
     if y is None:
         assert not accumulate, "accumulate=True needs the tensor to add to (y=)"
         y = torch.empty(batch, seqlen, nheads, headdim, device=x.device, dtype=y_dtype or C.dtype)
@@ -512,24 +514,19 @@ def _fused_chunk_state_state_passing_scan_fwd(B, x, C, dt, dA_cumsum, out_dtype=
     if initial_states is not None and initial_states.stride(-1) != 1:
         initial_states = initial_states.contiguous()
     final_states = torch.empty((batch, nheads, headdim, dstate), device=x.device, dtype=torch.float32)
-    dims = _lib.dims_arg(batch, seqlen, nheads, headdim, dstate, ngroups, chunk_size, nchunks)
-    T = _lib.tensor_arg
+    sizes = (batch, seqlen, nheads, headdim, dstate, ngroups, chunk_size, nchunks)
     pairs = batch * nheads * ((headdim + 31) // 32) * nchunks
-    used = ctypes.c_int32(0)
 
     def call(out):
         def launch(workspace, epoch):
-            opts = _lib.SsdFusedOpts(workspace.data_ptr(), workspace.numel() * 4, int(_spin_limit), int(_kernel),
-                                     int(_chunks_per_item), int(epoch), ctypes.pointer(used))
-            with torch.cuda.device(x.device):
-                return lib.ssd_fused_chunk_state_passing_scan_fwd(
-                    T(x), T(B), T(C), T(dt), T(dA_cumsum), T(seq_idx), T(initial_states), T(out), T(final_states), T(y),
-                    dims, 1 if _clamp else 0, int(bool(accumulate)), ctypes.byref(opts), _stream(x))
+            return _on_device(x, _lib.host().fused_scan, x, B, C, dt, dA_cumsum, seq_idx, initial_states, out, final_states, y,
+                              1 if _clamp else 0, int(bool(accumulate)), workspace.data_ptr(), workspace.numel() * 4,
+                              int(_spin_limit), int(_kernel), int(_chunks_per_item), int(epoch))
 
         if _workspace is not None:
-            return launch(_workspace, _epoch)
-        nbytes = int(lib.ssd_fused_scan_workspace_bytes(dims, 1 if out is not None else 0, int(_chunks_per_item)))
-        return _launch_on_own_workspace(x, nbytes, launch, used, pairs)
+            return launch(_workspace, _epoch)[0]
+        nbytes = _fused_scan_workspace_need(x.device.index, sizes, 1 if out is not None else 0, int(_chunks_per_item))
+        return _launch_on_own_workspace(x, nbytes, launch, pairs)
 
     out = None
     if return_states:
