@@ -116,9 +116,10 @@ int ssd_state_passing_fwd(const ssd_tensor *states, const ssd_tensor *dA_chunk, 
  * per-chunk states"; otherwise they are written as a side effect exactly as ssd_chunk_state_fwd would.
  * With few state tiles (batch * nheads * headdim / 32 below 512) and many chunks the call runs as a chunk-state launch
  * that keeps every compute unit busy plus a streaming recurrence; that needs a place for the chunk states: a fp32
- * `out` serves as one (the recurrence then works in place), and so does a fp32 `states` buffer.  With a 16-bit `out`
+ * `out` serves as one (the recurrence then works in place), and so does a fp32 `states` buffer.  The same holds for few
+ * tiles and four or more chunks, where that pair also goes in front of the kernel that takes a workspace.  With a 16-bit `out`
  * and no `states` such a problem stays on the kernel with one workgroup per tile, which is slower (the library never
- * allocates): a caller in that position gains by passing `states`.  Arguments that only the plain FMA kernel takes
+ * allocates): a caller in that position gains by passing `states`.  Arguments that only the fp32 matrix kernel takes
  * (fp32 or fp16 x / B, sizes off the MFMA tiling) run as the same two launches from two chunks upwards, given a fp32
  * `out` or a fp32 `states`.
  */
@@ -243,7 +244,7 @@ int ssd_fused_static_status(void *stream);
 
 /*
  * Which kernel family the three calls above would pick for these arguments: 1 = bf16 MFMA path,
- * 0 = generic FMA path (other element types or shapes the MFMA tiling does not cover), negative = rejected.
+ * 0 = generic fp32 path (other element types or shapes the MFMA tiling does not cover), negative = rejected.
  * Pure host logic; launches nothing.
  */
 int ssd_query_path(const ssd_tensor *x, const ssd_tensor *B, const ssd_dims *dims);

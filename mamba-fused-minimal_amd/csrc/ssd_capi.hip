@@ -120,8 +120,9 @@ PassParams pass_params_of(const Params &p)
     return q;
 }
 
-// Fused call with `states`: can it run as the chunk-state launch of the four-tile kernel + the recurrence?
-bool pair_supported(const Params &p)
+// Fused call with `states`: can it run as the chunk-state launch of the four-tile kernel (or, where the launch is small
+// anyway, the token-split one's) + the recurrence?
+bool pair_supported(const Params &p, bool small = false)
 {
     if (!p.states || !p.out || !p.fin) return false;
     if (p.dt_states != ssd::DT_F32) return false;      // the recurrence would start from rounded states
@@ -129,16 +130,7 @@ bool pair_supported(const Params &p)
     if (p.sst_p != p.dstate || p.so_p != p.dstate || p.sf_p != p.dstate || (p.init && p.sin_p != p.dstate)) return false;
     Params cs = p;
     cs.out = nullptr; cs.fin = nullptr; cs.init = nullptr;
-    return ssd::quad_chunk_state_supported(cs);
-}
-
-// chunk states into p.states, then the recurrence over them into p.out / p.fin (which may be the same buffer)
-hipError_t launch_pair(const Params &p, hipStream_t s, bool generic = false)
-{
-    Params cs = p;
-    cs.out = nullptr; cs.fin = nullptr; cs.init = nullptr;
-    const hipError_t e = generic ? ssd::launch_generic(cs, false, s) : ssd::launch_quad_chunk_state(cs, s);
-    return e == hipSuccess ? ssd::launch_state_passing(pass_params_of(p), s) : e;
+    return ssd::quad_chunk_state_supported(cs) || (small && ssd::mfma_supported(cs));
 }
 
 // The same for arguments only the fp32 matrix kernel takes (other element types, odd sizes): as a fused launch that
@@ -169,7 +161,18 @@ struct Choice {
     int family;
     bool states_in_out;      // chunk-state launch + recurrence: `out` doubles as the place for the chunk states
     bool generic_pair;       // F_GENERIC as chunk-state launch + recurrence
+    bool few;                // F_PAIR because of few units, in front of the chain kernel too
 };
+
+// The fused problem as the cost model sees it.
+ssd::cost::Problem problem_of(const Params &p, int64_t n_cu)
+{
+    ssd::cost::Problem q;
+    q.units = (int64_t)p.batch * p.nheads * (p.headdim / 32) / 4;
+    q.chunks = p.C; q.chunk_size = p.Q; q.dstate = p.dstate;
+    q.n_cu = n_cu > 0 ? (int)n_cu : 256;
+    return q;
+}
 
 // The kernel family of a call without a workspace.
 Choice choose(const Params &p, bool fused, int64_t n_cu)
@@ -179,25 +182,41 @@ Choice choose(const Params &p, bool fused, int64_t n_cu)
     // kernel, which puts four waves on every tile, has the shorter chunk.
     const int tiles = p.batch * p.nheads * (p.headdim / 32);
     const int forced = g_forced_split.load(std::memory_order_relaxed);      // one value for the whole choice
-    if (fused && (forced == 1 || (forced == 0 && tiles >= 2 * n_cu)) && ssd::quad_supported(p)) return {F_FOUR_TILE, false, false};
+    if (fused && (forced == 1 || (forced == 0 && tiles >= 2 * n_cu)) && ssd::quad_supported(p)) return {F_FOUR_TILE, false, false, false};
+    if (fused && forced == 0 && ssd::cost::few_units(problem_of(p, n_cu))) {
+        if (p.states ? pair_supported(p, true) : p.dt_out == ssd::DT_F32 && pair_supported(with_states_in_out(p), true))
+            return {F_PAIR, !p.states, false, true};
+    }
     // Few state tiles, many chunks, fp32 `out`: the chunk-state launch keeps every compute unit busy where the
     // fused kernels have one workgroup per tile.  It writes the chunk states into `out`, and the streaming
     // recurrence turns them into the passed states in place (b=1 L=32768 H=80: 330 us against 425 us).
     if (fused && !p.states && forced == 0 && tiles < 2 * n_cu && (int64_t)tiles * p.C >= 32 * n_cu &&
         p.dt_out == ssd::DT_F32 && pair_supported(with_states_in_out(p)))
-        return {F_PAIR, true, false};
+        return {F_PAIR, true, false, false};
     // The caller wants the per-chunk states as well: the chunk-state launch of the four-tile kernel, which keeps
     // every compute unit busy whatever the number of tiles, then the streaming recurrence over what it wrote
     // (b=1 L=32768 H=80: 336 us against 496 us for the token-split kernel doing both at once).
     if (fused && p.states && (forced == 1 || (forced == 0 && (int64_t)tiles * p.C >= 32 * n_cu)) && pair_supported(p))
-        return {F_PAIR, false, false};
+        return {F_PAIR, false, false, false};
     if (!fused && (forced == 1 || (forced == 0 && (int64_t)tiles * p.C >= 8 * n_cu)) && ssd::quad_chunk_state_supported(p))
-        return {F_FOUR_TILE, false, false};
-    if (ssd::mfma_supported(p)) return {F_TOKEN_SPLIT, false, false};
+        return {F_FOUR_TILE, false, false, false};
+    if (ssd::mfma_supported(p)) return {F_TOKEN_SPLIT, false, false, false};
     if (fused && forced == 0 && !p.states && p.dt_out == ssd::DT_F32 && generic_pair_supported(with_states_in_out(p)))
-        return {F_GENERIC, true, true};
-    if (fused && forced == 0 && p.states && generic_pair_supported(p)) return {F_GENERIC, false, true};
-    return {F_GENERIC, false, false};
+        return {F_GENERIC, true, true, false};
+    if (fused && forced == 0 && p.states && generic_pair_supported(p)) return {F_GENERIC, false, true, false};
+    return {F_GENERIC, false, false, false};
+}
+
+// chunk states into p.states, then the recurrence over them into p.out / p.fin (which may be the same buffer)
+hipError_t launch_pair(const Params &p, hipStream_t s, bool generic = false)
+{
+    Params cs = p;
+    cs.out = nullptr; cs.fin = nullptr; cs.init = nullptr;
+    hipError_t e;
+    if (generic) e = ssd::launch_generic(cs, false, s);
+    else if (choose(cs, false, p.n_cu > 0 ? p.n_cu : 256).family == F_TOKEN_SPLIT) e = ssd::launch_mfma(cs, false, s);
+    else e = ssd::launch_quad_chunk_state(cs, s);
+    return e == hipSuccess ? ssd::launch_state_passing(pass_params_of(p), s) : e;
 }
 
 int run(const Params &p_in, bool fused, void *stream)
@@ -248,16 +267,6 @@ hipError_t scratch_pointer(int **ptr)
     return hipSuccess;
 }
 
-// The fused problem as the cost model sees it.
-ssd::cost::Problem problem_of(const Params &p, int n_cu)
-{
-    ssd::cost::Problem q;
-    q.units = (int64_t)p.batch * p.nheads * (p.headdim / 32) / 4;
-    q.chunks = p.C; q.chunk_size = p.Q; q.dstate = p.dstate;
-    q.n_cu = n_cu > 0 ? n_cu : 256;
-    return q;
-}
-
 // Estimate for the family `c` (what the call would run without a workspace); a family the model does not cover
 // counts as slower than anything.
 double estimate_us(const ssd::cost::Problem &q, const Choice &c)
@@ -280,7 +289,8 @@ bool chain_preferred(const Params &p, int n_cu)
     ssd::cost::chain_chunks_per_item(q, &chain);
     // within the model's error the chain kernel gets the call: its time follows the amount of work, the others'
     // depends on how their workgroups happen to fall on the compute units
-    return chain < 1.05 * estimate_us(q, choose(p, true, q.n_cu));
+    const Choice c = choose(p, true, q.n_cu);
+    return !c.few && chain < 1.05 * estimate_us(q, c);
 }
 
 // Whether a fused call runs on the ticket / flag-chain kernel: a usable workspace came with it and that kernel is
@@ -640,7 +650,7 @@ int ssd_query_fused_plan(const ssd_dims *dims, int has_workspace, int compute_un
         double us = 0.;
         const int r = ssd::cost::chain_chunks_per_item(q, &us);
         plan->estimate_us[SSD_FAMILY_CHAIN] = (float)us;
-        if (has_workspace && g_forced_split.load(std::memory_order_relaxed) == 0 && us < 1.05 * estimate_us(q, c)) {
+        if (has_workspace && g_forced_split.load(std::memory_order_relaxed) == 0 && !c.few && us < 1.05 * estimate_us(q, c)) {
             plan->family = SSD_FAMILY_CHAIN;
             plan->chunks_per_item = r;
         }

@@ -98,5 +98,24 @@ inline double pair_us(const Problem &q)
     return 6.0 + (x_bytes + 3.0 * s_bytes) / 5.0e6 * (256.0 / q.n_cu);
 }
 
+// Few units: the pair, whatever the estimates say (they are fits to 24 and more heads and know the recurrence as a pure
+// bandwidth).  The other families then leave most of the chip idle -- a unit's chunks are one serial chain in each of
+// them -- where the chunk-state launch spreads over (tile, chunk) and the recurrence costs about 0.2 us a chunk.  dstate
+// 128, chunk 256, headdim 64, batch 1, the faster of the others against the pair, us:
+//     heads      4 chunks      8             16            32            64            128
+//     4          11.3 /  7.8   19.3 /  9.0   43.0 / 11.0   63.9 / 15.1   91.5 / 25.1   142.1 /  39.6
+//     16         11.6 /  8.9   19.8 / 11.0   45.2 / 17.0   66.4 / 26.7   90.7 / 34.9   142.1 /  59.9
+//     32         12.0 / 10.6   21.5 / 15.8   46.6 / 24.9   65.2 / 31.7   92.1 / 57.2   100.5 / 114.2
+//     48         13.0 / 13.1   22.3 / 20.6   46.3 / 28.6   65.2 / 42.7   95.7 / 86.5   154.8 / 174.6
+//     80                       24.1 / 24.8   41.3 / 38.4
+// (fewer than four chunks: 24 heads x 2, 7.6 / 8.3).  Hence: up to a tenth as many units as compute units while there are
+// fewer than three unit-chunks per compute unit, and any length below a twenty-fourth; between the two lines the
+// estimates decide as they do for more units (they keep 24 heads x 64 chunks on the chain kernel, 92.7 / 44.7).
+inline bool few_units(const Problem &q)
+{
+    if (q.chunks < 4) return false;
+    return q.units * 24 <= q.n_cu || (q.units * 10 <= q.n_cu && q.units * q.chunks < 3 * (int64_t)q.n_cu);
+}
+
 }  // namespace cost
 }  // namespace ssd

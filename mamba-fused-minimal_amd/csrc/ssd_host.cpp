@@ -234,9 +234,23 @@ PyObject *chunk_scan_states(PyObject *, PyObject *const *a, Py_ssize_t n)
     });
 }
 
+// batch, seqlen, nheads, headdim, dstate, ngroups, chunk_size, nchunks -> whether the fused call with a fp32 `out` (and a
+// workspace) would run as chunk states + recurrence
+PyObject *plans_pair(PyObject *, PyObject *const *a, Py_ssize_t n)
+{
+    return guarded(n, 8, [&]() -> PyObject * {
+        int32_t v[8];
+        for (int i = 0; i < 8; ++i) v[i] = size32(number(a[i]));
+        const ssd_dims d{v[0], v[1], v[2], v[3], v[4], v[5], v[6], v[7]};
+        ssd_fused_plan plan{};
+        return PyBool_FromLong(ssd_query_fused_plan(&d, 1, 0, &plan) == SSD_OK && plan.family == SSD_FAMILY_PAIR);
+    });
+}
+
 #define SSD_METHOD(name) {#name, (PyCFunction)(void (*)(void))name, METH_FASTCALL, nullptr}
 PyMethodDef methods[] = {SSD_METHOD(chunk_state), SSD_METHOD(state_passing), SSD_METHOD(fused), SSD_METHOD(fused_scan),
-                         SSD_METHOD(chunk_cumsum), SSD_METHOD(chunk_scan_states), {nullptr, nullptr, 0, nullptr}};
+                         SSD_METHOD(chunk_cumsum), SSD_METHOD(chunk_scan_states), SSD_METHOD(plans_pair),
+                         {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_ssd_host", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
 
 }  // namespace

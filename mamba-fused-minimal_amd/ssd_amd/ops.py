@@ -77,6 +77,7 @@ class _Kept:
         self.tensor = tensor
         self.epochs = _Epochs()
         self.lock = threading.Lock()
+        self.used = False                  # whether the last call ran the kernel that uses it
 
 
 def _workspace_key(device, stream=None):
@@ -134,6 +135,7 @@ def _launch_on_own_workspace(x, nbytes, launch, pairs):
         epoch = ent.epochs.next(pairs)
         rc, used = launch(ent.tensor, epoch)
         ent.epochs.done(epoch, rc, used, pairs)
+        ent.used = bool(used)
         return rc
 
 
@@ -152,6 +154,9 @@ def fused_status(device=None, stream=None):
     if ent is None:
         return 0
     with ent.lock, torch.cuda.device(device):
+        if not ent.used:                   # the record is an earlier call's
+            stream.synchronize()
+            return 0
         return int(_lib.load().ssd_fused_workspace_status(ctypes.c_void_p(ent.tensor.data_ptr()),
                                                           ctypes.c_void_p(stream.cuda_stream)))
 
@@ -271,6 +276,10 @@ def _fused_chunk_state_state_passing_fwd(B, x, dt, dA_cumsum, out_dtype, initial
     B, x, dt, dA_cumsum, seq_idx = _prep_inputs(B, x, dt, dA_cumsum, seq_idx)
     if initial_states is not None and initial_states.stride(-1) != 1:
         initial_states = initial_states.contiguous()
+    if (states is None and out_dtype != torch.float32 and x.dtype == torch.bfloat16 and _kernel == 0 and _workspace is None
+            and _lib.host().plans_pair(batch, seqlen, nheads, headdim, dstate, ngroups, chunk_size, nchunks)):
+        # chunk states + recurrence is the faster way, and 16-bit `out` is no place for the chunk states
+        states = torch.empty((batch, nchunks, nheads, headdim, dstate), device=x.device, dtype=torch.float32)
 
     def launch(workspace, epoch):
         return _on_device(x, _lib.host().fused, x, B, dt, dA_cumsum, seq_idx, initial_states, states, out, final_states,
@@ -531,10 +540,13 @@ def _fused_chunk_state_state_passing_scan_fwd(B, x, C, dt, dA_cumsum, out_dtype=
     out = None
     if return_states:
         out = torch.empty((batch, nchunks, nheads, headdim, dstate), device=x.device, dtype=out_dtype or torch.float32)
-    rc = call(out)
+    rc = _lib.SSD_ERR_SCRATCH
+    if (out is not None or _kernel != 0 or _workspace is not None
+            or not _lib.host().plans_pair(batch, seqlen, nheads, headdim, dstate, ngroups, chunk_size, nchunks)):
+        rc = call(out)
     if rc == _lib.SSD_ERR_SCRATCH and out is None and _kernel == 0:
-        # arguments the one-launch kernel does not take: the passed states then need a place, which this wrapper (the
-        # owner of all allocations) provides and drops again
+        # arguments the one-launch kernel does not take, or sizes it is the slower way for (it is the chain kernel): the
+        # passed states then need a place, which this wrapper (the owner of all allocations) provides and drops again
         rc = call(torch.empty((batch, nchunks, nheads, headdim, dstate), device=x.device, dtype=torch.float32))
     _lib.check(rc, "ssd_fused_chunk_state_passing_scan_fwd")
     return out, final_states, y

@@ -1,0 +1,75 @@
+"""Few state tiles and four or more chunks: chunk states + recurrence in front of the kernels that walk a sequence.  Both
+sides of the rule's lines, every form of the call that it now takes, against the token-split kernel on the same inputs."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def ops():
+    import ssd_amd
+    from ssd_amd import _lib
+    _lib.load()
+    assert torch.cuda.is_available(), "these tests need the MI355X"
+    return ssd_amd
+
+
+@pytest.mark.parametrize("kw,pair", [
+    (dict(L=1024, H=8), True),                             # four chunks
+    (dict(L=768, H=8), False),                             # three
+    (dict(L=1023, H=8, nseq=3), True),                     # ragged, packed
+    (dict(L=2100, H=6, P=96, N=64), True),                 # a unit and a half of tiles, dstate 64
+    (dict(L=1400, H=4, G=2, Q=128), True),                 # chunk 128, grouped B, ragged
+    (dict(L=3840, H=51), False),                           # above a twenty-fourth of the units, 25 x 15 unit-chunks: below three per CU
+    (dict(L=16384, H=24), False),                          # three unit-chunks per compute unit, 12 units
+    (dict(L=24576, H=20), True),                           # ten units, any length
+], ids=lambda v: "-".join(f"{k}{x}" for k, x in v.items()) if isinstance(v, dict) else str(v))
+def test_few_units(ops, oracle, kw, pair):
+    args = dict(b=1, P=64, N=128, G=1, Q=256, init=True, nseq=0)
+    args.update(kw)
+    d = oracle.make_inputs(1, **args)
+    H, P, N, G, Q, L = (args[k] for k in "HPNGQL")
+    if (L, H) != (3840, 51):
+        assert (ops.fused_plan(1, L, H, P, N, G, Q)["family"] == "pair") == pair
+    mv = lambda t: None if t is None else t.cuda()  # noqa: E731
+    x, B, dt, dA, seq, init = (mv(d[k]) for k in ("x", "B", "dt", "dA_cumsum", "seq_idx", "initial_states"))
+    print(f"[few] {kw}", flush=True)
+    fused = ops._fused_chunk_state_state_passing_fwd
+    old = ops.set_token_split(4)
+    try:
+        want, want_fin = fused(B, x, dt, dA, torch.float32, initial_states=init, seq_idx=seq)
+        want_y = ops._chunk_scan_states_fwd(mv(d["C"]), want, dA, seq_idx=seq, out_dtype=torch.float32)
+    finally:
+        ops.set_token_split(old)
+    # both sides split x * w into bf16 hi + lo (2^-17 of every product) and add in fp32 in another order
+    tol = dict(rtol=1e-4, atol=1e-4)
+    for out_dtype in (torch.float32, torch.bfloat16, torch.float16):
+        out, fin = fused(B, x, dt, dA, out_dtype, initial_states=init, seq_idx=seq)
+        assert out.dtype == out_dtype and fin.dtype == torch.float32
+        if out_dtype == torch.float32:
+            torch.testing.assert_close(out, want, **tol)
+        else:
+            torch.testing.assert_close(out.float(), want, rtol=2.0 ** (-7 if out_dtype == torch.bfloat16 else -10), atol=1e-4)
+        torch.testing.assert_close(fin, want_fin, **tol)
+    # a states buffer of the caller, the scan's state half behind it, a captured call replayed between eager ones
+    states = torch.full(want.shape, float("nan"), device="cuda")
+    out, fin = fused(B, x, dt, dA, torch.float32, initial_states=init, seq_idx=seq, states=states)
+    torch.testing.assert_close(out, want, **tol)
+    torch.testing.assert_close(states, ops._chunk_state_fwd(B, x, dt, dA, seq_idx=seq), **tol)
+    if H * P // 32 % 4 == 0 and H // G * P // 32 % 4 == 0:
+        none, fin, y = ops._fused_chunk_state_state_passing_scan_fwd(B, x, mv(d["C"]), dt, dA, initial_states=init, seq_idx=seq,
+                                                                     return_states=False, y_dtype=torch.float32)
+        assert none is None
+        torch.testing.assert_close(fin, want_fin, **tol)
+        torch.testing.assert_close(y, want_y, rtol=1e-3, atol=1e-3)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        g_out, g_fin = fused(B, x, dt, dA, torch.bfloat16, initial_states=init, seq_idx=seq)
+    for _ in range(3):
+        g_out.zero_()
+        g_fin.zero_()
+        graph.replay()
+        eager, eager_fin = fused(B, x, dt, dA, torch.bfloat16, initial_states=init, seq_idx=seq)
+        torch.cuda.synchronize()
+        assert torch.equal(g_out, eager) and torch.equal(g_fin, eager_fin)
