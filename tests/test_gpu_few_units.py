@@ -21,7 +21,8 @@ def ops():
     (dict(L=1023, H=8, nseq=3), True),                     # ragged, packed
     (dict(L=2100, H=6, P=96, N=64), True),                 # a unit and a half of tiles, dstate 64
     (dict(L=1400, H=4, G=2, Q=128), True),                 # chunk 128, grouped B, ragged
-    (dict(L=3840, H=51), False),                           # above a twenty-fourth of the units, 25 x 15 unit-chunks: below three per CU
+    (dict(L=3840, H=51), True),                            # 25 units, 15 chunks: a tenth of 256, below three unit-chunks per compute unit
+    (dict(L=2048, H=54), False),                           # 27 units
     (dict(L=16384, H=24), False),                          # three unit-chunks per compute unit, 12 units
     (dict(L=24576, H=20), True),                           # ten units, any length
 ], ids=lambda v: "-".join(f"{k}{x}" for k, x in v.items()) if isinstance(v, dict) else str(v))
@@ -30,8 +31,7 @@ def test_few_units(ops, oracle, kw, pair):
     args.update(kw)
     d = oracle.make_inputs(1, **args)
     H, P, N, G, Q, L = (args[k] for k in "HPNGQL")
-    if (L, H) != (3840, 51):
-        assert (ops.fused_plan(1, L, H, P, N, G, Q)["family"] == "pair") == pair
+    assert (ops.fused_plan(1, L, H, P, N, G, Q, compute_units=256)["family"] == "pair") == pair
     mv = lambda t: None if t is None else t.cuda()  # noqa: E731
     x, B, dt, dA, seq, init = (mv(d[k]) for k in ("x", "B", "dt", "dA_cumsum", "seq_idx", "initial_states"))
     print(f"[few] {kw}", flush=True)
