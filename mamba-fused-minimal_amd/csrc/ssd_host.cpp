@@ -234,16 +234,22 @@ PyObject *chunk_scan_states(PyObject *, PyObject *const *a, Py_ssize_t n)
     });
 }
 
-// batch, seqlen, nheads, headdim, dstate, ngroups, chunk_size, nchunks -> whether the fused call with a fp32 `out` (and a
-// workspace) would run as chunk states + recurrence
+// batch, seqlen, nheads, headdim, dstate, ngroups, chunk_size, nchunks, whether x is bf16 -> whether the fused call gains
+// from a place for fp32 chunk states: where it would run as chunk states + recurrence with a fp32 `out` (and a workspace).
+// The fp32 matrix kernel, which would walk the sequence otherwise, gains from four chunks on while 64 x 64 state tiles give
+// a compute unit no more than one and a half workgroups to walk with (fp16 out, walk against pair, us: 8 heads x 16 chunks
+// 48.6 / 17.9, 2 x 24 x 12 53.4 / 39.9, 4 x 48 x 12 140 / 123; 8 x 48 x 4 78.9 / 88.1; three chunks of 24 heads 11.7 / 14.0).
 PyObject *plans_pair(PyObject *, PyObject *const *a, Py_ssize_t n)
 {
-    return guarded(n, 8, [&]() -> PyObject * {
+    return guarded(n, 9, [&]() -> PyObject * {
         int32_t v[8];
         for (int i = 0; i < 8; ++i) v[i] = size32(number(a[i]));
         const ssd_dims d{v[0], v[1], v[2], v[3], v[4], v[5], v[6], v[7]};
         ssd_fused_plan plan{};
-        return PyBool_FromLong(ssd_query_fused_plan(&d, 1, 0, &plan) == SSD_OK && plan.family == SSD_FAMILY_PAIR);
+        if (ssd_query_fused_plan(&d, 1, 0, &plan) != SSD_OK) Py_RETURN_FALSE;
+        if (number(a[8]) && plan.family != SSD_FAMILY_GENERIC) return PyBool_FromLong(plan.family == SSD_FAMILY_PAIR);
+        const int64_t tiles = (int64_t)d.batch * d.nheads * ((d.headdim + 63) / 64) * ((d.dstate + 63) / 64);
+        return PyBool_FromLong(d.nchunks >= 4 && tiles <= 384);
     });
 }
 

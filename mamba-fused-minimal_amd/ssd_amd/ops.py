@@ -276,8 +276,9 @@ def _fused_chunk_state_state_passing_fwd(B, x, dt, dA_cumsum, out_dtype, initial
     B, x, dt, dA_cumsum, seq_idx = _prep_inputs(B, x, dt, dA_cumsum, seq_idx)
     if initial_states is not None and initial_states.stride(-1) != 1:
         initial_states = initial_states.contiguous()
-    if (states is None and out_dtype != torch.float32 and x.dtype == torch.bfloat16 and _kernel == 0 and _workspace is None
-            and _lib.host().plans_pair(batch, seqlen, nheads, headdim, dstate, ngroups, chunk_size, nchunks)):
+    if (states is None and out_dtype != torch.float32 and _kernel == 0 and _workspace is None
+            and _lib.host().plans_pair(batch, seqlen, nheads, headdim, dstate, ngroups, chunk_size, nchunks,
+                                       x.dtype == torch.bfloat16)):
         # chunk states + recurrence is the faster way, and 16-bit `out` is no place for the chunk states
         states = torch.empty((batch, nchunks, nheads, headdim, dstate), device=x.device, dtype=torch.float32)
 
@@ -542,7 +543,7 @@ def _fused_chunk_state_state_passing_scan_fwd(B, x, C, dt, dA_cumsum, out_dtype=
         out = torch.empty((batch, nchunks, nheads, headdim, dstate), device=x.device, dtype=out_dtype or torch.float32)
     rc = _lib.SSD_ERR_SCRATCH
     if (out is not None or _kernel != 0 or _workspace is not None
-            or not _lib.host().plans_pair(batch, seqlen, nheads, headdim, dstate, ngroups, chunk_size, nchunks)):
+            or not _lib.host().plans_pair(batch, seqlen, nheads, headdim, dstate, ngroups, chunk_size, nchunks, True)):
         rc = call(out)
     if rc == _lib.SSD_ERR_SCRATCH and out is None and _kernel == 0:
         # arguments the one-launch kernel does not take, or sizes it is the slower way for (it is the chain kernel): the
