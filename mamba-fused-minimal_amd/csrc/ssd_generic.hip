@@ -15,9 +15,9 @@
 // One workgroup owns a (16 A) x (16 S) tile of one (batch, head) and chunk; its SPLIT = 4 waves take a quarter of the
 // chunk's tokens each and add up through LDS, after which wave v holds accumulator q = v of every instruction.  In
 // fused mode it walks the chunks with the state in registers.  Short chunks leave a quarter too little to do between
-// a wave's start and the adding up: there a wave owns a tile by itself (SPLIT = 1).  Rows and columns past the edge of an odd headdim or
-// dstate are not loaded: the last lanes' vectors move up to end at the edge and repeat rows that their neighbours also
-// compute (equal values, stored twice).
+// a wave's start and the adding up: there a wave owns a tile by itself (SPLIT = 1).  Rows and columns past the edge of an
+// odd headdim or dstate are not loaded: the last lanes' vectors move up to end at the edge and repeat rows that their
+// neighbours also compute.  Both store them, the same bits: a sum's order does not depend on the wave or lane that forms it.
 //
 // Reference semantics: kernels/ssd_chunk_state.py:97-173, kernels/ssd_state_passing.py:27-84.
 #include "ssd_tile.h"
@@ -238,19 +238,23 @@ __global__ void __launch_bounds__(64 * kWaves, FUSED ? 2 : 3) generic_kernel(con
 #pragma unroll
                 for (int s = 0; s < S; ++s) part[q][slot][r][lane][s] = acc[r][s][q];
         });
-        float own[A][S];
-#pragma unroll
-        for (int r = 0; r < A; ++r)
-#pragma unroll
-            for (int s = 0; s < S; ++s)
-                own[r][s] = wv == 0 ? acc[r][s][0] : wv == 1 ? acc[r][s][1] : wv == 2 ? acc[r][s][2] : acc[r][s][3];
         __syncthreads();
-#pragma unroll
-        for (int o = 0; o < kWaves - 1; ++o)
+        // every wave adds the four parts up in the order of the tokens, so that a row does not depend on the wave that
+        // finishes it: rows that a moved-up vector repeats are stored by two waves (or workgroups), with the same bits
+        float own[A][S];
+        static_for<kWaves>([&](auto qc) {
+            constexpr int q = qc.value;
+            if (q != wv) return;
 #pragma unroll
             for (int r = 0; r < A; ++r)
 #pragma unroll
-                for (int s = 0; s < S; ++s) own[r][s] += part[wv][o][r][lane][s];
+                for (int s = 0; s < S; ++s) {
+                    auto of_wave = [&](int o) { return o == q ? acc[r][s][q] : part[q][o < q ? o : o - 1][r][lane][s]; };
+                    own[r][s] = of_wave(0);
+#pragma unroll
+                    for (int o = 1; o < kWaves; ++o) own[r][s] += of_wave(o);
+                }
+        });
         if (FUSED) __syncthreads();      // the next chunk's partial tiles go to the same place
 
         if (p.states && mine)

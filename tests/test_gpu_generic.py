@@ -86,3 +86,32 @@ def test_infinities_stay_where_they_are_and_tokens_behind_the_end_do_not_count(o
     want, _ = _chunk_states_64(d)
     want[0, 1, 1, 3] = 0.0
     torch.testing.assert_close(st.double(), want, rtol=1e-4, atol=1e-5)
+
+
+@pytest.mark.parametrize("kw", [
+    dict(P=80, N=128, L=2048, H=16, Q=128),                # tiles of 48 rows: row 77 ends one lane's vector and starts the next one's
+    dict(P=80, N=128, L=2048, H=16, Q=128, dtype="bf16"), dict(P=63, N=65, L=257, Q=256), dict(P=31, N=24, L=300, Q=100, dtype="fp16"),
+    dict(P=33, N=40, L=515, Q=128), dict(P=65, N=16, L=300, Q=300, dtype="bf16"), dict(P=77, N=129, L=700, Q=128),
+    dict(P=63, N=128, L=700, Q=128, b=8, H=48),
+], ids=lambda kw: "-".join(f"{k}{v}" for k, v in kw.items()))
+def test_a_row_does_not_depend_on_where_it_lies(ops, oracle, kw):
+    # Rows that two waves or workgroups hold (a lane's vector moved up to end at an odd headdim) are stored by both: the sums
+    # must have one order.  All headdim rows of x hold the same numbers, so all rows of a state must hold the same bits.
+    args = dict(b=1, H=3, G=1, init=False, nseq=0, dtype="fp32")
+    args.update(kw)
+    d = oracle.make_inputs(1, **args)
+    print(f"[generic] same rows {kw}", flush=True)
+    x, B, dt, dA = d["x"][..., :1].expand_as(d["x"]).contiguous().cuda(), d["B"].cuda(), d["dt"].cuda(), d["dA_cumsum"].cuda()
+    same = lambda t: torch.equal(t, t[..., :1, :].expand_as(t))  # noqa: E731
+    states = ops._chunk_state_fwd(B, x, dt, dA)
+    assert float(states.abs().max()) > 0 and same(states)
+    assert torch.equal(states, ops._chunk_state_fwd(B, x, dt, dA))
+    calls = [ops._fused_chunk_state_state_passing_fwd(B, x, dt, dA, torch.float32)]
+    old = ops.set_token_split(4)                           # the walk over the chunks
+    try:
+        calls += [ops._fused_chunk_state_state_passing_fwd(B, x, dt, dA, torch.float32) for _ in range(2)]
+    finally:
+        ops.set_token_split(old)
+    for out, fin in calls:
+        assert same(out) and same(fin)
+    assert torch.equal(calls[1][0], calls[2][0]) and torch.equal(calls[1][1], calls[2][1])
