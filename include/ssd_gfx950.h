@@ -272,6 +272,18 @@ typedef struct ssd_fused_plan {
 int ssd_query_fused_plan(const ssd_dims *dims, int has_workspace, int compute_units, ssd_fused_plan *plan);
 
 /*
+ * Whether ssd_fused_chunk_state_passing_fwd_ws (with a workspace and SSD_KERNEL_AUTO) on these very arguments is estimated
+ * to gain from a contiguous fp32 place for the chunk states that it does not have: 1 = yes, 0 = no, negative = rejected
+ * arguments.  `out` 16-bit: pass such a tensor as `states`; `out` absent (ssd_fused_chunk_state_passing_scan_fwd): pass
+ * one as `out`; fp32 `out`: always 0.  For a caller that can allocate (the library never does).  Strides, alignment,
+ * element types and the ssd_set_token_split hook count as they do in the call, the compute units are those of the
+ * current device (256 without one).  Pure host logic; launches nothing.
+ */
+int ssd_query_fused_wants_states(const ssd_tensor *x, const ssd_tensor *B, const ssd_tensor *dt, const ssd_tensor *dA_cumsum,
+                                 const ssd_tensor *seq_idx, const ssd_tensor *initial_states, const ssd_tensor *out,
+                                 const ssd_tensor *final_states, const ssd_dims *dims);
+
+/*
  * dt preparation and per-chunk cumulative sum, the producer of `dt` and `dA_cumsum` for the three calls above.
  * Replaces _chunk_cumsum_fwd / _chunk_cumsum_fwd_kernel (kernels/ssd_chunk_state.py:176-199, 33-79):
  *   d = float(dt[b,l,h]) (+ dt_bias[h]); d = log1p(exp(d)) where dt_softplus and d <= 20; d = clamp(d, dt_min, dt_max);

@@ -658,6 +658,35 @@ int ssd_query_fused_plan(const ssd_dims *dims, int has_workspace, int compute_un
     return SSD_OK;
 }
 
+int ssd_query_fused_wants_states(const ssd_tensor *x, const ssd_tensor *B, const ssd_tensor *dt, const ssd_tensor *dA_cumsum,
+                                 const ssd_tensor *seq_idx, const ssd_tensor *initial_states, const ssd_tensor *out,
+                                 const ssd_tensor *final_states, const ssd_dims *dims)
+{
+    Params p;
+    int rc = fill_fused(p, x, B, dt, dA_cumsum, seq_idx, initial_states, nullptr, out, final_states, dims, 1, true);
+    if (rc) return rc;
+    if (p.out && p.dt_out == ssd::DT_F32) return 0;
+    const int n_cu = compute_units() > 0 ? compute_units() : 256;
+    // a contiguous fp32 (b,C,H,P,N) at a made-up, well-aligned address
+    const int64_t plane = (int64_t)p.headdim * p.dstate;
+    void *const somewhere = (void *)(uintptr_t)4096;
+    const ssd_tensor f32 = {somewhere, SSD_F32, 0, {p.C * p.nheads * plane, p.nheads * plane, plane, p.dstate, 1}};
+    Params as_out, as_states;
+    rc = fill_fused(as_out, x, B, dt, dA_cumsum, seq_idx, initial_states, nullptr, &f32, final_states, dims, 1);
+    if (rc == SSD_OK) rc = fill_fused(as_states, x, B, dt, dA_cumsum, seq_idx, initial_states, &f32, p.out ? out : &f32, final_states, dims, 1);
+    if (rc) return rc;
+    // what the call runs with a fp32 `out`, and whether it still does with the place it would be given
+    const Choice c = choose(as_out, true, n_cu), given = p.out ? choose(as_states, true, n_cu) : c;
+    if (c.family == F_PAIR)
+        return given.family == F_PAIR && !(ssd::chain_supported(as_out) && chain_preferred(as_out, n_cu)) ? 1 : 0;
+    // The fp32 matrix kernel, which would walk the sequence otherwise, gains from four chunks on while 64 x 64 state tiles
+    // give a compute unit no more than one and a half workgroups to walk with (fp16 out, walk against pair, us: 8 heads x
+    // 16 chunks 48.6 / 17.9, 2 x 24 x 12 53.4 / 39.9, 4 x 48 x 12 140 / 123; 8 x 48 x 4 78.9 / 88.1; three chunks of 24
+    // heads 11.7 / 14.0).
+    const int64_t tiles = (int64_t)p.batch * p.nheads * ((p.headdim + 63) / 64) * ((p.dstate + 63) / 64);
+    return c.generic_pair && given.generic_pair && p.C >= 4 && 2 * tiles <= 3 * n_cu ? 1 : 0;
+}
+
 int ssd_chunk_cumsum_fwd(const ssd_tensor *dt, const ssd_tensor *A, const ssd_tensor *dt_bias, const ssd_tensor *dt_out,
                          const ssd_tensor *dA_cumsum, int32_t batch, int32_t seqlen, int32_t nheads, int32_t chunk_size,
                          int dt_softplus, float dt_min, float dt_max, void *stream)

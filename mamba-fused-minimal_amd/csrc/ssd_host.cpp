@@ -234,28 +234,21 @@ PyObject *chunk_scan_states(PyObject *, PyObject *const *a, Py_ssize_t n)
     });
 }
 
-// batch, seqlen, nheads, headdim, dstate, ngroups, chunk_size, nchunks, whether x is bf16 -> whether the fused call gains
-// from a place for fp32 chunk states: where it would run as chunk states + recurrence with a fp32 `out` (and a workspace).
-// The fp32 matrix kernel, which would walk the sequence otherwise, gains from four chunks on while 64 x 64 state tiles give
-// a compute unit no more than one and a half workgroups to walk with (fp16 out, walk against pair, us: 8 heads x 16 chunks
-// 48.6 / 17.9, 2 x 24 x 12 53.4 / 39.9, 4 x 48 x 12 140 / 123; 8 x 48 x 4 78.9 / 88.1; three chunks of 24 heads 11.7 / 14.0).
-PyObject *plans_pair(PyObject *, PyObject *const *a, Py_ssize_t n)
+// x, B, dt, dA_cumsum, seq_idx, initial_states, out (or None), final_states -> whether the fused call gains from a place for
+// fp32 chunk states (arguments it would reject: no, the call itself says so)
+PyObject *wants_states(PyObject *, PyObject *const *a, Py_ssize_t n)
 {
-    return guarded(n, 9, [&]() -> PyObject * {
-        int32_t v[8];
-        for (int i = 0; i < 8; ++i) v[i] = size32(number(a[i]));
-        const ssd_dims d{v[0], v[1], v[2], v[3], v[4], v[5], v[6], v[7]};
-        ssd_fused_plan plan{};
-        if (ssd_query_fused_plan(&d, 1, 0, &plan) != SSD_OK) Py_RETURN_FALSE;
-        if (number(a[8]) && plan.family != SSD_FAMILY_GENERIC) return PyBool_FromLong(plan.family == SSD_FAMILY_PAIR);
-        const int64_t tiles = (int64_t)d.batch * d.nheads * ((d.headdim + 63) / 64) * ((d.dstate + 63) / 64);
-        return PyBool_FromLong(d.nchunks >= 4 && tiles <= 384);
+    return guarded(n, 8, [&]() -> PyObject * {
+        ssd_tensor t[8];
+        for (int i = 0; i < 8; ++i) t[i] = tensor(a[i]);
+        const ssd_dims d = dims_of(a[0], a[1], a[2]);
+        return PyBool_FromLong(ssd_query_fused_wants_states(&t[0], &t[1], &t[2], &t[3], &t[4], &t[5], &t[6], &t[7], &d) == 1);
     });
 }
 
 #define SSD_METHOD(name) {#name, (PyCFunction)(void (*)(void))name, METH_FASTCALL, nullptr}
 PyMethodDef methods[] = {SSD_METHOD(chunk_state), SSD_METHOD(state_passing), SSD_METHOD(fused), SSD_METHOD(fused_scan),
-                         SSD_METHOD(chunk_cumsum), SSD_METHOD(chunk_scan_states), SSD_METHOD(plans_pair),
+                         SSD_METHOD(chunk_cumsum), SSD_METHOD(chunk_scan_states), SSD_METHOD(wants_states),
                          {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_ssd_host", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
 

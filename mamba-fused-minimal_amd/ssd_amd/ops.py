@@ -35,6 +35,15 @@ def _on_device(t, call, *args):
         return call(*args, _raw_stream(index))
 
 
+def _wants_states(x, *args):
+    """Whether the fused call on these tensors gains from a place for fp32 chunk states (ssd_query_fused_wants_states):
+    chunk states + recurrence is then the faster way, and neither a 16-bit nor an absent ``out`` is such a place."""
+    if x.device.index == torch.cuda.current_device():
+        return _lib.host().wants_states(x, *args)
+    with torch.cuda.device(x.device.index):
+        return _lib.host().wants_states(x, *args)
+
+
 # Workspaces of the ticket / flag-chain kernel that the wrappers keep to themselves: one per (device, stream), grown on
 # demand, with the epoch of the last launch on it.  A workspace nobody else writes to lets a call tell the library that
 # the launch before left it in order (ssd_fused_opts.epoch), which saves the fill launch in front of the kernel.
@@ -277,9 +286,7 @@ def _fused_chunk_state_state_passing_fwd(B, x, dt, dA_cumsum, out_dtype, initial
     if initial_states is not None and initial_states.stride(-1) != 1:
         initial_states = initial_states.contiguous()
     if (states is None and out_dtype != torch.float32 and _kernel == 0 and _workspace is None
-            and _lib.host().plans_pair(batch, seqlen, nheads, headdim, dstate, ngroups, chunk_size, nchunks,
-                                       x.dtype == torch.bfloat16)):
-        # chunk states + recurrence is the faster way, and 16-bit `out` is no place for the chunk states
+            and _wants_states(x, B, dt, dA_cumsum, seq_idx, initial_states, out, final_states)):
         states = torch.empty((batch, nchunks, nheads, headdim, dstate), device=x.device, dtype=torch.float32)
 
     def launch(workspace, epoch):
@@ -543,7 +550,7 @@ def _fused_chunk_state_state_passing_scan_fwd(B, x, C, dt, dA_cumsum, out_dtype=
         out = torch.empty((batch, nchunks, nheads, headdim, dstate), device=x.device, dtype=out_dtype or torch.float32)
     rc = _lib.SSD_ERR_SCRATCH
     if (out is not None or _kernel != 0 or _workspace is not None
-            or not _lib.host().plans_pair(batch, seqlen, nheads, headdim, dstate, ngroups, chunk_size, nchunks, True)):
+            or not _wants_states(x, B, dt, dA_cumsum, seq_idx, initial_states, None, final_states)):
         rc = call(out)
     if rc == _lib.SSD_ERR_SCRATCH and out is None and _kernel == 0:
         # arguments the one-launch kernel does not take, or sizes it is the slower way for (it is the chain kernel): the

@@ -73,3 +73,24 @@ def test_few_units(ops, oracle, kw, pair):
         eager, eager_fin = fused(B, x, dt, dA, torch.bfloat16, initial_states=init, seq_idx=seq)
         torch.cuda.synchronize()
         assert torch.equal(g_out, eager) and torch.equal(g_fin, eager_fin)
+
+
+def test_a_strided_initial_plane_keeps_the_kernel_it_had(ops, oracle):
+    # initial states out of a wider cache: the recurrence walks a head's plane as one row and cannot take them, so no buffer
+    # is made and the chain kernel serves bf16 `out` as it would without the rule (32 chunks of 8 heads)
+    d = oracle.make_inputs(1, b=1, L=8192, H=8, init=True)
+    x, B, dt, dA = (d[k].cuda() for k in ("x", "B", "dt", "dA_cumsum"))
+    init = torch.zeros(1, 8, 64, 160, device="cuda")[..., :128]
+    init.copy_(d["initial_states"])
+    want_out, want_fin = oracle.fused_ref(d["B"], d["x"], d["dt"], d["dA_cumsum"], initial_states=d["initial_states"])
+    ops.release_workspaces()
+    out, fin = ops._fused_chunk_state_state_passing_fwd(B, x, dt, dA, torch.bfloat16, initial_states=init)
+    torch.cuda.synchronize()
+    from ssd_amd.ops import _WORKSPACES
+    assert [k.epochs.last for k in _WORKSPACES.values()] == [1] and ops.fused_status() == 0
+    torch.testing.assert_close(out.float().cpu(), want_out, rtol=2.0 ** -7, atol=1e-3)
+    torch.testing.assert_close(fin.cpu(), want_fin, rtol=2e-3, atol=1e-3)
+    # where only the fp32 matrix kernel applies: its walk, no buffer beside it
+    y, yf = ops._fused_chunk_state_state_passing_fwd(B.half(), x.half(), dt, dA, torch.float16, initial_states=init)
+    torch.testing.assert_close(y.float().cpu(), want_out, rtol=2e-3, atol=1e-3)
+    torch.testing.assert_close(yf.cpu(), want_fin, rtol=2e-3, atol=1e-3)

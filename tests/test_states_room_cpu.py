@@ -1,0 +1,52 @@
+"""When a wrapper lends the fused call a place for fp32 chunk states: the library's answer for the very tensors of a call
+(host logic only, the tensors' memory is not touched)."""
+import pytest
+import torch
+
+import ssd_amd as ops
+from ssd_amd import _lib
+
+
+def _wants(b=1, L=4096, H=8, P=64, N=128, G=1, Q=256, dtype=torch.bfloat16, out=torch.bfloat16, init=None, x=None, seq=None):
+    C = -(-L // Q)
+    x = torch.empty(b, L, H, P, dtype=dtype) if x is None else x
+    dt = torch.empty(b, H, C, Q)
+    out = None if out is None else torch.empty(b, C, H, P, N, dtype=out)
+    return _lib.host().wants_states(x, torch.empty(b, L, G, N, dtype=dtype), dt, dt, seq, init, out, torch.empty(b, H, P, N))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
+def test_what_the_call_would_run_decides(dtype):
+    # 8 heads x 16 chunks: chunk states + recurrence, with a place for the chunk states, on the bf16 kernels and on the
+    # fp32 matrix kernel
+    assert _wants(dtype=dtype, out=dtype) and _wants(dtype=dtype, out=None)
+    assert not _wants(dtype=dtype, out=torch.float32)                       # `out` is such a place
+    assert not _wants(dtype=dtype, out=dtype, L=768)                        # three chunks: the walk
+    init = torch.empty(1, 8, 64, 128)
+    assert _wants(dtype=dtype, out=dtype, init=init)
+    # planes that are not one row (a slice of a wider cache): the recurrence cannot walk them, so the call would run on the
+    # kernels that walk a sequence and write the chunk states beside it
+    sliced = torch.empty(1, 8, 64, 160)[..., :128]
+    assert not _wants(dtype=dtype, out=dtype, init=sliced) and not _wants(dtype=dtype, out=None, init=sliced)
+    # a batch or head stride is no matter
+    assert _wants(dtype=dtype, out=dtype, init=torch.empty(1, 16, 64, 128)[:, ::2])
+    old = ops.set_token_split(4)                                            # a kernel is forced: no chunk states wanted
+    try:
+        assert not _wants(dtype=dtype, out=dtype)
+    finally:
+        ops.set_token_split(old)
+
+
+def test_views_off_the_bf16_tiling_are_the_fp32_kernels_business():
+    # 384 state tiles of 64 x 64 are its line; an odd token stride keeps bf16 x off the bf16 kernels
+    assert _wants(b=4, L=3072, H=48, dtype=torch.float16, out=torch.float16)
+    assert not _wants(b=8, L=1024, H=48, dtype=torch.float16, out=torch.float16)
+    odd = torch.empty(4, 3072, 48 * 64 + 1, dtype=torch.bfloat16)[..., :48 * 64].unflatten(-1, (48, 64))
+    assert _wants(b=4, L=3072, H=48, x=odd) and not _wants(b=4, L=3072, H=48)
+
+
+def test_arguments_the_call_rejects_are_left_to_it():
+    assert not _wants(H=9, G=2, L=1024)
+    assert not _wants(x=torch.empty(1, 4096, 64, 8, dtype=torch.bfloat16).transpose(2, 3))
+    with pytest.raises(TypeError):
+        _wants(dtype=torch.float64)
