@@ -174,8 +174,8 @@ ssd::cost::Problem problem_of(const Params &p, int64_t n_cu)
     return q;
 }
 
-// The kernel family of a call without a workspace.
-Choice choose(const Params &p, bool fused, int64_t n_cu)
+// The kernel family of a call without a workspace.  few: whether the rule for few units counts.
+Choice choose(const Params &p, bool fused, int64_t n_cu, bool few = true)
 {
     // Fused launch: with at least two state tiles per compute unit the four-tiles-per-workgroup kernel wins (B is
     // fetched once per four tiles and the state never leaves the accumulators); with fewer, the token-split
@@ -183,7 +183,7 @@ Choice choose(const Params &p, bool fused, int64_t n_cu)
     const int tiles = p.batch * p.nheads * (p.headdim / 32);
     const int forced = g_forced_split.load(std::memory_order_relaxed);      // one value for the whole choice
     if (fused && (forced == 1 || (forced == 0 && tiles >= 2 * n_cu)) && ssd::quad_supported(p)) return {F_FOUR_TILE, false, false, false};
-    if (fused && forced == 0 && ssd::cost::few_units(problem_of(p, n_cu))) {
+    if (fused && few && forced == 0 && ssd::cost::few_units(problem_of(p, n_cu))) {
         if (p.states ? pair_supported(p, true) : p.dt_out == ssd::DT_F32 && pair_supported(with_states_in_out(p), true))
             return {F_PAIR, !p.states, false, true};
     }
@@ -289,8 +289,14 @@ bool chain_preferred(const Params &p, int n_cu)
     ssd::cost::chain_chunks_per_item(q, &chain);
     // within the model's error the chain kernel gets the call: its time follows the amount of work, the others'
     // depends on how their workgroups happen to fall on the compute units
-    const Choice c = choose(p, true, q.n_cu);
-    return !c.few && chain < 1.05 * estimate_us(q, c);
+    Choice c = choose(p, true, q.n_cu);
+    if (c.few) {
+        // in front of this kernel too -- with packed sequences, which cut its chains, only where that never loses; elsewhere
+        // it stays in front of the kernels that this one is not preferred to
+        if (!p.seq || ssd::cost::few_units_packed(q)) return false;
+        c = choose(p, true, q.n_cu, false);
+    }
+    return chain < 1.05 * estimate_us(q, c);
 }
 
 // Whether a fused call runs on the ticket / flag-chain kernel: a usable workspace came with it and that kernel is

@@ -117,5 +117,22 @@ inline bool few_units(const Problem &q)
     return q.units * 24 <= q.n_cu || (q.units * 10 <= q.n_cu && q.units * q.chunks < 3 * (int64_t)q.n_cu);
 }
 
+// The same against the chain kernel for packed sequences (seq_idx): its chains are then as long as a sequence, and how
+// long those are only the device knows, so the pair goes in front only where it is no slower with a sequence start in
+// every chunk.  Chain kernel with four starts a chunk against the pair, us -- fp32 out, bf16 out, call with the scan's
+// state half:
+//     heads x chunks      dstate 128, chunk 256                      dstate 64, chunk 128
+//     8 x 32              33.0 / 19.9   33.9 / 22.3   42.2 / 30.1    19.9 / 14.2   20.2 / 16.9   24.0 / 22.1
+//     16 x 24 (one start) 35.3 / 23.6   36.0 / 24.9   45.2 / 34.1    21.4 / 15.0   21.7 / 16.9   26.1 / 23.8
+//     12 x 32 (chunk 128) 24.6 / 21.9   25.4 / 24.0   31.0 / 32.1    19.7 / 16.4   20.0 / 18.9   24.6 / 25.2
+//     20 x 32             35.2 / 29.3   35.6 / 31.3   44.8 / 46.2    20.3 / 20.4   20.4 / 22.5   26.3 / 29.8
+//     8 x 64              34.1 / 32.7   34.4 / 37.3   43.8 / 44.0    20.4 / 24.2   20.6 / 29.6   25.6 / 33.3
+// (with four sequences in a row the pair is ahead to 512 chunks: 4 heads x 512 260 / 127, 16 heads x 64 60.5 / 37.9; with
+// 64 of them 4 heads x 512 are 67.5 / 126.)
+inline bool few_units_packed(const Problem &q)
+{
+    return few_units(q) && q.units * 24 <= q.n_cu && q.chunks <= 32 && q.units * q.chunks * 4 <= 3 * (int64_t)q.n_cu;
+}
+
 }  // namespace cost
 }  // namespace ssd

@@ -94,3 +94,23 @@ def test_a_strided_initial_plane_keeps_the_kernel_it_had(ops, oracle):
     y, yf = ops._fused_chunk_state_state_passing_fwd(B.half(), x.half(), dt, dA, torch.float16, initial_states=init)
     torch.testing.assert_close(y.float().cpu(), want_out, rtol=2e-3, atol=1e-3)
     torch.testing.assert_close(yf.cpu(), want_fin, rtol=2e-3, atol=1e-3)
+
+
+@pytest.mark.parametrize("nseq,L,chain", [(7, 16384, True), (0, 16384, False), (7, 8192, False)])
+def test_packed_rows_run_the_chain_kernel_beyond_the_packed_line(ops, oracle, nseq, L, chain):
+    d = oracle.make_inputs(1, b=1, L=L, H=8, init=True, nseq=nseq)
+    mv = lambda t: None if t is None else t.cuda()  # noqa: E731
+    args = [mv(d[k]) for k in ("B", "x", "dt", "dA_cumsum")]
+    kw = dict(initial_states=mv(d["initial_states"]), seq_idx=mv(d["seq_idx"]))
+    want_out, want_fin = oracle.fused_ref(d["B"], d["x"], d["dt"], d["dA_cumsum"], initial_states=d["initial_states"], seq_idx=d["seq_idx"])
+    from ssd_amd.ops import _WORKSPACES
+    calls = [lambda o=o: ops._fused_chunk_state_state_passing_fwd(*args, o, **kw) for o in (torch.float32, torch.bfloat16)]
+    calls.append(lambda: ops._fused_chunk_state_state_passing_scan_fwd(args[0], args[1], mv(d["C"]), *args[2:], return_states=False, **kw))
+    for call in calls:
+        ops.release_workspaces()
+        got = call()
+        torch.cuda.synchronize()
+        assert [k.epochs.last for k in _WORKSPACES.values()] == [int(chain)] and ops.fused_status() == 0
+        torch.testing.assert_close(got[1].cpu(), want_fin, rtol=2e-3, atol=1e-3)
+        if got[0] is not None:
+            torch.testing.assert_close(got[0].float().cpu(), want_out, rtol=2e-3 if got[0].dtype == torch.float32 else 2.0 ** -7, atol=1e-3)

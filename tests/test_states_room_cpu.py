@@ -50,3 +50,14 @@ def test_arguments_the_call_rejects_are_left_to_it():
     assert not _wants(x=torch.empty(1, 4096, 64, 8, dtype=torch.bfloat16).transpose(2, 3))
     with pytest.raises(TypeError):
         _wants(dtype=torch.float64)
+
+
+@pytest.mark.parametrize("L,H,seq,want", [
+    (8192, 8, True, True), (16384, 8, True, False), (16384, 8, False, True),        # 32 and 64 chunks
+    (6144, 16, True, True), (6400, 16, True, False), (6400, 16, False, True),       # 192 and 200 unit-chunks
+    (4096, 24, True, False), (4096, 24, False, True),                               # twelve units
+    (2048, 48, True, True),                                                         # ... and no chain kernel to compare with
+])
+def test_packed_sequences_keep_the_chain_kernel_where_its_chains_are_cut(L, H, seq, want):
+    seq = torch.zeros(1, L, dtype=torch.int32) if seq else None
+    assert _wants(L=L, H=H, seq=seq) == want and _wants(L=L, H=H, seq=seq, out=None) == want
