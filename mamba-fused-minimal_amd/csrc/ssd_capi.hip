@@ -683,8 +683,16 @@ int ssd_query_fused_wants_states(const ssd_tensor *x, const ssd_tensor *B, const
     if (rc) return rc;
     // what the call runs with a fp32 `out`, and whether it still does with the place it would be given
     const Choice c = choose(as_out, true, n_cu), given = p.out ? choose(as_states, true, n_cu) : c;
-    if (c.family == F_PAIR)
-        return given.family == F_PAIR && !(ssd::chain_supported(as_out) && chain_preferred(as_out, n_cu)) ? 1 : 0;
+    if (c.family == F_PAIR) {
+        if (given.family != F_PAIR || (ssd::chain_supported(as_out) && chain_preferred(as_out, n_cu))) return 0;
+        // Packed rows so long that a fp32 `out` runs the pair whatever the number of units: these calls have the chain
+        // kernel instead, whose chains are cut (8 heads x 512 chunks, chain against pair, us: 8 sequences 259 / 196, 128
+        // sequences 101 / 196; with the scan's state half 482 / 249 and 213 / 249).
+        if (p.seq && !ssd::cost::few_units_packed(problem_of(p, n_cu)) && ssd::chain_supported(p.out ? p : as_out) &&
+            choose(as_out, true, n_cu, false).family == F_PAIR)
+            return 0;
+        return 1;
+    }
     // The fp32 matrix kernel, which would walk the sequence otherwise, gains from four chunks on while 64 x 64 state tiles
     // give a compute unit no more than one and a half workgroups to walk with (fp16 out, walk against pair, us: 8 heads x
     // 16 chunks 48.6 / 17.9, 2 x 24 x 12 53.4 / 39.9, 4 x 48 x 12 140 / 123; 8 x 48 x 4 78.9 / 88.1; three chunks of 24

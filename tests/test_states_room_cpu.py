@@ -57,7 +57,10 @@ def test_arguments_the_call_rejects_are_left_to_it():
     (6144, 16, True, True), (6400, 16, True, False), (6400, 16, False, True),       # 192 and 200 unit-chunks
     (4096, 24, True, False), (4096, 24, False, True),                               # twelve units
     (2048, 48, True, True),                                                         # ... and no chain kernel to compare with
+    (131072, 8, True, False), (131072, 8, False, True),                             # long enough for the pair at any number of units
 ])
 def test_packed_sequences_keep_the_chain_kernel_where_its_chains_are_cut(L, H, seq, want):
     seq = torch.zeros(1, L, dtype=torch.int32) if seq else None
     assert _wants(L=L, H=H, seq=seq) == want and _wants(L=L, H=H, seq=seq, out=None) == want
+    if seq is not None:                                                             # fp16 `out`: not the chain kernel's
+        assert _wants(L=L, H=H, seq=seq, out=torch.float16) == (want or L == 131072)
