@@ -44,6 +44,23 @@ def _wants_states(x, *args):
         return _lib.host().wants_states(x, *args)
 
 
+# What a call may take for chunk states that it neither returns nor was given: twice a 16-bit ``out``.  Every size the rules
+# behind _wants_states were measured on stays below (20 heads x 512 chunks x 64 x 128: 320 MiB); beyond, and where the memory
+# is not there, the call runs on the kernel that needs no such room.
+_STATES_ROOM_BYTES = 1 << 30
+
+
+def _states_room(x, shape):
+    """An fp32 tensor of that shape on x's device, or None where that is too much.  It belongs to one call: freed behind the
+    launches on the current stream."""
+    if 4 * math.prod(shape) > _STATES_ROOM_BYTES:
+        return None
+    try:
+        return torch.empty(shape, device=x.device, dtype=torch.float32)
+    except torch.OutOfMemoryError:
+        return None
+
+
 # Workspaces of the ticket / flag-chain kernel that the wrappers keep to themselves: one per (device, stream), grown on
 # demand, with the epoch of the last launch on it.  A workspace nobody else writes to lets a call tell the library that
 # the launch before left it in order (ssd_fused_opts.epoch), which saves the fill launch in front of the kernel.
@@ -287,7 +304,7 @@ def _fused_chunk_state_state_passing_fwd(B, x, dt, dA_cumsum, out_dtype, initial
         initial_states = initial_states.contiguous()
     if (states is None and out_dtype != torch.float32 and _kernel == 0 and _workspace is None
             and _wants_states(x, B, dt, dA_cumsum, seq_idx, initial_states, out, final_states)):
-        states = torch.empty((batch, nchunks, nheads, headdim, dstate), device=x.device, dtype=torch.float32)
+        states = _states_room(x, (batch, nchunks, nheads, headdim, dstate))
 
     def launch(workspace, epoch):
         return _on_device(x, _lib.host().fused, x, B, dt, dA_cumsum, seq_idx, initial_states, states, out, final_states,
@@ -548,13 +565,14 @@ def _fused_chunk_state_state_passing_scan_fwd(B, x, C, dt, dA_cumsum, out_dtype=
     out = None
     if return_states:
         out = torch.empty((batch, nchunks, nheads, headdim, dstate), device=x.device, dtype=out_dtype or torch.float32)
-    rc = _lib.SSD_ERR_SCRATCH
-    if (out is not None or _kernel != 0 or _workspace is not None
-            or not _wants_states(x, B, dt, dA_cumsum, seq_idx, initial_states, None, final_states)):
-        rc = call(out)
+    room = None
+    if (out is None and _kernel == 0 and _workspace is None
+            and _wants_states(x, B, dt, dA_cumsum, seq_idx, initial_states, None, final_states)):
+        room = _states_room(x, (batch, nchunks, nheads, headdim, dstate))
+    rc = call(out if room is None else room)
     if rc == _lib.SSD_ERR_SCRATCH and out is None and _kernel == 0:
-        # arguments the one-launch kernel does not take, or sizes it is the slower way for (it is the chain kernel): the
-        # passed states then need a place, which this wrapper (the owner of all allocations) provides and drops again
+        # arguments the one-launch kernel does not take: the passed states then need a place, which this wrapper (the
+        # owner of all allocations) provides and drops again
         rc = call(torch.empty((batch, nchunks, nheads, headdim, dstate), device=x.device, dtype=torch.float32))
     _lib.check(rc, "ssd_fused_chunk_state_passing_scan_fwd")
     return out, final_states, y

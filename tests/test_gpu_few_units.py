@@ -114,3 +114,29 @@ def test_packed_rows_run_the_chain_kernel_beyond_the_packed_line(ops, oracle, ns
         torch.testing.assert_close(got[1].cpu(), want_fin, rtol=2e-3, atol=1e-3)
         if got[0] is not None:
             torch.testing.assert_close(got[0].float().cpu(), want_out, rtol=2e-3 if got[0].dtype == torch.float32 else 2.0 ** -7, atol=1e-3)
+
+
+def test_without_room_for_chunk_states_the_call_runs_on_its_former_kernel(ops, oracle, monkeypatch):
+    # 8 heads x 32 chunks: bf16 out and the scan call on the chain kernel, fp16 on the walk of the fp32 matrix kernel
+    d = oracle.make_inputs(1, b=1, L=8192, H=8, init=True)
+    x, B, C, dt, dA, init = (d[k].cuda() for k in ("x", "B", "C", "dt", "dA_cumsum", "initial_states"))
+    want_out, want_fin = oracle.fused_ref(d["B"], d["x"], d["dt"], d["dA_cumsum"], initial_states=d["initial_states"])
+    want_y = oracle.chunk_scan_states_ref(d["C"], want_out, d["dA_cumsum"])
+    from ssd_amd import ops as impl
+    for limit, chain in ((impl._STATES_ROOM_BYTES, 0), (1 << 20, 1)):
+        monkeypatch.setattr(impl, "_STATES_ROOM_BYTES", limit)
+        for bf16 in (True, False):
+            ops.release_workspaces()
+            out, fin = ops._fused_chunk_state_state_passing_fwd(B if bf16 else B.half(), x if bf16 else x.half(), dt, dA,
+                                                                torch.bfloat16 if bf16 else torch.float16, initial_states=init)
+            torch.cuda.synchronize()
+            assert [k.epochs.last for k in impl._WORKSPACES.values()] == [chain if bf16 else 0]
+            torch.testing.assert_close(out.float().cpu(), want_out, rtol=2.0 ** -7 if bf16 else 2e-3, atol=1e-3)
+            torch.testing.assert_close(fin.cpu(), want_fin, rtol=2e-3, atol=1e-3)
+        ops.release_workspaces()
+        none, fin, y = ops._fused_chunk_state_state_passing_scan_fwd(B, x, C, dt, dA, initial_states=init, return_states=False,
+                                                                     y_dtype=torch.float32)
+        torch.cuda.synchronize()
+        assert none is None and [k.epochs.last for k in impl._WORKSPACES.values()] == [chain] and ops.fused_status() == 0
+        torch.testing.assert_close(fin.cpu(), want_fin, rtol=2e-3, atol=1e-3)
+        torch.testing.assert_close(y.cpu(), want_y, rtol=2e-3, atol=1e-3)
