@@ -61,6 +61,15 @@ def _states_room(x, shape):
         return None
 
 
+def _room_wanted(x, B, dt, dA_cumsum, seq_idx, initial_states, out, final_states):
+    """Room for the chunk states of a fused call on these tensors where it gains from that and has none itself."""
+    if out is not None and out.dtype == torch.float32:
+        return None
+    if not _wants_states(x, B, dt, dA_cumsum, seq_idx, initial_states, out, final_states):
+        return None
+    return _states_room(x, (x.shape[0], dt.shape[2], x.shape[2], x.shape[3], B.shape[3]))
+
+
 # Workspaces of the ticket / flag-chain kernel that the wrappers keep to themselves: one per (device, stream), grown on
 # demand, with the epoch of the last launch on it.  A workspace nobody else writes to lets a call tell the library that
 # the launch before left it in order (ssd_fused_opts.epoch), which saves the fill launch in front of the kernel.
@@ -302,9 +311,18 @@ def _fused_chunk_state_state_passing_fwd(B, x, dt, dA_cumsum, out_dtype, initial
     B, x, dt, dA_cumsum, seq_idx = _prep_inputs(B, x, dt, dA_cumsum, seq_idx)
     if initial_states is not None and initial_states.stride(-1) != 1:
         initial_states = initial_states.contiguous()
-    if (states is None and out_dtype != torch.float32 and _kernel == 0 and _workspace is None
-            and _wants_states(x, B, dt, dA_cumsum, seq_idx, initial_states, out, final_states)):
-        states = _states_room(x, (batch, nchunks, nheads, headdim, dstate))
+    if states is None and _kernel == 0 and _workspace is None:
+        states = _room_wanted(x, B, dt, dA_cumsum, seq_idx, initial_states, out, final_states)
+    _fused_into(out, final_states, B, x, dt, dA_cumsum, initial_states, seq_idx, states, _clamp, _kernel, _spin_limit, _workspace,
+                _chunks_per_item, _epoch)
+    return out, final_states
+
+
+def _fused_into(out, final_states, B, x, dt, dA_cumsum, initial_states, seq_idx, states, _clamp=True, _kernel=0, _spin_limit=0,
+                _workspace=None, _chunks_per_item=0, _epoch=0):
+    """The fused call on tensors as the library takes them."""
+    batch, seqlen, nheads, headdim = x.shape
+    nchunks, dstate = out.shape[1], out.shape[4]
 
     def launch(workspace, epoch):
         return _on_device(x, _lib.host().fused, x, B, dt, dA_cumsum, seq_idx, initial_states, states, out, final_states,
@@ -316,11 +334,10 @@ def _fused_chunk_state_state_passing_fwd(B, x, dt, dA_cumsum, out_dtype, initial
     else:
         # bf16 passed states: the workspace also takes the fp32 states that cross between work items (a quarter of
         # an fp32 `out`, as a rule); with a `states` buffer the call runs on other kernels anyway
-        nbytes = _fused_workspace_need(x.device.index, (batch, seqlen, nheads, headdim, dstate, ngroups, chunk_size, nchunks),
-                                       _lib._DTYPES.get(out_dtype, -1), int(_chunks_per_item), states is not None)
+        nbytes = _fused_workspace_need(x.device.index, (batch, seqlen, nheads, headdim, dstate, B.shape[2], dt.shape[3], nchunks),
+                                       _lib._DTYPES.get(out.dtype, -1), int(_chunks_per_item), states is not None)
         rc = _launch_on_own_workspace(x, nbytes, launch, batch * nheads * ((headdim + 31) // 32) * nchunks)
     _lib.check(rc, "ssd_fused_chunk_state_passing_fwd_ws")
-    return out, final_states
 
 
 def _fused_chunk_state_state_passing_fwd_static(B, x, dt, dA_cumsum, out, final_states, initial_states=None, seq_idx=None,
@@ -408,10 +425,14 @@ def _chunk_cumsum_fwd(dt, A, chunk_size, dt_bias=None, dt_softplus=False, dt_lim
     nchunks = math.ceil(seqlen / chunk_size)
     dt_out = torch.empty(batch, nheads, nchunks, chunk_size, device=dt.device, dtype=torch.float32)
     dA_cumsum = torch.empty(batch, nheads, nchunks, chunk_size, device=dt.device, dtype=torch.float32)
-    rc = _on_device(dt, _lib.host().chunk_cumsum, dt, A, dt_bias, dt_out, dA_cumsum, int(chunk_size), int(bool(dt_softplus)),
+    _cumsum_into(dt_out, dA_cumsum, dt, A, dt_bias, dt_softplus, dt_limit)
+    return dA_cumsum, dt_out
+
+
+def _cumsum_into(dt_out, dA_cumsum, dt, A, dt_bias, dt_softplus, dt_limit):
+    rc = _on_device(dt, _lib.host().chunk_cumsum, dt, A, dt_bias, dt_out, dA_cumsum, int(dt_out.shape[-1]), int(bool(dt_softplus)),
                     float(dt_limit[0]), float(dt_limit[1]))
     _lib.check(rc, "ssd_chunk_cumsum_fwd")
-    return dA_cumsum, dt_out
 
 
 def _fused_cumsum_chunk_state_state_passing_fwd(B, x, dt, A, chunk_size, out_dtype, dt_bias=None, dt_softplus=False,
@@ -450,6 +471,12 @@ def _fused_cumsum_chunk_state_state_passing_fwd(B, x, dt, A, chunk_size, out_dty
     dA_cumsum = torch.empty(batch, nheads, nchunks, chunk_size, device=x.device, dtype=torch.float32)
     out = torch.empty((batch, nchunks, nheads, headdim, dstate), device=x.device, dtype=out_dtype or torch.float32)
     final_states = torch.empty((batch, nheads, headdim, dstate), device=x.device, dtype=torch.float32)
+    if _kernel == 0 and _workspace is None:
+        room = _room_wanted(x, B, dt_out, dA_cumsum, seq_idx, initial_states, out, final_states)
+        if room is not None:               # the C entry has no place for it: the two calls it consists of
+            _cumsum_into(dt_out, dA_cumsum, dt, A, dt_bias, dt_softplus, dt_limit)
+            _fused_into(out, final_states, B, x, dt_out, dA_cumsum, initial_states, seq_idx, room, _clamp)
+            return out, final_states, dA_cumsum, dt_out
     dims = _lib.dims_arg(batch, seqlen, nheads, headdim, dstate, ngroups, chunk_size, nchunks)
     T = _lib.tensor_arg
     lib = _lib.load()
@@ -566,9 +593,14 @@ def _fused_chunk_state_state_passing_scan_fwd(B, x, C, dt, dA_cumsum, out_dtype=
     if return_states:
         out = torch.empty((batch, nchunks, nheads, headdim, dstate), device=x.device, dtype=out_dtype or torch.float32)
     room = None
-    if (out is None and _kernel == 0 and _workspace is None
-            and _wants_states(x, B, dt, dA_cumsum, seq_idx, initial_states, None, final_states)):
-        room = _states_room(x, (batch, nchunks, nheads, headdim, dstate))
+    if _kernel == 0 and _workspace is None:
+        room = _room_wanted(x, B, dt, dA_cumsum, seq_idx, initial_states, out, final_states)
+    if room is not None and out is not None:
+        # 16-bit passed states that are wanted: the C entry takes no chunk states beside them, so the two calls it consists of
+        _fused_into(out, final_states, B, x, dt, dA_cumsum, initial_states, seq_idx, room, _clamp)
+        rc = _on_device(C, _lib.host().chunk_scan_states, C, out, dA_cumsum, seq_idx, y, int(bool(accumulate)))
+        _lib.check(rc, "ssd_chunk_scan_states_fwd")
+        return out, final_states, y
     rc = call(out if room is None else room)
     if rc == _lib.SSD_ERR_SCRATCH and out is None and _kernel == 0:
         # arguments the one-launch kernel does not take: the passed states then need a place, which this wrapper (the

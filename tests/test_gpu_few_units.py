@@ -140,3 +140,32 @@ def test_without_room_for_chunk_states_the_call_runs_on_its_former_kernel(ops, o
         assert none is None and [k.epochs.last for k in impl._WORKSPACES.values()] == [chain] and ops.fused_status() == 0
         torch.testing.assert_close(fin.cpu(), want_fin, rtol=2e-3, atol=1e-3)
         torch.testing.assert_close(y.cpu(), want_y, rtol=2e-3, atol=1e-3)
+
+
+@pytest.mark.parametrize("kw,dtype", [(dict(L=8192, H=8), "bf16"), (dict(L=2048, H=8, nseq=3), "bf16"), (dict(L=3001, H=6, P=48, N=40, Q=100), "fp16")])
+def test_the_calls_in_one_equal_the_calls_one_by_one(ops, oracle, kw, dtype):
+    # dt preparation + fused call, and fused call + scan's state half with the passed states wanted in 16 bits: the very
+    # kernels of the separate calls, also where those lend the fused call room for the chunk states
+    args = dict(b=1, G=1, init=True, dtype=dtype)
+    args.update(kw)
+    d = oracle.make_inputs(1, **args)
+    mv = lambda t: None if t is None else t.cuda()  # noqa: E731
+    x, B, C, dt, dA, init, seq = (mv(d[k]) for k in ("x", "B", "C", "dt", "dA_cumsum", "initial_states", "seq_idx"))
+    raw = dt.flatten(2).transpose(1, 2)[:, :x.shape[1]].contiguous()
+    A = -torch.rand(x.shape[2], device="cuda")
+    Q = dt.shape[-1]
+    for out_dtype in (x.dtype, torch.float32):
+        dA1, dt1 = ops._chunk_cumsum_fwd(raw, A, Q)
+        out1, fin1 = ops._fused_chunk_state_state_passing_fwd(B, x, dt1, dA1, out_dtype, initial_states=init, seq_idx=seq)
+        out, fin, dA2, dt2 = ops._fused_cumsum_chunk_state_state_passing_fwd(B, x, raw, A, Q, out_dtype, initial_states=init, seq_idx=seq)
+        assert out.dtype == out_dtype
+        for got, want in ((dA2, dA1), (dt2, dt1), (out, out1), (fin, fin1)):
+            assert torch.equal(got, want)
+        y1 = ops._chunk_scan_states_fwd(C, out1, dA1, seq_idx=seq)
+        out, fin, y = ops._fused_chunk_state_state_passing_scan_fwd(B, x, C, dt1, dA1, out_dtype, initial_states=init, seq_idx=seq)
+        assert torch.equal(out, out1) and torch.equal(fin, fin1) and torch.equal(y, y1)
+        half = torch.full_like(y, 0.25)
+        _, _, y2 = ops._fused_chunk_state_state_passing_scan_fwd(B, x, C, dt1, dA1, out_dtype, initial_states=init, seq_idx=seq, y=half,
+                                                                 accumulate=True)
+        want = ops._chunk_scan_states_fwd(C, out1, dA1, seq_idx=seq, out=torch.full_like(y, 0.25), accumulate=True)
+        assert y2 is half and torch.equal(y2, want)
