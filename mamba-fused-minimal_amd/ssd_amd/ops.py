@@ -112,7 +112,6 @@ class _Kept:
         self.tensor = tensor
         self.epochs = _Epochs()
         self.lock = threading.Lock()
-        self.used = False                  # whether the last call ran the kernel that uses it
 
 
 def _workspace_key(device, stream=None):
@@ -170,17 +169,16 @@ def _launch_on_own_workspace(x, nbytes, launch, pairs):
         epoch = ent.epochs.next(pairs)
         rc, used = launch(ent.tensor, epoch)
         ent.epochs.done(epoch, rc, used, pairs)
-        ent.used = bool(used)
         return rc
 
 
 def fused_status(device=None, stream=None):
-    """What the last fused call of this module on ``device`` and ``stream`` (defaults: the current ones) left in the
-    workspace the wrappers keep for them: waits for the stream and returns 0, or the negative ssd_status of
-    ssd_fused_workspace_status (-7 a flag wait ran out, -8 two XCDs drew from one counter, -9 a counter that owns work
-    was never served, -10 the workspace was not what the epoch promised) -- the outputs of that call are then
-    unusable.  Ask before the next fused call on the same stream, which starts the record afresh.  0 also when no call
-    has used that workspace (another kernel family served it).  The reference's fused kernels have no such report:
+    """What the last launch of the ticket / flag-chain kernel by a fused call of this module on ``device`` and ``stream``
+    (defaults: the current ones) left in the workspace the wrappers keep for them: waits for the stream and returns 0, or
+    the negative ssd_status of ssd_fused_workspace_status (-7 a flag wait ran out, -8 two XCDs drew from one counter, -9 a
+    counter that owns work was never served, -10 the workspace was not what the epoch promised) -- the outputs of that call
+    are then unusable.  The record stands until that kernel runs again on the stream (a call that another kernel family
+    serves leaves it alone); 0 also when no call has used the workspace.  The reference's fused kernels have no such report:
     their spin loops are unbounded and a failure is a hang (kernels/fused_concurrent.py:11, 300)."""
     device = torch.device("cuda", torch.cuda.current_device()) if device is None else torch.device(device)
     stream = torch.cuda.current_stream(device) if stream is None else stream
@@ -189,9 +187,6 @@ def fused_status(device=None, stream=None):
     if ent is None:
         return 0
     with ent.lock, torch.cuda.device(device):
-        if not ent.used:                   # the record is an earlier call's
-            stream.synchronize()
-            return 0
         return int(_lib.load().ssd_fused_workspace_status(ctypes.c_void_p(ent.tensor.data_ptr()),
                                                           ctypes.c_void_p(stream.cuda_stream)))
 

@@ -444,18 +444,21 @@ def test_chain_reports_a_workspace_that_is_not_what_the_epoch_promises(ops, orac
 
 def test_chain_failures_reach_the_caller_of_the_plain_wrappers(ops, oracle):
     """The drop-in wrappers keep their workspace to themselves; fused_status() is how their caller learns that the last
-    launch failed.  One poll allowed: waves give up (and still raise their flags, so the launch drains) -> -7; the next
-    call is clean."""
-    d = oracle.make_inputs(1, b=1, L=8192, H=8)
-    args = [_dev(d[k]) for k in ("B", "x", "dt", "dA_cumsum")]
+    launch failed.  One poll allowed: waves give up (and still raise their flags, so the launch drains) -> -7; the record
+    stands while other kernel families serve the calls, and the next launch of the chain kernel is clean."""
+    d, few = oracle.make_inputs(1, b=1, L=8192, H=80), oracle.make_inputs(1, b=1, L=8192, H=8)
+    of = lambda d: [_dev(d[k]) for k in ("B", "x", "dt", "dA_cumsum")]  # noqa: E731
+    from ssd_amd.ops import _WORKSPACES
     ops.release_workspaces()
     assert ops.fused_status() == 0                              # nothing kept yet
-    ops._fused_chunk_state_state_passing_fwd(*args, torch.float32, _kernel=GLOBAL, _chunks_per_item=1, _spin_limit=1)
+    ops._fused_chunk_state_state_passing_fwd(*of(d), torch.float32, _kernel=GLOBAL, _chunks_per_item=1, _spin_limit=1)
     assert ops.fused_status() == -7
-    out, fin = ops._fused_chunk_state_state_passing_fwd_concurrent(*args, torch.float32)
-    assert ops.fused_status() == 0
-    want_out, want_fin = oracle.fused_ref(d["B"], d["x"], d["dt"], d["dA_cumsum"])
-    assert _mismatches(out, want_out)[0] == 0 and _mismatches(fin, want_fin)[0] == 0
+    (kept,) = _WORKSPACES.values()
+    for d, epoch, status in ((few, 1, -7), (d, 2, 0)):          # chunk states + recurrence; the chain kernel
+        out, fin = ops._fused_chunk_state_state_passing_fwd_concurrent(*of(d), torch.float32)
+        assert list(_WORKSPACES.values()) == [kept] and kept.epochs.last == epoch and ops.fused_status() == status
+        want_out, want_fin = oracle.fused_ref(d["B"], d["x"], d["dt"], d["dA_cumsum"])
+        assert _mismatches(out, want_out)[0] == 0 and _mismatches(fin, want_fin)[0] == 0
 
 
 def test_chain_reports_xcds_that_are_not_what_it_assumed(ops, oracle):
