@@ -111,13 +111,16 @@ def test_chain_bf16_passed_states(ops, oracle, kw, kernel, r):
 def test_chain_bf16_passed_states_left_to_the_library(ops, oracle):
     # no hooks: the wrapper sizes its own workspace for bf16 `out` and the library picks the kernel (32 chunks on 40
     # units: the chain kernel); a second call reuses the workspace with the next epoch
-    d = oracle.make_inputs(2, b=1, L=8192, H=40)
+    d = oracle.make_inputs(2, b=1, L=8192, H=80)
+    from ssd_amd.ops import _WORKSPACES
+    ops.release_workspaces()
     want_out, want_fin = oracle.fused_ref(d["B"], d["x"], d["dt"], d["dA_cumsum"], initial_states=d["initial_states"])
     args = [_dev(d[k]) for k in ("B", "x", "dt", "dA_cumsum")]
     for i in range(2):
         out, fin = ops._fused_chunk_state_state_passing_fwd(*args, torch.bfloat16, initial_states=_dev(d["initial_states"]))
         torch.cuda.synchronize()
         assert out.dtype == torch.bfloat16
+        assert [k.epochs.last for k in _WORKSPACES.values()] == [i + 1] and ops.fused_status() == 0
         bad, worst = _mismatches(out, want_out, rtol=RTOL + 2.0 ** -8)
         assert bad == 0, f"call {i}: out {bad} mismatches, max {worst:.3e}"
         bad, worst = _mismatches(fin, want_fin)

@@ -1,5 +1,6 @@
 """Few state tiles and four or more chunks: chunk states + recurrence in front of the kernels that walk a sequence.  Both
-sides of the rule's lines, every form of the call that it now takes, against the token-split kernel on the same inputs."""
+sides of the rule's lines, every form of the call that it takes, against the token-split kernel on the same inputs and
+against the oracle."""
 import pytest
 import torch
 
@@ -23,7 +24,7 @@ def ops():
     (dict(L=1400, H=4, G=2, Q=128), True),                 # chunk 128, grouped B, ragged
     (dict(L=3840, H=51), True),                            # 25 units, 15 chunks: a tenth of 256, below three unit-chunks per compute unit
     (dict(L=2048, H=54), False),                           # 27 units
-    (dict(L=16384, H=24), False),                          # three unit-chunks per compute unit, 12 units
+    (dict(L=16384, H=24), False),                          # three unit-chunks per compute unit, 12 units: the chain kernel
     (dict(L=24576, H=20), True),                           # ten units, any length
 ], ids=lambda v: "-".join(f"{k}{x}" for k, x in v.items()) if isinstance(v, dict) else str(v))
 def test_few_units(ops, oracle, kw, pair):
@@ -42,13 +43,18 @@ def test_few_units(ops, oracle, kw, pair):
         want_y = ops._chunk_scan_states_fwd(mv(d["C"]), want, dA, seq_idx=seq, out_dtype=torch.float32)
     finally:
         ops.set_token_split(old)
+    o_out, o_fin = oracle.fused_ref(d["B"], d["x"], d["dt"], d["dA_cumsum"], initial_states=d["initial_states"], seq_idx=d["seq_idx"])
+    torch.testing.assert_close(want.cpu(), o_out, rtol=2e-3, atol=1e-3)
+    torch.testing.assert_close(want_fin.cpu(), o_fin, rtol=2e-3, atol=1e-3)
     # both sides split x * w into bf16 hi + lo (2^-17 of every product) and add in fp32 in another order
     tol = dict(rtol=1e-4, atol=1e-4)
     for out_dtype in (torch.float32, torch.bfloat16, torch.float16):
         out, fin = fused(B, x, dt, dA, out_dtype, initial_states=init, seq_idx=seq)
         assert out.dtype == out_dtype and fin.dtype == torch.float32
+        torch.testing.assert_close(fin.cpu(), o_fin, rtol=2e-3, atol=1e-3)
         if out_dtype == torch.float32:
             torch.testing.assert_close(out, want, **tol)
+            torch.testing.assert_close(out.cpu(), o_out, rtol=2e-3, atol=1e-3)
         else:
             torch.testing.assert_close(out.float(), want, rtol=2.0 ** (-7 if out_dtype == torch.bfloat16 else -10), atol=1e-4)
         torch.testing.assert_close(fin, want_fin, **tol)

@@ -119,8 +119,11 @@ def test_fused_scan_sequence_starts_everywhere(ops, oracle):
 
 
 def test_fused_scan_equals_the_two_calls(ops, oracle):
-    # the one-launch result against the library's own fused call followed by its stand-alone consumer
-    d = oracle.make_inputs(2, b=2, L=4096, H=16)
+    # the one-launch result against the library's own fused call followed by its stand-alone consumer; units enough that the
+    # library itself chooses the one launch where no passed states are wanted
+    d = oracle.make_inputs(2, b=4, L=4096, H=80)
+    from ssd_amd.ops import _WORKSPACES
+    ops.release_workspaces()
     args = [_dev(d[k]) for k in ("B", "x")]
     Cd, dtd, dAd, initd = _dev(d["C"]), _dev(d["dt"]), _dev(d["dA_cumsum"]), _dev(d["initial_states"])
     out2, fin2 = ops._fused_chunk_state_state_passing_fwd(*args, dtd, dAd, torch.float32, initial_states=initd)
@@ -137,11 +140,17 @@ def test_fused_scan_equals_the_two_calls(ops, oracle):
                                                                    y_dtype=torch.float32)
     torch.cuda.synchronize()
     assert torch.equal(out3, out2) and torch.equal(fin3, fin2) and torch.equal(y3, y2)
-    # ... and without `out` it is the one launch
+    # ... and without `out` it is the one launch, on the workspace the wrapper keeps: a launch of the chain kernel more, and a
+    # kernel that wrote no passed states (the room for them would be 168 MB)
+    before = max(k.epochs.last for k in _WORKSPACES.values())
+    torch.cuda.reset_peak_memory_stats()
+    held = torch.cuda.memory_allocated()
     none, fin4, y4 = ops._fused_chunk_state_state_passing_scan_fwd(*args, Cd, dtd, dAd, torch.float32, initial_states=initd,
                                                                    y_dtype=torch.float32, return_states=False)
     torch.cuda.synchronize()
-    assert none is None and ops.fused_status() == 0
+    (kept,) = _WORKSPACES.values()
+    assert none is None and ops.fused_status() == 0 and kept.epochs.last in (1, before + 1)
+    assert torch.cuda.max_memory_allocated() - held < fin4.numel() * 4 + y4.numel() * 4 + kept.tensor.numel() * 4 + (1 << 20)
     assert float((fin4 - fin2).abs().max()) <= 1e-4 and float((y4 - y2).abs().max()) <= 2e-3
 
 

@@ -42,6 +42,29 @@ def test_recurrence_around_its_groups_and_windows(ops, chunks, heads, dim, packe
     torch.testing.assert_close(fin.cpu().double(), s, **tol)
 
 
+@pytest.mark.parametrize("chunks", [5, 20, 80])            # four, eight and sixteen chunks in flight
+@pytest.mark.parametrize("dim,gap", [(260, 0), (260, 12), (260, 3), (7, 2)])     # planes apart: 4-element loads, then single ones
+@pytest.mark.parametrize("dtype,out_dtype", [(torch.bfloat16, torch.bfloat16), (torch.float16, torch.float32), (torch.float32, torch.float16)])
+def test_recurrence_over_16_bit_and_strided_planes(ops, chunks, dim, gap, dtype, out_dtype):
+    g = torch.Generator().manual_seed(chunks + dim)
+    b, heads = 2, 3
+    wide = torch.randn(b, chunks, heads, dim + gap, generator=g).to(dtype)
+    states = wide[..., :dim]
+    da = -torch.rand(b, heads, chunks, generator=g)
+    init = torch.randn(b, heads, dim + gap, generator=g)[..., :dim]
+    s, want = init.double(), []
+    for c in range(chunks):
+        want.append(s)
+        s = torch.exp(da[:, :, c].double())[..., None] * s + states[:, c].double()
+    want = torch.stack(want, dim=1)
+    out, fin = ops._state_passing_fwd(wide.cuda()[..., :dim], da.cuda(), initial_states=init.cuda(), out_dtype=out_dtype)
+    assert out.dtype == out_dtype and fin.dtype == torch.float32
+    # the sums are fp32 whatever the planes are stored as; a 16-bit `out` rounds once on its way
+    torch.testing.assert_close(fin.cpu().double(), s, rtol=1e-5, atol=1e-5)
+    half = {torch.float32: 0.0, torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11}[out_dtype]
+    torch.testing.assert_close(out.cpu().double(), want, rtol=1e-5 + half, atol=1e-5)
+
+
 @pytest.mark.parametrize("L", [16, 64 * 5, 64 * 70 + 1])
 def test_in_place_behind_the_chunk_states(ops, oracle, L):
     # fp32 inputs: the chunk states are written into `out` and turned into the passed states there
