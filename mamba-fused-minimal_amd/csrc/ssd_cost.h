@@ -108,9 +108,12 @@ inline double pair_us(const Problem &q)
 //     32         12.0 / 10.6   21.5 / 15.8   46.6 / 24.9   65.2 / 31.7   92.1 / 57.2   100.5 / 114.2
 //     48         13.0 / 13.1   22.3 / 20.6   46.3 / 28.6   65.2 / 42.7   95.7 / 86.5   154.8 / 174.6
 //     80                       24.1 / 24.8   41.3 / 38.4
-// (fewer than four chunks: 24 heads x 2, 7.6 / 8.3).  Hence: up to a tenth as many units as compute units while there are
-// fewer than three unit-chunks per compute unit, and any length below a twenty-fourth; between the two lines the
-// estimates decide as they do for more units (they keep 24 heads x 64 chunks on the chain kernel, 92.7 / 44.7).
+// (fewer than four chunks: 24 heads x 2, 7.6 / 8.3; no seq_idx).  The lines are drawn inside what was measured: up to a
+// tenth as many units as compute units while there are fewer than three unit-chunks per compute unit, and any length below a
+// twenty-fourth.  With dstate 64, chunk 128 or batches the pair is ahead inside them too (48 heads x 8 chunks of 128: as
+// fast).  They are not where the pair stops paying: beyond them it is no candidate until there are 32 state-tile chunks per
+// compute unit (choose in ssd_capi.hip), so that 32 heads x 64 chunks, 48 x 32, 48 x 64 and 24 x 64 (92.7 / 44.7) stay on the
+// chain kernel although the table or the estimates have the pair ahead.
 inline bool few_units(const Problem &q)
 {
     if (q.chunks < 4) return false;
@@ -118,20 +121,21 @@ inline bool few_units(const Problem &q)
 }
 
 // The same against the chain kernel for packed sequences (seq_idx): its chains are then as long as a sequence, and how
-// long those are only the device knows, so the pair goes in front only where it is no slower with a sequence start in
-// every chunk.  Chain kernel with four starts a chunk against the pair, us -- fp32 out, bf16 out, call with the scan's
-// state half:
-//     heads x chunks      dstate 128, chunk 256                      dstate 64, chunk 128
-//     8 x 32              33.0 / 19.9   33.9 / 22.3   42.2 / 30.1    19.9 / 14.2   20.2 / 16.9   24.0 / 22.1
-//     16 x 24 (one start) 35.3 / 23.6   36.0 / 24.9   45.2 / 34.1    21.4 / 15.0   21.7 / 16.9   26.1 / 23.8
-//     12 x 32 (chunk 128) 24.6 / 21.9   25.4 / 24.0   31.0 / 32.1    19.7 / 16.4   20.0 / 18.9   24.6 / 25.2
-//     20 x 32             35.2 / 29.3   35.6 / 31.3   44.8 / 46.2    20.3 / 20.4   20.4 / 22.5   26.3 / 29.8
-//     8 x 64              34.1 / 32.7   34.4 / 37.3   43.8 / 44.0    20.4 / 24.2   20.6 / 29.6   25.6 / 33.3
-// (with four sequences in a row the pair is ahead to 512 chunks: 4 heads x 512 260 / 127, 16 heads x 64 60.5 / 37.9; with
-// 64 of them 4 heads x 512 are 67.5 / 126.)
+// long those are only the device knows, so the pair goes in front only where it does not lose with a sequence start in
+// every chunk.  The chain kernel's time is then that of its busiest compute unit's items, the pair's grows with the
+// chunks of a row and with all unit-chunks, so the two lines scale with the work of a unit-chunk.  At the lines, one start
+// / four starts a chunk, chain kernel against pair, us:
+//     dstate, chunk   heads x chunks   fp32 out                     bf16 out                     call with the scan's state half
+//     128, 256         4 x 64          35.2 / 25.4   33.7 / 25.6    36.3 / 30.7   34.5 / 30.8    46.9 / 33.8   42.4 / 33.9
+//                      8 x 57          37.7 / 30.9   34.0 / 30.8    38.7 / 34.1   34.3 / 34.0    49.4 / 42.5   43.6 / 41.9
+//                     20 x 23          36.3 / 25.4   34.3 / 25.4    36.9 / 26.0   34.7 / 26.0    46.4 / 36.2   44.0 / 35.8
+//     128, 128         8 x 41          26.4 / 22.5   24.6 / 22.5    27.2 / 25.4   25.5 / 25.4    34.0 / 32.4   30.4 / 32.5
+//     64, 128          8 x 33          21.0 / 15.1   19.6 / 15.1    21.6 / 17.8   19.8 / 17.8    26.4 / 23.5   24.1 / 23.6
+// and beyond them: 8 x 64 34.1 / 32.7 (four starts), bf16 34.4 / 37.3; 16 x 128 in 64 sequences 46.0 / 64.2; 4 x 512 in 4, 16
+// and 64 sequences 260 / 127, 121 / 127 and 69 / 126.
 inline bool few_units_packed(const Problem &q)
 {
-    return few_units(q) && q.units * 24 <= q.n_cu && q.chunks <= 32 && q.units * q.chunks * 4 <= 3 * (int64_t)q.n_cu;
+    return few_units(q) && q.units * 24 <= q.n_cu && q.chunks <= 64 * work(q) && (double)(q.units * q.chunks) <= 0.9 * work(q) * q.n_cu;
 }
 
 }  // namespace cost

@@ -53,8 +53,9 @@ def test_arguments_the_call_rejects_are_left_to_it():
 
 
 @pytest.mark.parametrize("L,H,seq,want", [
-    (8192, 8, True, True), (16384, 8, True, False), (16384, 8, False, True),        # 32 and 64 chunks
-    (6144, 16, True, True), (6400, 16, True, False), (6400, 16, False, True),       # 192 and 200 unit-chunks
+    (14592, 8, True, True), (14848, 8, True, False), (16384, 8, False, True),       # 57 and 58 chunks on four units
+    (16384, 4, True, True), (16640, 4, True, False), (16640, 4, False, True),       # 64 and 65 chunks
+    (7168, 16, True, True), (7424, 16, True, False), (7424, 16, False, True),       # 28 and 29 chunks on eight units
     (4096, 24, True, False), (4096, 24, False, True),                               # twelve units
     (2048, 48, True, True),                                                         # ... and no chain kernel to compare with
     (131072, 8, True, False), (131072, 8, False, True),                             # long enough for the pair at any number of units
