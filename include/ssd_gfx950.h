@@ -117,11 +117,12 @@ int ssd_state_passing_fwd(const ssd_tensor *states, const ssd_tensor *dA_chunk, 
  * With few state tiles (batch * nheads * headdim / 32 below 512) and many chunks the call runs as a chunk-state launch
  * that keeps every compute unit busy plus a streaming recurrence; that needs a place for the chunk states: a fp32
  * `out` serves as one (the recurrence then works in place), and so does a fp32 `states` buffer.  The same holds for few
- * tiles and four or more chunks, where that pair also goes in front of the kernel that takes a workspace.  With a 16-bit `out`
- * and no `states` such a problem stays on the kernel with one workgroup per tile, which is slower (the library never
- * allocates): a caller in that position gains by passing `states`.  Arguments that only the fp32 matrix kernel takes
- * (fp32 or fp16 x / B, sizes off the MFMA tiling) run as the same two launches from two chunks upwards, given a fp32
- * `out` or a fp32 `states`.
+ * tiles and four or more chunks, where that pair also goes in front of the kernel that takes a workspace (with seq_idx only
+ * while the row is short: that kernel gains from sequence starts).  With a 16-bit `out` and no `states` such a problem
+ * stays on the kernel with one workgroup per tile, or on the one that takes the workspace, which is slower (the library
+ * never allocates): a caller in that position gains by passing `states`; ssd_query_fused_wants_states says when.
+ * Arguments that only the fp32 matrix kernel takes (fp32 or fp16 x / B, sizes off the MFMA tiling) run as the same two
+ * launches from two chunks upwards, given a fp32 `out` or a fp32 `states`.
  */
 int ssd_fused_chunk_state_passing_fwd(const ssd_tensor *x, const ssd_tensor *B, const ssd_tensor *dt,
                                       const ssd_tensor *dA_cumsum, const ssd_tensor *seq_idx,
@@ -254,7 +255,7 @@ int ssd_query_path(const ssd_tensor *x, const ssd_tensor *B, const ssd_dims *dim
  * kernels by an estimate of their duration (a fit to measured times, per compute unit) and this call returns the
  * ranking.  Assumed: bf16 x / B, fp32 dt / dA_cumsum / out / final_states, contiguous, no `states` output -- the
  * arguments every family covers.  has_workspace != 0 asks about ssd_fused_chunk_state_passing_fwd_ws with a
- * workspace of ssd_fused_workspace_bytes(dims) and SSD_KERNEL_AUTO, 0 about ssd_fused_chunk_state_passing_fwd.
+ * workspace of ssd_fused_workspace_bytes(dims) and SSD_KERNEL_AUTO, 0 about ssd_fused_chunk_state_passing_fwd; no seq_idx.
  * compute_units: of the device the call would run on; 0 = 256 (MI355X).  Pure host logic: touches no device and
  * launches nothing, so it also answers on a machine without a GPU.  No counterpart in the reference, whose two fused
  * wrappers each have one kernel (kernels/fused_globalbar.py:201-266, kernels/fused_concurrent.py:255-331).

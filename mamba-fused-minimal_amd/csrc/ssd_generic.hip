@@ -2,15 +2,17 @@
 // kernels do not take: fp32 and fp16 inputs, any headdim, dstate, chunk size and alignment.  The weighted x and B enter
 // v_mfma_f32_16x16x4_f32 as fp32 values and every sum is fp32, so fp32 inputs keep fp32 accuracy.
 //
-// What bounds it: the fp32 matrix instructions (256 flop per clock and compute unit, a sixteenth of bf16's) -- fp32, batch
-// 2 x 2048 tokens x 24 heads x 64 x 128: 1.6 GFLOP, 10 us, and 41 MB, 8 us; 21 us measured, the matrix units 58 % busy (an
-// FMA kernel that staged both operands through LDS: 92 us); fp16, batch 8 x 3001 x 48 heads: 18.9 GFLOP in 187 us.  So
-// the operands must cost next to no issue slots: a lane loads A consecutive headdim elements of one token's x row and S consecutive dstate elements of its B
-// row with one load each, and that *is* the operand layout -- lane i of a 16-lane group stands for rows A i .. A i + A-1
-// and columns S i .. S i + S-1 of the tile, the four lane groups for four consecutive tokens, and matrix instruction
-// (r, s) multiplies the r-th element of every x vector with the s-th of every B vector.  No LDS on the way in, no
-// barrier in the loop, whole rows per load; the accumulators of one lane are S consecutive columns, so rows leave as
-// vectors as well.
+// Where its time goes: the fp32 matrix instructions (256 flop per clock and compute unit, a sixteenth of bf16's) are the
+// largest part -- fp32, batch 2 x 2048 tokens x 24 heads x 64 x 128: 1.6 GFLOP, 10 us, and 41 MB, 8 us; 21 us measured (an
+// FMA kernel that staged both operands through LDS: 92 us); fp16, batch 8 x 3001 x 48 heads: 18.9 GFLOP in 187 us.  The
+// matrix units are busy 56 % of that fp32 launch; a wave waits 64 % of its clocks to issue, with three of them on a SIMD, and
+// 19 % in s_waitcnt, and the rest of the launch is where the waves of a SIMD start, or add up and store, together.  So the
+// operands must cost next to no issue slots: a lane loads A consecutive headdim elements of one token's x row and S
+// consecutive dstate elements of its B row with one load each, and that *is* the operand layout -- lane i of a 16-lane group
+// stands for rows A i .. A i + A-1 and columns S i .. S i + S-1 of the tile, the four lane groups for four consecutive tokens,
+// and matrix instruction (r, s) multiplies the r-th element of every x vector with the s-th of every B vector.  No LDS on the
+// way in, no barrier in the loop, whole rows per load; the accumulators of one lane are S consecutive columns, so rows leave
+// as vectors as well.
 //
 // One workgroup owns a (16 A) x (16 S) tile of one (batch, head) and chunk; its SPLIT = 4 waves take a quarter of the
 // chunk's tokens each and add up through LDS, after which wave v holds accumulator q = v of every instruction.  In
