@@ -35,39 +35,37 @@ def _on_device(t, call, *args):
         return call(*args, _raw_stream(index))
 
 
-def _wants_states(x, *args):
-    """Whether the fused call on these tensors gains from a place for fp32 chunk states (ssd_query_fused_wants_states):
-    chunk states + recurrence is then the faster way, and neither a 16-bit nor an absent ``out`` is such a place."""
-    if x.device.index == torch.cuda.current_device():
-        return _lib.host().wants_states(x, *args)
-    with torch.cuda.device(x.device.index):
-        return _lib.host().wants_states(x, *args)
-
-
 # What a call may take for chunk states that it neither returns nor was given: twice a 16-bit ``out``.  Every size the rules
 # behind _wants_states were measured on stays below (20 heads x 512 chunks x 64 x 128: 320 MiB); beyond, and where the memory
 # is not there, the call runs on the kernel that needs no such room.
 _STATES_ROOM_BYTES = 1 << 30
 
 
-def _states_room(x, shape):
+def _states_room(x, batch, nchunks, nheads, headdim, dstate):
     """An fp32 tensor of that shape on x's device, or None where that is too much.  It belongs to one call: freed behind the
     launches on the current stream."""
-    if 4 * math.prod(shape) > _STATES_ROOM_BYTES:
+    if 4 * batch * nchunks * nheads * headdim * dstate > _STATES_ROOM_BYTES:
         return None
     try:
-        return torch.empty(shape, device=x.device, dtype=torch.float32)
+        return torch.empty((batch, nchunks, nheads, headdim, dstate), device=x.device, dtype=torch.float32)
     except torch.OutOfMemoryError:
         return None
 
 
-def _room_wanted(x, B, dt, dA_cumsum, seq_idx, initial_states, out, final_states):
-    """Room for the chunk states of a fused call on these tensors where it gains from that and has none itself."""
-    if out is not None and out.dtype == torch.float32:
+def _room_wanted(sizes, x, B, dt, dA_cumsum, seq_idx, initial_states, out, final_states):
+    """Room for the chunk states of a fused call on these tensors where it gains from that (ssd_query_fused_wants_states;
+    never below four chunks): chunk states + recurrence is then the faster way, and neither a 16-bit nor an absent ``out``
+    is a place for them."""
+    batch, _, nheads, headdim, dstate, _, _, nchunks = sizes
+    if nchunks < 4:
         return None
-    if not _wants_states(x, B, dt, dA_cumsum, seq_idx, initial_states, out, final_states):
-        return None
-    return _states_room(x, (x.shape[0], dt.shape[2], x.shape[2], x.shape[3], B.shape[3]))
+    index = x.device.index
+    if index == torch.cuda.current_device():
+        wanted = _lib.host().wants_states(x, B, dt, dA_cumsum, seq_idx, initial_states, out, final_states)
+    else:
+        with torch.cuda.device(index):
+            wanted = _lib.host().wants_states(x, B, dt, dA_cumsum, seq_idx, initial_states, out, final_states)
+    return _states_room(x, batch, nchunks, nheads, headdim, dstate) if wanted else None
 
 
 # Workspaces of the ticket / flag-chain kernel that the wrappers keep to themselves: one per (device, stream), grown on
@@ -120,13 +118,12 @@ def _workspace_key(device, stream=None):
 
 
 @functools.lru_cache(maxsize=1024)
-def _fused_workspace_need(device, sizes, out_code, chunks_per_item, pairs_only):
+def _fused_workspace_need(device, sizes, out_code, chunks_per_item):
     """Bytes of workspace for a fused call of these sizes: a question about sizes only, asked once.  0 = that kernel is not
     offered for these arguments, its plain workspace then."""
     lib = _lib.load()
     dims = _lib.dims_arg(*sizes)
-    nbytes = 0 if pairs_only else int(lib.ssd_fused_workspace_bytes_for(dims, out_code, chunks_per_item))
-    return nbytes or int(lib.ssd_fused_workspace_bytes(dims))
+    return int(lib.ssd_fused_workspace_bytes_for(dims, out_code, chunks_per_item)) or int(lib.ssd_fused_workspace_bytes(dims))
 
 
 @functools.lru_cache(maxsize=1024)
@@ -306,32 +303,29 @@ def _fused_chunk_state_state_passing_fwd(B, x, dt, dA_cumsum, out_dtype, initial
     B, x, dt, dA_cumsum, seq_idx = _prep_inputs(B, x, dt, dA_cumsum, seq_idx)
     if initial_states is not None and initial_states.stride(-1) != 1:
         initial_states = initial_states.contiguous()
-    if states is None and _kernel == 0 and _workspace is None:
-        states = _room_wanted(x, B, dt, dA_cumsum, seq_idx, initial_states, out, final_states)
-    _fused_into(out, final_states, B, x, dt, dA_cumsum, initial_states, seq_idx, states, _clamp, _kernel, _spin_limit, _workspace,
-                _chunks_per_item, _epoch)
+    sizes = (batch, seqlen, nheads, headdim, dstate, ngroups, chunk_size, nchunks)
+    if out_dtype != torch.float32 and states is None and _kernel == 0 and _workspace is None:
+        states = _room_wanted(sizes, x, B, dt, dA_cumsum, seq_idx, initial_states, out, final_states)
+    _fused_into(sizes, out, final_states, B, x, dt, dA_cumsum, initial_states, seq_idx, states, _clamp, _kernel, _spin_limit,
+                _workspace, _chunks_per_item, _epoch)
     return out, final_states
 
 
-def _fused_into(out, final_states, B, x, dt, dA_cumsum, initial_states, seq_idx, states, _clamp=True, _kernel=0, _spin_limit=0,
+def _fused_into(sizes, out, final_states, B, x, dt, dA_cumsum, initial_states, seq_idx, states, _clamp, _kernel=0, _spin_limit=0,
                 _workspace=None, _chunks_per_item=0, _epoch=0):
-    """The fused call on tensors as the library takes them."""
-    batch, seqlen, nheads, headdim = x.shape
-    nchunks, dstate = out.shape[1], out.shape[4]
-
+    """The fused call on tensors as the library takes them.  sizes: those of ssd_dims."""
     def launch(workspace, epoch):
+        address, nbytes = (0, 0) if workspace is None else (workspace.data_ptr(), workspace.numel() * 4)
         return _on_device(x, _lib.host().fused, x, B, dt, dA_cumsum, seq_idx, initial_states, states, out, final_states,
-                          1 if _clamp else 0, workspace.data_ptr(), workspace.numel() * 4, int(_spin_limit), int(_kernel),
-                          int(_chunks_per_item), int(epoch))
+                          1 if _clamp else 0, address, nbytes, int(_spin_limit), int(_kernel), int(_chunks_per_item), int(epoch))
 
-    if _workspace is not None:
+    if _workspace is not None or states is not None:       # (no kernel that writes chunk states uses a workspace)
         rc = launch(_workspace, _epoch)[0]
     else:
         # bf16 passed states: the workspace also takes the fp32 states that cross between work items (a quarter of
-        # an fp32 `out`, as a rule); with a `states` buffer the call runs on other kernels anyway
-        nbytes = _fused_workspace_need(x.device.index, (batch, seqlen, nheads, headdim, dstate, B.shape[2], dt.shape[3], nchunks),
-                                       _lib._DTYPES.get(out.dtype, -1), int(_chunks_per_item), states is not None)
-        rc = _launch_on_own_workspace(x, nbytes, launch, batch * nheads * ((headdim + 31) // 32) * nchunks)
+        # an fp32 `out`, as a rule)
+        nbytes = _fused_workspace_need(x.device.index, sizes, _lib._DTYPES.get(out.dtype, -1), int(_chunks_per_item))
+        rc = _launch_on_own_workspace(x, nbytes, launch, sizes[0] * sizes[2] * ((sizes[3] + 31) // 32) * sizes[7])
     _lib.check(rc, "ssd_fused_chunk_state_passing_fwd_ws")
 
 
@@ -466,13 +460,14 @@ def _fused_cumsum_chunk_state_state_passing_fwd(B, x, dt, A, chunk_size, out_dty
     dA_cumsum = torch.empty(batch, nheads, nchunks, chunk_size, device=x.device, dtype=torch.float32)
     out = torch.empty((batch, nchunks, nheads, headdim, dstate), device=x.device, dtype=out_dtype or torch.float32)
     final_states = torch.empty((batch, nheads, headdim, dstate), device=x.device, dtype=torch.float32)
-    if _kernel == 0 and _workspace is None:
-        room = _room_wanted(x, B, dt_out, dA_cumsum, seq_idx, initial_states, out, final_states)
+    sizes = (batch, seqlen, nheads, headdim, dstate, ngroups, chunk_size, nchunks)
+    if out.dtype != torch.float32 and _kernel == 0 and _workspace is None:
+        room = _room_wanted(sizes, x, B, dt_out, dA_cumsum, seq_idx, initial_states, out, final_states)
         if room is not None:               # the C entry has no place for it: the two calls it consists of
             _cumsum_into(dt_out, dA_cumsum, dt, A, dt_bias, dt_softplus, dt_limit)
-            _fused_into(out, final_states, B, x, dt_out, dA_cumsum, initial_states, seq_idx, room, _clamp)
+            _fused_into(sizes, out, final_states, B, x, dt_out, dA_cumsum, initial_states, seq_idx, room, _clamp)
             return out, final_states, dA_cumsum, dt_out
-    dims = _lib.dims_arg(batch, seqlen, nheads, headdim, dstate, ngroups, chunk_size, nchunks)
+    dims = _lib.dims_arg(*sizes)
     T = _lib.tensor_arg
     lib = _lib.load()
 
@@ -588,11 +583,11 @@ def _fused_chunk_state_state_passing_scan_fwd(B, x, C, dt, dA_cumsum, out_dtype=
     if return_states:
         out = torch.empty((batch, nchunks, nheads, headdim, dstate), device=x.device, dtype=out_dtype or torch.float32)
     room = None
-    if _kernel == 0 and _workspace is None:
-        room = _room_wanted(x, B, dt, dA_cumsum, seq_idx, initial_states, out, final_states)
+    if (out is None or out.dtype != torch.float32) and _kernel == 0 and _workspace is None:
+        room = _room_wanted(sizes, x, B, dt, dA_cumsum, seq_idx, initial_states, out, final_states)
     if room is not None and out is not None:
         # 16-bit passed states that are wanted: the C entry takes no chunk states beside them, so the two calls it consists of
-        _fused_into(out, final_states, B, x, dt, dA_cumsum, initial_states, seq_idx, room, _clamp)
+        _fused_into(sizes, out, final_states, B, x, dt, dA_cumsum, initial_states, seq_idx, room, _clamp)
         rc = _on_device(C, _lib.host().chunk_scan_states, C, out, dA_cumsum, seq_idx, y, int(bool(accumulate)))
         _lib.check(rc, "ssd_chunk_scan_states_fwd")
         return out, final_states, y

@@ -116,7 +116,7 @@ def test_packed_rows_run_the_chain_kernel_beyond_the_packed_line(ops, oracle, ns
         ops.release_workspaces()
         got = call()
         torch.cuda.synchronize()
-        assert [k.epochs.last for k in _WORKSPACES.values()] == [int(chain)] and ops.fused_status() == 0
+        assert max((k.epochs.last for k in _WORKSPACES.values()), default=0) == int(chain) and ops.fused_status() == 0
         torch.testing.assert_close(got[1].cpu(), want_fin, rtol=2e-3, atol=1e-3)
         if got[0] is not None:
             torch.testing.assert_close(got[0].float().cpu(), want_out, rtol=2e-3 if got[0].dtype == torch.float32 else 2.0 ** -7, atol=1e-3)
@@ -136,14 +136,15 @@ def test_without_room_for_chunk_states_the_call_runs_on_its_former_kernel(ops, o
             out, fin = ops._fused_chunk_state_state_passing_fwd(B if bf16 else B.half(), x if bf16 else x.half(), dt, dA,
                                                                 torch.bfloat16 if bf16 else torch.float16, initial_states=init)
             torch.cuda.synchronize()
-            assert [k.epochs.last for k in impl._WORKSPACES.values()] == [chain if bf16 else 0]
+            assert max((k.epochs.last for k in impl._WORKSPACES.values()), default=0) == (chain if bf16 else 0)
             torch.testing.assert_close(out.float().cpu(), want_out, rtol=2.0 ** -7 if bf16 else 2e-3, atol=1e-3)
             torch.testing.assert_close(fin.cpu(), want_fin, rtol=2e-3, atol=1e-3)
         ops.release_workspaces()
         none, fin, y = ops._fused_chunk_state_state_passing_scan_fwd(B, x, C, dt, dA, initial_states=init, return_states=False,
                                                                      y_dtype=torch.float32)
         torch.cuda.synchronize()
-        assert none is None and [k.epochs.last for k in impl._WORKSPACES.values()] == [chain] and ops.fused_status() == 0
+        assert none is None and max((k.epochs.last for k in impl._WORKSPACES.values()), default=0) == chain
+        assert ops.fused_status() == 0
         torch.testing.assert_close(fin.cpu(), want_fin, rtol=2e-3, atol=1e-3)
         torch.testing.assert_close(y.cpu(), want_y, rtol=2e-3, atol=1e-3)
 

@@ -70,11 +70,11 @@ def test_packed_sequences_keep_the_chain_kernel_where_its_chains_are_cut(L, H, s
 def test_room_is_bounded_and_a_call_does_without_it(monkeypatch):
     from ssd_amd import ops as impl
     x = torch.empty(1)
-    assert impl._states_room(x, (1, 16, 8, 64, 128)).shape == (1, 16, 8, 64, 128)
+    assert impl._states_room(x, 1, 16, 8, 64, 128).shape == (1, 16, 8, 64, 128)
     def full(*args, **kw):
         raise torch.OutOfMemoryError("no memory")
     monkeypatch.setattr(impl.torch, "empty", full)
-    assert impl._states_room(x, (1, 16, 8, 64, 128)) is None                # the memory is not there
+    assert impl._states_room(x, 1, 16, 8, 64, 128) is None                # the memory is not there
     monkeypatch.setattr(impl.torch, "empty", lambda *args, **kw: pytest.fail("more than the bound was asked for"))
     limit = impl._STATES_ROOM_BYTES // (4 * 8 * 64 * 128)
-    assert impl._states_room(x, (1, limit + 1, 8, 64, 128)) is None
+    assert impl._states_room(x, 1, limit + 1, 8, 64, 128) is None
