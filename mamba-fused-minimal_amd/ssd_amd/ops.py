@@ -7,6 +7,7 @@ Same names, positional order, defaults, shape asserts and output shapes/dtypes a
   kernels/fused_concurrent.py:255-331      _fused_chunk_state_state_passing_fwd_concurrent
 of the reference.  The wrappers own allocation and argument checking; the arithmetic runs in the gfx950 HIP
 kernels behind the C ABI of libssd_gfx950.so, asynchronously on the current torch stream."""
+import contextlib
 import ctypes
 import functools
 import math
@@ -36,8 +37,8 @@ def _on_device(t, call, *args):
 
 
 # What a call may take for chunk states that it neither returns nor was given: twice a 16-bit ``out``.  Every size the rules
-# behind _wants_states were measured on stays below (20 heads x 512 chunks x 64 x 128: 320 MiB); beyond, and where the memory
-# is not there, the call runs on the kernel that needs no such room.
+# behind ssd_query_fused_wants_states were measured on stays below (20 heads x 512 chunks x 64 x 128: 320 MiB); beyond, and
+# where the memory is not there, the call runs on the kernel that needs no such room.
 _STATES_ROOM_BYTES = 1 << 30
 
 
@@ -104,12 +105,18 @@ class _Epochs:
 
 class _Kept:
     """A workspace the wrappers keep for one (device, stream), the epochs of the launches on it and the lock that
-    keeps those launches in order (epochs must reach the stream in the order they were handed out)."""
+    keeps those launches in order (epochs must reach the stream in the order they were handed out).  before: the smaller
+    one it replaces, whose lock and last record it takes over."""
 
-    def __init__(self, tensor):
+    def __init__(self, tensor, before=None):
         self.tensor = tensor
         self.epochs = _Epochs()
-        self.lock = threading.Lock()
+        self.lock = threading.Lock() if before is None else before.lock
+        # memory whose header the last launch of the chain kernel wrote: `tensor`, a copy of the header in front of the
+        # first such launch on a larger workspace, None before any (new memory may hold a freed workspace's header)
+        self.record = None
+        if before is not None and before.record is not None:
+            self.record = before.record[:_lib.SSD_WORKSPACE_HEADER_INTS].clone()
 
 
 def _workspace_key(device, stream=None):
@@ -142,7 +149,9 @@ def _own_workspace(x, nbytes):
     with _WORKSPACES_LOCK:
         ent = _WORKSPACES.get(key)
         if ent is None or ent.tensor.numel() * 4 < nbytes:
-            ent = _Kept(torch.empty((max(nbytes, 1 << 16) + 3) // 4, device=x.device, dtype=torch.int32))
+            tensor = torch.empty((max(nbytes, 1 << 16) + 3) // 4, device=x.device, dtype=torch.int32)
+            with contextlib.nullcontext() if ent is None else ent.lock:
+                ent = _Kept(tensor, ent)
             _WORKSPACES[key] = ent
     return ent
 
@@ -166,6 +175,8 @@ def _launch_on_own_workspace(x, nbytes, launch, pairs):
         epoch = ent.epochs.next(pairs)
         rc, used = launch(ent.tensor, epoch)
         ent.epochs.done(epoch, rc, used, pairs)
+        if used and not rc:
+            ent.record = ent.tensor
         return rc
 
 
@@ -184,7 +195,10 @@ def fused_status(device=None, stream=None):
     if ent is None:
         return 0
     with ent.lock, torch.cuda.device(device):
-        return int(_lib.load().ssd_fused_workspace_status(ctypes.c_void_p(ent.tensor.data_ptr()),
+        if ent.record is None:
+            stream.synchronize()
+            return 0
+        return int(_lib.load().ssd_fused_workspace_status(ctypes.c_void_p(ent.record.data_ptr()),
                                                           ctypes.c_void_p(stream.cuda_stream)))
 
 

@@ -249,6 +249,18 @@ def test_kept_workspaces_can_be_released():
     assert not ops._WORKSPACES
 
 
+def test_a_larger_kept_workspace_takes_over_the_record():
+    # the last chain launch's record is asked for until the next one, and launches on one stream keep one lock
+    from ssd_amd import _lib, ops
+    small = ops._Kept(torch.arange(200, dtype=torch.int32))
+    assert small.record is None and ops._Kept(torch.zeros(400, dtype=torch.int32), small).record is None
+    small.record = small.tensor
+    large = ops._Kept(torch.zeros(400, dtype=torch.int32), small)
+    assert large.lock is small.lock and large.epochs.last == 0
+    assert torch.equal(large.record, torch.arange(_lib.SSD_WORKSPACE_HEADER_INTS, dtype=torch.int32))
+    assert large.record.data_ptr() != small.tensor.data_ptr()
+
+
 def test_epochs_of_a_kept_workspace():
     # what the wrappers pass as ssd_fused_opts.epoch for the workspace they keep per device and stream
     from ssd_amd.ops import _Epochs

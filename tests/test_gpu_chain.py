@@ -464,6 +464,30 @@ def test_chain_failures_reach_the_caller_of_the_plain_wrappers(ops, oracle):
         assert _mismatches(out, want_out)[0] == 0 and _mismatches(fin, want_fin)[0] == 0
 
 
+def test_the_record_of_a_failure_outlives_a_larger_workspace_and_not_a_released_one(ops, oracle):
+    """A call that another kernel family serves may need a larger workspace than the one with the record (here 2 heads x 4200
+    chunks of 2 tokens, fp32); and the memory of a released one may come back with the old header in it."""
+    d, many = oracle.make_inputs(1, b=1, L=8192, H=80), oracle.make_inputs(1, b=1, L=8400, H=2, P=64, N=16, Q=2, dtype="fp32")
+    of = lambda d: [_dev(d[k]) for k in ("B", "x", "dt", "dA_cumsum")]  # noqa: E731
+    d, many = of(d), of(many)
+    from ssd_amd.ops import _WORKSPACES
+    ops.release_workspaces()
+    ops._fused_chunk_state_state_passing_fwd(*d, torch.float32, _kernel=GLOBAL, _chunks_per_item=1, _spin_limit=1)
+    (small,) = _WORKSPACES.values()
+    for _ in range(2):
+        ops._fused_chunk_state_state_passing_fwd(*many, torch.float32)
+        (large,) = _WORKSPACES.values()
+        assert large.tensor.numel() > small.tensor.numel() and large.epochs.last == 0 and ops.fused_status() == -7
+    ops._fused_chunk_state_state_passing_fwd(*d, torch.float32)
+    assert list(_WORKSPACES.values()) == [large] and large.epochs.last == 1 and ops.fused_status() == 0
+    ops._fused_chunk_state_state_passing_fwd(*d, torch.float32, _kernel=GLOBAL, _chunks_per_item=1, _spin_limit=1)
+    assert ops.fused_status() == -7
+    del small, large
+    ops.release_workspaces()                                    # its memory is the next workspace's, as a rule
+    ops._fused_chunk_state_state_passing_fwd(*many, torch.float32)
+    assert ops.fused_status() == 0
+
+
 def test_chain_reports_xcds_that_are_not_what_it_assumed(ops, oracle):
     """LOCAL deals the units to one ticket counter per XCD and relies on a workgroup of every XCD showing up.  With the
     test hook the library is told a wrong number of XCDs: 4 makes pairs of XCDs share a counter (SSD_ERR_CHAIN_XCD), 16
