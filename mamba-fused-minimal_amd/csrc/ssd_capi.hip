@@ -281,8 +281,8 @@ double estimate_us(const ssd::cost::Problem &q, const Choice &c)
 
 // Whether the ticket / flag-chain kernel is the better fused kernel for a problem it covers: it keeps every compute
 // unit busy whatever the number of state tiles, at the price of its start, of reading each passed state back once per
-// item and of a link per item.
-bool chain_preferred(const Params &p, int n_cu)
+// item and of a link per item.  scan: the call is the one with the scan's state half.
+bool chain_preferred(const Params &p, int n_cu, bool scan = false)
 {
     const ssd::cost::Problem q = problem_of(p, n_cu);
     double chain = 0.;
@@ -293,7 +293,7 @@ bool chain_preferred(const Params &p, int n_cu)
     if (c.few) {
         // in front of this kernel too -- with packed sequences, which cut its chains, only where that never loses; elsewhere
         // it stays in front of the kernels that this one is not preferred to
-        if (!p.seq || ssd::cost::few_units_packed(q)) return false;
+        if (!p.seq || ssd::cost::few_units_packed(q, scan)) return false;
         c = choose(p, true, q.n_cu, false);
     }
     return chain < 1.05 * estimate_us(q, c);
@@ -676,7 +676,7 @@ int ssd_query_fused_wants_states(const ssd_tensor *x, const ssd_tensor *B, const
     // a contiguous fp32 (b,C,H,P,N) at a made-up, well-aligned address
     const int64_t plane = (int64_t)p.headdim * p.dstate;
     void *const somewhere = (void *)(uintptr_t)4096;
-    const ssd_tensor f32 = {somewhere, SSD_F32, 0, {p.C * p.nheads * plane, p.nheads * plane, plane, p.dstate, 1}};
+    const ssd_tensor f32 = {somewhere, SSD_F32, 0, {(int64_t)p.C * p.nheads * plane, p.nheads * plane, plane, p.dstate, 1}};
     Params as_out, as_states;
     rc = fill_fused(as_out, x, B, dt, dA_cumsum, seq_idx, initial_states, nullptr, &f32, final_states, dims, 1);
     if (rc == SSD_OK) rc = fill_fused(as_states, x, B, dt, dA_cumsum, seq_idx, initial_states, &f32, p.out ? out : &f32, final_states, dims, 1);
@@ -684,11 +684,11 @@ int ssd_query_fused_wants_states(const ssd_tensor *x, const ssd_tensor *B, const
     // what the call runs with a fp32 `out`, and whether it still does with the place it would be given
     const Choice c = choose(as_out, true, n_cu), given = p.out ? choose(as_states, true, n_cu) : c;
     if (c.family == F_PAIR) {
-        if (given.family != F_PAIR || (ssd::chain_supported(as_out) && chain_preferred(as_out, n_cu))) return 0;
+        if (given.family != F_PAIR || (ssd::chain_supported(as_out) && chain_preferred(as_out, n_cu, !p.out))) return 0;
         // Packed rows so long that a fp32 `out` runs the pair whatever the number of units: these calls have the chain
         // kernel instead, whose chains are cut (8 heads x 512 chunks, chain against pair, us: 8 sequences 259 / 196, 128
         // sequences 101 / 196; with the scan's state half 482 / 249 and 213 / 249).
-        if (p.seq && !ssd::cost::few_units_packed(problem_of(p, n_cu)) && ssd::chain_supported(p.out ? p : as_out) &&
+        if (p.seq && !ssd::cost::few_units_packed(problem_of(p, n_cu), !p.out) && ssd::chain_supported(p.out ? p : as_out) &&
             choose(as_out, true, n_cu, false).family == F_PAIR)
             return 0;
         return 1;

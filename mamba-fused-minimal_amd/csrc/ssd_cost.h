@@ -121,21 +121,34 @@ inline bool few_units(const Problem &q)
 }
 
 // The same against the chain kernel for packed sequences (seq_idx): its chains are then as long as a sequence, and how
-// long those are only the device knows, so the pair goes in front only where it does not lose with a sequence start in
-// every chunk.  The chain kernel's time is then that of its busiest compute unit's items, the pair's grows with the
-// chunks of a row and with all unit-chunks, so the two lines scale with the work of a unit-chunk.  At the lines, one start
-// / four starts a chunk, chain kernel against pair, us:
-//     dstate, chunk   heads x chunks   fp32 out                     bf16 out                     call with the scan's state half
-//     128, 256         4 x 64          35.2 / 25.4   33.7 / 25.6    36.3 / 30.7   34.5 / 30.8    46.9 / 33.8   42.4 / 33.9
-//                      8 x 57          37.7 / 30.9   34.0 / 30.8    38.7 / 34.1   34.3 / 34.0    49.4 / 42.5   43.6 / 41.9
-//                     20 x 23          36.3 / 25.4   34.3 / 25.4    36.9 / 26.0   34.7 / 26.0    46.4 / 36.2   44.0 / 35.8
-//     128, 128         8 x 41          26.4 / 22.5   24.6 / 22.5    27.2 / 25.4   25.5 / 25.4    34.0 / 32.4   30.4 / 32.5
-//     64, 128          8 x 33          21.0 / 15.1   19.6 / 15.1    21.6 / 17.8   19.8 / 17.8    26.4 / 23.5   24.1 / 23.6
-// and beyond them: 8 x 64 34.1 / 32.7 (four starts), bf16 34.4 / 37.3; 16 x 128 in 64 sequences 46.0 / 64.2; 4 x 512 in 4, 16
-// and 64 sequences 260 / 127, 121 / 127 and 69 / 126.
-inline bool few_units_packed(const Problem &q)
+// long those are only the device knows, so the pair goes in front only where it does not lose (3 % at most) with four starts in
+// every chunk.  The chain kernel's time is then about 35 us for a unit-chunk of work 1 while it runs items of four chunks
+// (22 - 24 with shorter items, below 17 chunks of work 1), the pair's grows by 0.14 us a chunk and 0.022 a unit-chunk.  At
+// the line, heads x chunks, five sequences / one start a chunk / four, chain kernel against pair, us:
+//     dstate, chunk                fp32 out                                   bf16 out
+//     128, 256      8 x 48         49.4 / 27.2   36.1 / 27.0   34.2 / 27.0    52.9 / 30.8   37.0 / 30.7   34.7 / 30.8
+//                  12 x 48         54.4 / 31.1   36.2 / 30.9   34.6 / 30.8    59.3 / 34.4   36.9 / 34.3   34.7 / 34.3
+//                  24 x 32         45.3 / 30.5   37.5 / 30.5   36.0 / 30.5    47.2 / 32.6   38.2 / 32.8   36.4 / 32.8
+//                  48 x 17         39.1 / 30.5   37.4 / 30.3   35.3 / 30.0    40.0 / 30.2   37.9 / 30.0   35.9 / 30.1
+//                  24 x 16         33.9 / 22.6   25.0 / 22.4   22.4 / 22.5    37.1 / 23.5   25.7 / 23.4   22.7 / 23.3
+//     128, 128     24 x 23         35.7 / 24.1   27.6 / 24.5   25.6 / 24.3    38.0 / 27.0   28.3 / 26.8   26.4 / 26.9
+//     64, 128      24 x 18         23.3 / 15.5   21.1 / 15.4   20.1 / 15.5    24.2 / 16.6   21.4 / 16.4   20.2 / 16.5
+// and beyond it: 8 x 64 64.4 / 32.1, 36.1 / 32.0, 34.1 / 31.9, bf16 72.0 / 37.0, 36.7 / 36.9, 34.4 / 37.0; 12 x 64 bf16 35.4 /
+// 40.1 with four starts; 48 x 16 32.5 / 28.9, 26.1 / 29.2, 23.6 / 29.1; 128, 128: 12 x 46 46.4 / 27.8, 27.6 / 27.8, 26.0 / 27.9;
+// 16 x 128 98.1 / 63.2, 41.9 / 62.1, 40.6 / 61.8; 4 x 512 in 4, 16 and 64 sequences 260 / 127, 121 / 127 and 69 / 126.
+//
+// scan: the call with the scan's state half, whose consumer is a launch of its own behind the pair and costs it 0.1 us a
+// unit-chunk, against the chain kernel's variant that computes that half (44 us with four starts a chunk).  At its line:
+// 24 x 20 55.6 / 35.5, 46.0 / 35.2, 44.0 / 35.1; 20 x 27 59.1 / 43.7, 45.6 / 43.6, 44.1 / 43.4; 12 x 40 74.0 / 38.6, 49.4 / 38.5, 43.9 /
+// 38.4; 8 x 57 86.9 / 41.8, 49.5 / 41.9, 43.7 / 41.3; 128, 128: 8 x 41 59.8 / 29.7, 34.1 / 29.7, 30.3 / 29.7; 64, 128: 16 x 19 30.9 /
+// 22.0, 25.4 / 22.0, 24.3 / 21.9; beyond it: 24 x 32 59.7 / 49.8, 49.1 / 49.7, 45.0 / 49.5.
+inline bool few_units_packed(const Problem &q, bool scan)
 {
-    return few_units(q) && q.units * 24 <= q.n_cu && q.chunks <= 64 * work(q) && (double)(q.units * q.chunks) <= 0.9 * work(q) * q.n_cu;
+    if (!few_units(q)) return false;
+    const double unit_chunks = (double)(q.units * q.chunks);
+    if (scan && q.chunks / 200.0 + unit_chunks / (1.25 * q.n_cu) > work(q)) return false;
+    if (chain_chunks_per_item(q, nullptr) < 4) return unit_chunks <= 0.75 * q.n_cu;
+    return q.chunks / 95.0 + unit_chunks / (2.3 * q.n_cu) <= work(q);
 }
 
 }  // namespace cost

@@ -102,9 +102,11 @@ def test_a_strided_initial_plane_keeps_the_kernel_it_had(ops, oracle):
     torch.testing.assert_close(yf.cpu(), want_fin, rtol=2e-3, atol=1e-3)
 
 
-@pytest.mark.parametrize("nseq,L,chain", [(7, 16384, True), (0, 16384, False), (7, 8192, False)])
-def test_packed_rows_run_the_chain_kernel_beyond_the_packed_line(ops, oracle, nseq, L, chain):
-    d = oracle.make_inputs(1, b=1, L=L, H=8, init=True, nseq=nseq)
+# chain: of the calls with fp32, bf16 and no passed states, which run the chain kernel
+@pytest.mark.parametrize("nseq,L,H,chain", [(7, 16384, 8, (1, 1, 1)), (0, 16384, 8, (0, 0, 0)), (7, 8192, 8, (0, 0, 0)),
+                                            (5, 4096, 24, (0, 0, 0)), (5, 8192, 24, (0, 0, 1)), (5, 4096, 48, (1, 1, 1)), (5, 4352, 48, (0, 0, 1))])
+def test_packed_rows_run_the_chain_kernel_beyond_the_packed_line(ops, oracle, nseq, L, H, chain):
+    d = oracle.make_inputs(1, b=1, L=L, H=H, init=True, nseq=nseq)
     mv = lambda t: None if t is None else t.cuda()  # noqa: E731
     args = [mv(d[k]) for k in ("B", "x", "dt", "dA_cumsum")]
     kw = dict(initial_states=mv(d["initial_states"]), seq_idx=mv(d["seq_idx"]))
@@ -112,11 +114,11 @@ def test_packed_rows_run_the_chain_kernel_beyond_the_packed_line(ops, oracle, ns
     from ssd_amd.ops import _WORKSPACES
     calls = [lambda o=o: ops._fused_chunk_state_state_passing_fwd(*args, o, **kw) for o in (torch.float32, torch.bfloat16)]
     calls.append(lambda: ops._fused_chunk_state_state_passing_scan_fwd(args[0], args[1], mv(d["C"]), *args[2:], return_states=False, **kw))
-    for call in calls:
+    for call, on_chain in zip(calls, chain):
         ops.release_workspaces()
         got = call()
         torch.cuda.synchronize()
-        assert max((k.epochs.last for k in _WORKSPACES.values()), default=0) == int(chain) and ops.fused_status() == 0
+        assert max((k.epochs.last for k in _WORKSPACES.values()), default=0) == on_chain and ops.fused_status() == 0
         torch.testing.assert_close(got[1].cpu(), want_fin, rtol=2e-3, atol=1e-3)
         if got[0] is not None:
             torch.testing.assert_close(got[0].float().cpu(), want_out, rtol=2e-3 if got[0].dtype == torch.float32 else 2.0 ** -7, atol=1e-3)

@@ -52,17 +52,22 @@ def test_arguments_the_call_rejects_are_left_to_it():
         _wants(dtype=torch.float64)
 
 
-@pytest.mark.parametrize("L,H,seq,want", [
-    (14592, 8, True, True), (14848, 8, True, False), (16384, 8, False, True),       # 57 and 58 chunks on four units
-    (16384, 4, True, True), (16640, 4, True, False), (16640, 4, False, True),       # 64 and 65 chunks
-    (7168, 16, True, True), (7424, 16, True, False), (7424, 16, False, True),       # 28 and 29 chunks on eight units
-    (4096, 24, True, False), (4096, 24, False, True),                               # twelve units
-    (2048, 48, True, True),                                                         # ... and no chain kernel to compare with
-    (131072, 8, True, False), (131072, 8, False, True),                             # long enough for the pair at any number of units
+@pytest.mark.parametrize("L,H,seq,want,scan", [
+    (14592, 8, True, True, True), (14848, 8, True, False, False), (16384, 8, False, True, True),     # 57 and 58 chunks on four units
+    (18176, 4, True, True, True),                                                                    # 71 and 72 chunks on two units
+    (18432, 4, True, False, False), (18432, 4, False, True, True),
+    (8448, 16, True, True, True), (8704, 16, True, True, False), (10496, 16, True, True, False),     # 33, 34, 41 and 42 chunks on eight units
+    (10752, 16, True, False, False), (10752, 16, False, True, True),
+    (5888, 24, True, True, True), (6144, 24, True, True, False), (8192, 24, True, True, False),      # twelve units: 23, 24, 32 and 33 chunks
+    (8448, 24, True, False, False),
+    (4096, 24, False, True, True),
+    (2048, 48, True, True, True),                                                   # ... and no chain kernel to compare with
+    (4096, 48, True, False, False), (4352, 48, True, True, False),                  # 16 chunks in items of two, 17 in items of four
+    (131072, 8, True, False, False), (131072, 8, False, True, True),                # long enough for the pair at any number of units
 ])
-def test_packed_sequences_keep_the_chain_kernel_where_its_chains_are_cut(L, H, seq, want):
+def test_packed_sequences_keep_the_chain_kernel_where_its_chains_are_cut(L, H, seq, want, scan):
     seq = torch.zeros(1, L, dtype=torch.int32) if seq else None
-    assert _wants(L=L, H=H, seq=seq) == want and _wants(L=L, H=H, seq=seq, out=None) == want
+    assert _wants(L=L, H=H, seq=seq) == want and _wants(L=L, H=H, seq=seq, out=None) == scan
     if seq is not None:                                                             # fp16 `out`: not the chain kernel's
         assert _wants(L=L, H=H, seq=seq, out=torch.float16) == (want or L == 131072)
 
