@@ -279,10 +279,18 @@ double estimate_us(const ssd::cost::Problem &q, const Choice &c)
     }
 }
 
+// What a fused call returns, as the line for packed sequences asks: without passed states it is the call with the scan's
+// state half.
+ssd::cost::PackedForm packed_form(const Params &p)
+{
+    if (!p.out) return ssd::cost::PACKED_SCAN;
+    return p.dt_out == ssd::DT_F32 ? ssd::cost::PACKED_OUT_F32 : ssd::cost::PACKED_OUT_16BIT;
+}
+
 // Whether the ticket / flag-chain kernel is the better fused kernel for a problem it covers: it keeps every compute
 // unit busy whatever the number of state tiles, at the price of its start, of reading each passed state back once per
-// item and of a link per item.  scan: the call is the one with the scan's state half.
-bool chain_preferred(const Params &p, int n_cu, bool scan = false)
+// item and of a link per item.  form: what the call returns, for rows of packed sequences.
+bool chain_preferred(const Params &p, int n_cu, ssd::cost::PackedForm form)
 {
     const ssd::cost::Problem q = problem_of(p, n_cu);
     double chain = 0.;
@@ -293,7 +301,7 @@ bool chain_preferred(const Params &p, int n_cu, bool scan = false)
     if (c.few) {
         // in front of this kernel too -- with packed sequences, which cut its chains, only where that never loses; elsewhere
         // it stays in front of the kernels that this one is not preferred to
-        if (!p.seq || ssd::cost::few_units_packed(q, scan)) return false;
+        if (!p.seq || ssd::cost::few_units_packed(q, form)) return false;
         c = choose(p, true, q.n_cu, false);
     }
     return chain < 1.05 * estimate_us(q, c);
@@ -318,7 +326,7 @@ int chain_decision(const Params &p, const ssd_dims *dims, const ssd_fused_opts *
                          opts->workspace_bytes >= need && !(out16 && r < 2);
     // with the scan's state half asked for, the chain kernel is the only one that computes it in the same launch
     if (have_ws && ssd::chain_supported(p) &&
-        (kernel != SSD_KERNEL_AUTO || p.y || (g_forced_split.load(std::memory_order_relaxed) == 0 && chain_preferred(p, compute_units())))) {
+        (kernel != SSD_KERNEL_AUTO || p.y || (g_forced_split.load(std::memory_order_relaxed) == 0 && chain_preferred(p, compute_units(), packed_form(p))))) {
         *use = true;
         if (opts->used_workspace) *opts->used_workspace = 1;
         return check_device();
@@ -684,11 +692,11 @@ int ssd_query_fused_wants_states(const ssd_tensor *x, const ssd_tensor *B, const
     // what the call runs with a fp32 `out`, and whether it still does with the place it would be given
     const Choice c = choose(as_out, true, n_cu), given = p.out ? choose(as_states, true, n_cu) : c;
     if (c.family == F_PAIR) {
-        if (given.family != F_PAIR || (ssd::chain_supported(as_out) && chain_preferred(as_out, n_cu, !p.out))) return 0;
+        if (given.family != F_PAIR || (ssd::chain_supported(as_out) && chain_preferred(as_out, n_cu, packed_form(p)))) return 0;
         // Packed rows so long that a fp32 `out` runs the pair whatever the number of units: these calls have the chain
         // kernel instead, whose chains are cut (8 heads x 512 chunks, chain against pair, us: 8 sequences 259 / 196, 128
         // sequences 101 / 196; with the scan's state half 482 / 249 and 213 / 249).
-        if (p.seq && !ssd::cost::few_units_packed(problem_of(p, n_cu), !p.out) && ssd::chain_supported(p.out ? p : as_out) &&
+        if (p.seq && !ssd::cost::few_units_packed(problem_of(p, n_cu), packed_form(p)) && ssd::chain_supported(p.out ? p : as_out) &&
             choose(as_out, true, n_cu, false).family == F_PAIR)
             return 0;
         return 1;

@@ -121,34 +121,37 @@ inline bool few_units(const Problem &q)
 }
 
 // The same against the chain kernel for packed sequences (seq_idx): its chains are then as long as a sequence, and how
-// long those are only the device knows, so the pair goes in front only where it does not lose (3 % at most) with four starts in
-// every chunk.  The chain kernel's time is then about 35 us for a unit-chunk of work 1 while it runs items of four chunks
-// (22 - 24 with shorter items, below 17 chunks of work 1), the pair's grows by 0.14 us a chunk and 0.022 a unit-chunk.  At
-// the line, heads x chunks, five sequences / one start a chunk / four, chain kernel against pair, us:
-//     dstate, chunk                fp32 out                                   bf16 out
-//     128, 256      8 x 48         49.4 / 27.2   36.1 / 27.0   34.2 / 27.0    52.9 / 30.8   37.0 / 30.7   34.7 / 30.8
-//                  12 x 48         54.4 / 31.1   36.2 / 30.9   34.6 / 30.8    59.3 / 34.4   36.9 / 34.3   34.7 / 34.3
-//                  24 x 32         45.3 / 30.5   37.5 / 30.5   36.0 / 30.5    47.2 / 32.6   38.2 / 32.8   36.4 / 32.8
-//                  48 x 17         39.1 / 30.5   37.4 / 30.3   35.3 / 30.0    40.0 / 30.2   37.9 / 30.0   35.9 / 30.1
-//                  24 x 16         33.9 / 22.6   25.0 / 22.4   22.4 / 22.5    37.1 / 23.5   25.7 / 23.4   22.7 / 23.3
-//     128, 128     24 x 23         35.7 / 24.1   27.6 / 24.5   25.6 / 24.3    38.0 / 27.0   28.3 / 26.8   26.4 / 26.9
-//     64, 128      24 x 18         23.3 / 15.5   21.1 / 15.4   20.1 / 15.5    24.2 / 16.6   21.4 / 16.4   20.2 / 16.5
-// and beyond it: 8 x 64 64.4 / 32.1, 36.1 / 32.0, 34.1 / 31.9, bf16 72.0 / 37.0, 36.7 / 36.9, 34.4 / 37.0; 12 x 64 bf16 35.4 /
-// 40.1 with four starts; 48 x 16 32.5 / 28.9, 26.1 / 29.2, 23.6 / 29.1; 128, 128: 12 x 46 46.4 / 27.8, 27.6 / 27.8, 26.0 / 27.9;
-// 16 x 128 98.1 / 63.2, 41.9 / 62.1, 40.6 / 61.8; 4 x 512 in 4, 16 and 64 sequences 260 / 127, 121 / 127 and 69 / 126.
-//
-// scan: the call with the scan's state half, whose consumer is a launch of its own behind the pair and costs it 0.1 us a
-// unit-chunk, against the chain kernel's variant that computes that half (44 us with four starts a chunk).  At its line:
-// 24 x 20 55.6 / 35.5, 46.0 / 35.2, 44.0 / 35.1; 20 x 27 59.1 / 43.7, 45.6 / 43.6, 44.1 / 43.4; 12 x 40 74.0 / 38.6, 49.4 / 38.5, 43.9 /
-// 38.4; 8 x 57 86.9 / 41.8, 49.5 / 41.9, 43.7 / 41.3; 128, 128: 8 x 41 59.8 / 29.7, 34.1 / 29.7, 30.3 / 29.7; 64, 128: 16 x 19 30.9 /
-// 22.0, 25.4 / 22.0, 24.3 / 21.9; beyond it: 24 x 32 59.7 / 49.8, 49.1 / 49.7, 45.0 / 49.5.
-inline bool few_units_packed(const Problem &q, bool scan)
+// long those are only the device knows.  The pair goes in front where it loses next to nothing (a twentieth at most) with a
+// sequence start in every second chunk; it is then ahead by up to threefold with a few long sequences a row and loses up to
+// a fifth with a start in every chunk.  The chain kernel's time hardly depends on the size there (38 - 42 us for a
+// unit-chunk of work 1; beyond 512 unit-chunks 80 us and more with the scan's state half, which runs items of two chunks),
+// the pair's grows with the chunks of a row and with all unit-chunks.  Around the lines, two sequences a row / a start in
+// every fourth chunk / second / every one, chain kernel against pair, us:
+//     dstate, chunk   heads x chunks
+//     128, 256, fp32 out      4 x 89        94.5 / 33.7   47.6 / 33.7   39.6 / 33.7   35.9 / 33.8
+//                             8 x 110      109.5 / 43.8   46.2 / 43.4   41.3 / 43.6   37.7 / 43.3      (beyond)
+//                            16 x 50        73.1 / 34.0   46.6 / 34.0   39.8 / 33.4   38.0 / 33.3
+//                            16 x 69        87.5 / 41.2   44.7 / 41.1   40.3 / 41.2   37.8 / 41.1
+//                            32 x 47        63.9 / 42.8   46.1 / 43.2   42.2 / 43.1   38.6 / 43.2
+//                             4 x 512 in 4, 16 and 64 sequences: 260 / 127, 121 / 127, 69 / 126               (beyond)
+//     128, 256, bf16 out      4 x 89       106.6 / 41.0   50.7 / 41.1   41.1 / 41.1   36.7 / 41.1
+//                            12 x 63        84.7 / 39.3   48.3 / 39.3   41.3 / 39.2   38.4 / 39.2
+//                            20 x 64        81.6 / 45.5   51.3 / 46.9   45.2 / 45.6   39.0 / 45.7      (beyond)
+//                            40 x 38        66.0 / 46.4   49.6 / 44.0   43.5 / 44.1   40.8 / 43.4
+//     128, 256, scan          4 x 89       135.0 / 43.6   62.5 / 43.4   52.4 / 43.5   47.0 / 43.4
+//                            12 x 63       103.5 / 54.7   60.6 / 54.7   51.8 / 54.5   47.6 / 54.2      (beyond)
+//                            24 x 35        77.1 / 53.8   60.9 / 53.6   55.6 / 53.2   47.1 / 53.2
+//                            48 x 18        63.2 / 52.0   54.8 / 52.1   51.4 / 52.2   46.1 / 51.8
+//     128, 128, fp32 out      8 x 59        69.0 / 28.8   36.2 / 28.7   31.3 / 28.3   27.4 / 28.7
+//     64, 128, fp32 out      24 x 35        36.5 / 23.7   26.2 / 23.5   24.1 / 23.5   22.9 / 23.8
+enum PackedForm { PACKED_OUT_F32, PACKED_OUT_16BIT, PACKED_SCAN };      // scan: no passed states, the scan's state half instead
+inline bool few_units_packed(const Problem &q, PackedForm form)
 {
     if (!few_units(q)) return false;
-    const double unit_chunks = (double)(q.units * q.chunks);
-    if (scan && q.chunks / 200.0 + unit_chunks / (1.25 * q.n_cu) > work(q)) return false;
-    if (chain_chunks_per_item(q, nullptr) < 4) return unit_chunks <= 0.75 * q.n_cu;
-    return q.chunks / 95.0 + unit_chunks / (2.3 * q.n_cu) <= work(q);
+    const double chunks = q.chunks, per_cu = (double)(q.units * q.chunks) / q.n_cu;
+    if (form == PACKED_OUT_16BIT) return chunks / 100.0 + per_cu / 6.0 <= work(q);
+    if (form == PACKED_SCAN && chunks / 260.0 + per_cu / 1.8 > work(q)) return false;       // and the fused part's own
+    return chunks / 160.0 + per_cu / 4.6 <= work(q);
 }
 
 }  // namespace cost

@@ -103,8 +103,8 @@ def test_a_strided_initial_plane_keeps_the_kernel_it_had(ops, oracle):
 
 
 # chain: of the calls with fp32, bf16 and no passed states, which run the chain kernel
-@pytest.mark.parametrize("nseq,L,H,chain", [(7, 16384, 8, (1, 1, 1)), (0, 16384, 8, (0, 0, 0)), (7, 8192, 8, (0, 0, 0)),
-                                            (5, 4096, 24, (0, 0, 0)), (5, 8192, 24, (0, 0, 1)), (5, 4096, 48, (1, 1, 1)), (5, 4352, 48, (0, 0, 1))])
+@pytest.mark.parametrize("nseq,L,H,chain", [(7, 26624, 8, (1, 1, 1)), (0, 26624, 8, (0, 0, 0)), (7, 16384, 8, (0, 0, 0)), (5, 9216, 24, (0, 0, 1)),
+                                            (5, 24576, 4, (0, 1, 0)), (5, 7936, 48, (0, 0, 1)), (5, 4352, 48, (0, 0, 0))])
 def test_packed_rows_run_the_chain_kernel_beyond_the_packed_line(ops, oracle, nseq, L, H, chain):
     d = oracle.make_inputs(1, b=1, L=L, H=H, init=True, nseq=nseq)
     mv = lambda t: None if t is None else t.cuda()  # noqa: E731

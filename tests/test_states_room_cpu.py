@@ -52,24 +52,21 @@ def test_arguments_the_call_rejects_are_left_to_it():
         _wants(dtype=torch.float64)
 
 
-@pytest.mark.parametrize("L,H,seq,want,scan", [
-    (14592, 8, True, True, True), (14848, 8, True, False, False), (16384, 8, False, True, True),     # 57 and 58 chunks on four units
-    (18176, 4, True, True, True),                                                                    # 71 and 72 chunks on two units
-    (18432, 4, True, False, False), (18432, 4, False, True, True),
-    (8448, 16, True, True, True), (8704, 16, True, True, False), (10496, 16, True, True, False),     # 33, 34, 41 and 42 chunks on eight units
-    (10752, 16, True, False, False), (10752, 16, False, True, True),
-    (5888, 24, True, True, True), (6144, 24, True, True, False), (8192, 24, True, True, False),      # twelve units: 23, 24, 32 and 33 chunks
-    (8448, 24, True, False, False),
-    (4096, 24, False, True, True),
-    (2048, 48, True, True, True),                                                   # ... and no chain kernel to compare with
-    (4096, 48, True, False, False), (4352, 48, True, True, False),                  # 16 chunks in items of two, 17 in items of four
-    (131072, 8, True, False, False), (131072, 8, False, True, True),                # long enough for the pair at any number of units
+@pytest.mark.parametrize("chunks,H,seq,want,scan", [
+    (88, 4, True, True, True), (89, 4, True, False, True), (122, 4, True, False, True), (123, 4, True, False, False), (123, 4, False, True, True),
+    (79, 8, True, True, True), (80, 8, True, False, False), (80, 8, False, True, True),
+    (47, 16, True, True, True), (48, 16, True, True, False), (65, 16, True, True, False), (66, 16, True, False, False), (66, 16, False, True, True),
+    (33, 24, True, True, True), (34, 24, True, True, False), (56, 24, True, True, False), (57, 24, True, False, False), (57, 24, False, True, True),
+    (17, 48, True, True, True), (18, 48, True, True, False), (31, 48, True, True, False), (32, 48, False, False, False),     # few no more
+    (512, 8, True, False, False), (512, 8, False, True, True),                      # long enough for the pair at any number of units
 ])
-def test_packed_sequences_keep_the_chain_kernel_where_its_chains_are_cut(L, H, seq, want, scan):
+def test_packed_sequences_keep_the_chain_kernel_where_its_chains_are_cut(chunks, H, seq, want, scan):
+    # chunks of 256 tokens, dstate 128; want: bf16 `out`, scan: the call without passed states
+    L = chunks * 256
     seq = torch.zeros(1, L, dtype=torch.int32) if seq else None
     assert _wants(L=L, H=H, seq=seq) == want and _wants(L=L, H=H, seq=seq, out=None) == scan
     if seq is not None:                                                             # fp16 `out`: not the chain kernel's
-        assert _wants(L=L, H=H, seq=seq, out=torch.float16) == (want or L == 131072)
+        assert _wants(L=L, H=H, seq=seq, out=torch.float16) == (want or chunks == 512)
 
 
 def test_room_is_bounded_and_a_call_does_without_it(monkeypatch):
