@@ -179,7 +179,8 @@ typedef struct ssd_fused_opts {
                                  workspace and its epoch --, to 0 if another kernel family served it */
 } ssd_fused_opts;
 
-enum { SSD_KERNEL_AUTO = 0, SSD_KERNEL_CHAIN = 1, SSD_KERNEL_CHAIN_LOCAL = 2, SSD_KERNEL_CHAIN_GLOBAL = 3 };
+enum { SSD_KERNEL_AUTO = 0, SSD_KERNEL_CHAIN = 1, SSD_KERNEL_CHAIN_LOCAL = 2, SSD_KERNEL_CHAIN_GLOBAL = 3,
+       SSD_KERNEL_ROWS = 4 };
 
 uint64_t ssd_fused_workspace_bytes(const ssd_dims *dims);
 /*
@@ -251,8 +252,8 @@ int ssd_fused_static_status(void *stream);
 int ssd_query_path(const ssd_tensor *x, const ssd_tensor *B, const ssd_dims *dims);
 
 /*
- * Which kernel family a fused call on plain tensors of these sizes would run, and why: the library ranks its fused
- * kernels by an estimate of their duration (a fit to measured times, per compute unit) and this call returns the
+ * Which kernel family a fused call on plain tensors of these sizes would run where the row kernel does not take it
+ * (ssd_query_fused_rows), and why: the library ranks its other fused kernels by an estimate of their duration (a fit to measured times, per compute unit) and this call returns the
  * ranking.  Assumed: bf16 x / B, fp32 dt / dA_cumsum / out / final_states, contiguous, no `states` output -- the
  * arguments every family covers.  has_workspace != 0 asks about ssd_fused_chunk_state_passing_fwd_ws with a
  * workspace of ssd_fused_workspace_bytes(dims) and SSD_KERNEL_AUTO, 0 about ssd_fused_chunk_state_passing_fwd; no seq_idx.
@@ -265,12 +266,22 @@ enum { SSD_FAMILY_GENERIC = 0, SSD_FAMILY_TOKEN_SPLIT = 1, SSD_FAMILY_FOUR_TILE 
        SSD_FAMILY_CHAIN = 4, SSD_FAMILY_COUNT = 5 };
 
 typedef struct ssd_fused_plan {
-    int32_t family;                         /* SSD_FAMILY_* the call would run */
+    int32_t family;                         /* SSD_FAMILY_* the call would run (behind ssd_query_fused_rows) */
     int32_t chunks_per_item;                /* of the chain kernel when that is the family, else 0 */
     float estimate_us[SSD_FAMILY_COUNT];    /* the model's estimate per family (chain: at its best chunks per item) */
 } ssd_fused_plan;
 
 int ssd_query_fused_plan(const ssd_dims *dims, int has_workspace, int compute_units, ssd_fused_plan *plan);
+
+/*
+ * The same question about the row kernel, which goes in front of those families where it is estimated to be faster:
+ * workgroups of 1 .. 5 slices of 16 state rows, at most one per compute unit, each walking its whole sequence.  Returns the
+ * slices per workgroup, 0 where the call runs what ssd_query_fused_plan says, or a negative status.  It takes bf16 x / B with
+ * headdim % 16 == 0, dstate 64 or 128, chunk_size % 128 == 0, any number of heads; x rows whose heads lie within the token
+ * pitch; fp32 or 16-bit out.  ssd_fused_chunk_state_passing_fwd_ws insists on it with opts->kernel = SSD_KERNEL_ROWS and
+ * opts->chunks_per_item = the slices (SSD_ERR_SHAPE where it does not apply; the other calls refuse that value).
+ */
+int ssd_query_fused_rows(const ssd_dims *dims, int has_workspace, int compute_units);
 
 /*
  * Whether ssd_fused_chunk_state_passing_fwd_ws (with a workspace and SSD_KERNEL_AUTO) on these very arguments is estimated

@@ -219,6 +219,8 @@ hipError_t launch_pair(const Params &p, hipStream_t s, bool generic = false)
     return e == hipSuccess ? ssd::launch_state_passing(pass_params_of(p), s) : e;
 }
 
+int rows_preferred(const Params &p, int n_cu, bool workspace);
+
 int run(const Params &p_in, bool fused, void *stream)
 {
     int rc = check_device();
@@ -226,6 +228,8 @@ int run(const Params &p_in, bool fused, void *stream)
     Params p = p_in;
     p.n_cu = compute_units();
     hipStream_t s = (hipStream_t)stream;
+    if (fused)
+        if (const int kr = rows_preferred(p, p.n_cu > 0 ? p.n_cu : 256, false)) return (int)ssd::launch_rows(p, kr, s);
     const Choice c = choose(p, fused, p.n_cu > 0 ? p.n_cu : 256);
     hipError_t e;
     switch (c.family) {
@@ -307,6 +311,31 @@ bool chain_preferred(const Params &p, int n_cu, ssd::cost::PackedForm form)
     return chain < 1.05 * estimate_us(q, c);
 }
 
+// Slices per workgroup of the row kernel where a fused call runs on it, else 0.  workspace: the chain kernel is a candidate.
+// Where few units go to chunk states + recurrence the call does so in front of this kernel too (2 x 2048 x 24 heads: 22 us
+// against 21, 1 x 1536 x 24: 15 against 13).
+int rows_preferred(const Params &p, int n_cu, bool workspace)
+{
+    if (g_forced_split.load(std::memory_order_relaxed) != 0 || !ssd::rows_supported(p)) return 0;
+    const ssd::cost::Problem q = problem_of(p, n_cu);
+    double us = 0.;
+    const int64_t slices = (int64_t)(p.nheads / p.ngroups) * (p.headdim / 16), groups = (int64_t)p.batch * p.ngroups;
+    const int kr = ssd::cost::rows_slices(q, slices, groups, ssd::kMaxRowSlices, &us);
+    if (!kr) return 0;
+    Choice c = choose(p, true, q.n_cu);
+    if (c.few) {
+        if (!p.seq || ssd::cost::few_units_packed(q, packed_form(p))) return 0;
+        c = choose(p, true, q.n_cu, false);
+    }
+    if (us >= estimate_us(q, c)) return 0;
+    if (workspace && ssd::chain_supported(p)) {
+        double chain = 0.;
+        ssd::cost::chain_chunks_per_item(q, &chain);
+        if (us >= chain) return 0;
+    }
+    return kr;
+}
+
 // Whether a fused call runs on the ticket / flag-chain kernel: a usable workspace came with it and that kernel is
 // asked for or estimated to be the faster one.  Returns a status (a kernel forced where it cannot run).
 int chain_decision(const Params &p, const ssd_dims *dims, const ssd_fused_opts *opts, bool *use)
@@ -326,12 +355,25 @@ int chain_decision(const Params &p, const ssd_dims *dims, const ssd_fused_opts *
                          opts->workspace_bytes >= need && !(out16 && r < 2);
     // with the scan's state half asked for, the chain kernel is the only one that computes it in the same launch
     if (have_ws && ssd::chain_supported(p) &&
-        (kernel != SSD_KERNEL_AUTO || p.y || (g_forced_split.load(std::memory_order_relaxed) == 0 && chain_preferred(p, compute_units(), packed_form(p))))) {
+        (kernel != SSD_KERNEL_AUTO || p.y || (g_forced_split.load(std::memory_order_relaxed) == 0 && !rows_preferred(p, compute_units() > 0 ? compute_units() : 256, true) &&
+          chain_preferred(p, compute_units(), packed_form(p))))) {
         *use = true;
         if (opts->used_workspace) *opts->used_workspace = 1;
         return check_device();
     }
     return kernel != SSD_KERNEL_AUTO ? SSD_ERR_SCRATCH : SSD_OK;     // forced, but no workspace or not a shape it covers
+}
+
+// The row kernel where it is insisted on: chunks_per_item slices per workgroup (a test and tuning hook).
+int run_rows_forced(const Params &p_in, const ssd_fused_opts *opts, void *stream)
+{
+    if (opts->used_workspace) *opts->used_workspace = 0;
+    if (!ssd::rows_supported(p_in) || opts->chunks_per_item < 1 || opts->chunks_per_item > ssd::kMaxRowSlices) return SSD_ERR_SHAPE;
+    const int rc = check_device();
+    if (rc) return rc;
+    Params p = p_in;
+    p.n_cu = compute_units();
+    return (int)ssd::launch_rows(p, opts->chunks_per_item, (hipStream_t)stream);
 }
 
 int run_chain(Params &p, const ssd_fused_opts *opts, void *stream)
@@ -479,6 +521,7 @@ int ssd_fused_chunk_state_passing_fwd_ws(const ssd_tensor *x, const ssd_tensor *
     Params p;
     int rc = fill_fused(p, x, B, dt, dA_cumsum, seq_idx, initial_states, states, out, final_states, dims, clamp);
     if (rc) return rc;
+    if (opts && opts->kernel == SSD_KERNEL_ROWS) return run_rows_forced(p, opts, stream);
     bool chain = false;
     rc = chain_decision(p, dims, opts, &chain);
     if (rc) return rc;
@@ -633,13 +676,12 @@ int ssd_query_path(const ssd_tensor *x, const ssd_tensor *B, const ssd_dims *dim
     return ssd::mfma_supported(p) ? 1 : 0;
 }
 
-int ssd_query_fused_plan(const ssd_dims *dims, int has_workspace, int compute_units, ssd_fused_plan *plan)
+// A fused call on plain tensors of these sizes at a made-up, well-aligned address: only sizes, strides and types are looked at.
+static int plain_fused(Params &p, const ssd_dims *dims, int compute_units)
 {
-    if (!plan) return SSD_ERR_NULL;
     int rc = check_dims(dims);
     if (rc) return rc;
     if (compute_units < 0) return SSD_ERR_SHAPE;
-    // plain tensors of these sizes at a made-up, well-aligned address: only sizes, strides and types are looked at
     const int64_t L = dims->seqlen, H = dims->nheads, P = dims->headdim, N = dims->dstate,
                   G = dims->ngroups, Q = dims->chunk_size, C = dims->nchunks;
     void *const somewhere = (void *)(uintptr_t)4096;
@@ -648,11 +690,22 @@ int ssd_query_fused_plan(const ssd_dims *dims, int has_workspace, int compute_un
     const ssd_tensor dt = {somewhere, SSD_F32, 0, {H * C * Q, C * Q, Q, 1, 0}};
     const ssd_tensor out = {somewhere, SSD_F32, 0, {C * H * P * N, H * P * N, P * N, N, 1}};
     const ssd_tensor fin = {somewhere, SSD_F32, 0, {H * P * N, P * N, N, 1, 0}};
-    Params p;
     rc = fill_fused(p, &x, &B, &dt, &dt, nullptr, nullptr, nullptr, &out, &fin, dims, 1);
     if (rc) return rc;
-    const int n_cu = compute_units > 0 ? compute_units : 256;
-    p.n_cu = n_cu;
+    p.n_cu = compute_units > 0 ? compute_units : 256;
+    return SSD_OK;
+}
+
+int ssd_query_fused_plan(const ssd_dims *dims, int has_workspace, int compute_units, ssd_fused_plan *plan)
+{
+    if (!plan) return SSD_ERR_NULL;
+    int rc = check_dims(dims);
+    if (rc) return rc;
+    if (compute_units < 0) return SSD_ERR_SHAPE;
+    Params p;
+    rc = plain_fused(p, dims, compute_units);
+    if (rc) return rc;
+    const int n_cu = p.n_cu;
     memset(plan, 0, sizeof(*plan));
     const ssd::cost::Problem q = problem_of(p, n_cu);
     const Choice c = choose(p, true, n_cu);
@@ -670,6 +723,14 @@ int ssd_query_fused_plan(const ssd_dims *dims, int has_workspace, int compute_un
         }
     }
     return SSD_OK;
+}
+
+int ssd_query_fused_rows(const ssd_dims *dims, int has_workspace, int compute_units)
+{
+    Params p;
+    const int rc = plain_fused(p, dims, compute_units);
+    if (rc) return rc;
+    return rows_preferred(p, p.n_cu, has_workspace != 0);
 }
 
 int ssd_query_fused_wants_states(const ssd_tensor *x, const ssd_tensor *B, const ssd_tensor *dt, const ssd_tensor *dA_cumsum,

@@ -98,6 +98,41 @@ inline double pair_us(const Problem &q)
     return 6.0 + (x_bytes + 3.0 * s_bytes) / 5.0e6 * (256.0 / q.n_cu);
 }
 
+// Row kernel (ssd_rows.hip): workgroups of kr slices of 16 state rows, one per compute unit, each walking its whole sequence.
+// Per chunk and relative to dstate 128, chunk 256 (measured 0.61 at chunk 128, 0.75 at dstate 64, 0.45 at both):
+inline double rows_us(const Problem &q, int kr)
+{
+    static const double t_chunk[6] = {0., 1.5, 1.85, 3.0, 3.75, 5.2};
+    const double k = q.chunk_size / 256.0, n = q.dstate / 128.0;
+    return 5.5 + q.chunks * t_chunk[kr] * (0.08 + 0.42 * k + 0.14 * n + 0.36 * k * n);
+}
+
+// Slices per workgroup of the row kernel, 0 where it is no candidate.  slices: 16-row slices of a (batch, group); groups:
+// (batch, group) pairs.  There is a workgroup per compute unit at most: a second round of workgroups costs as much as the
+// first (8 x 2048 x 48 heads: 66 us, the others 57).  A workgroup reads the same few columns of x to the end, so long rows
+// depend on how those columns fall on the memory channels, and a third of the workgroups finish up to a fifth late: up to 5120
+// tokens the kernel is ahead wherever its estimate is, beyond that only with four slices at dstate 128 or with chunks of
+// 128.  Inputs from memory, the faster of the others against this kernel, us (slices):
+//     8 x 2048 x 24 heads       48.4 /  35.9 (3)      4 x 8192 x 64                   143.5 / 132.7 (4)
+//     2 x 2048 x 80             49.0 /  34.9 (3)      4 x 8192 x 80                   175.7 / 177.1 (5)   (not taken)
+//     1 x 4096 x 80             53.9 /  46.3 (2)      1 x 8192 x 80                    70.9 /  85.9 (2)   (not taken)
+//     4 x 4096 x 48             67.4 /  60.0 (4)      8 x 8192 x 24                   117.2 / 123.6 (3)   (not taken)
+//     4 x 2048 x 80             56.3 /  48.5 (5)      4 x 8192 x 80, chunk 128        249.2 / 228.5 (5)
+//     8 x 2048 x 24, chunk 128  64.9 /  42.7 (3)      4 x 8192 x 80, dstate 64        130.2 / 137.0 (5)   (not taken)
+//     8 x 2048 x 24, dstate 64  34.7 /  28.9 (3)      8 x 3729 x 24, 8 groups, dstate 64, chunk 128   75.7 / 54.7 (3)
+inline int rows_slices(const Problem &q, int64_t slices, int64_t groups, int most, double *us)
+{
+    int best = 0;
+    const bool long_rows = (int64_t)q.chunks * q.chunk_size > 5120;
+    for (int kr = 1; kr <= most; ++kr) {
+        if (groups * ceil_div(slices, kr) > q.n_cu) continue;
+        if (long_rows && !(kr >= 4 && (q.chunk_size == 128 || (kr == 4 && q.dstate == 128)))) continue;
+        const double t = rows_us(q, kr);
+        if (!best || t < *us) { best = kr; *us = t; }
+    }
+    return best;
+}
+
 // Few units: the pair, whatever the estimates say (they are fits to 24 and more heads and know the recurrence as a pure
 // bandwidth).  The other families then leave most of the chip idle -- a unit's chunks are one serial chain in each of
 // them -- where the chunk-state launch spreads over (tile, chunk) and the recurrence costs about 0.2 us a chunk.  dstate

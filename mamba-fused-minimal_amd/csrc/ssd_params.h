@@ -171,6 +171,10 @@ hipError_t launch_quad_chunk_state(const Params &p, hipStream_t s);     // chunk
 bool quad_chunk_state_supported(const Params &p);
 bool quad_inputs_supported(const Params &p);     // what the four-tile kernel asks of x, B, dt, dA_cumsum and the shape
 int set_quad_segment_chunks(int n);     // 0 = automatic; chunks per workgroup of the above; returns the old value
+// fused, workgroups of 1 .. kMaxRowSlices slices of 16 state rows
+constexpr int kMaxRowSlices = 5;
+bool rows_supported(const Params &p);
+hipError_t launch_rows(const Params &p, int slices, hipStream_t s);
 // fused, work items drawn by ticket and chained by flags: every compute unit busy whatever the number of tiles
 hipError_t launch_chain(const Params &p, int n_cu, int mode, hipStream_t s);
 bool chain_supported(const Params &p);

@@ -287,8 +287,9 @@ def _fused_chunk_state_state_passing_fwd(B, x, dt, dA_cumsum, out_dtype, initial
     kernels/fused_concurrent.py:296-298); so does this one: a small int32 workspace for the ticket counter and the
     flags of the kernel that spreads a sequence's chunks over all compute units (plus, with bf16 ``out_dtype``, the
     fp32 copies of the states that cross between that kernel's work items).  ``_kernel`` (0 = let the library
-    choose, 1 = insist on that kernel, 2 / 3 = and on its per-XCD / device-wide variant), ``_chunks_per_item``
-    (1, 2 or 4 consecutive chunks per work item of that kernel, 0 = choose), ``_spin_limit`` (polls before a flag wait gives up, 0 = default) and
+    choose, 1 = insist on that kernel, 2 / 3 = and on its per-XCD / device-wide variant, 4 = on the row kernel),
+    ``_chunks_per_item`` (1, 2 or 4 consecutive chunks per work item of that kernel, 0 = choose; slices per workgroup of the
+    row kernel), ``_spin_limit`` (polls before a flag wait gives up, 0 = default) and
     ``_workspace`` (an int32 tensor to use instead of the wrapper's own, which it keeps per device and stream and whose
     fill launch it saves from the second call on) with ``_epoch`` (ssd_fused_opts.epoch for that tensor) are test and
     tuning hooks."""
@@ -392,13 +393,15 @@ def fused_plan(batch, seqlen, nheads, headdim, dstate, ngroups, chunk_size, work
     """Which kernel family the fused call would run on plain bf16 / fp32 tensors of these sizes and the library's
     estimate of every family's duration (no counterpart in the reference, whose fused wrappers have one kernel each:
     kernels/fused_globalbar.py:201-266, kernels/fused_concurrent.py:255-331).  Host logic only: needs no GPU.
-    Returns {"family": name, "chunks_per_item": R or 0, "estimate_us": {name: microseconds or None}}."""
+    Returns {"rows": slices, "family": name, "chunks_per_item": R or 0, "estimate_us": {name: microseconds or None}}: where
+    "rows" is not 0 the row kernel runs with that many slices of 16 state rows per workgroup, elsewhere "family" does."""
     nchunks = (seqlen + chunk_size - 1) // chunk_size
     dims = _lib.dims_arg(batch, seqlen, nheads, headdim, dstate, ngroups, chunk_size, nchunks)
     plan = _lib.SsdFusedPlan()
     _lib.check(_lib.load().ssd_query_fused_plan(dims, 1 if workspace else 0, int(compute_units), ctypes.byref(plan)),
                "ssd_query_fused_plan")
-    return {"family": _lib.SSD_FAMILIES[plan.family], "chunks_per_item": int(plan.chunks_per_item),
+    rows = _lib.load().ssd_query_fused_rows(dims, 1 if workspace else 0, int(compute_units))
+    return {"rows": max(int(rows), 0), "family": _lib.SSD_FAMILIES[plan.family], "chunks_per_item": int(plan.chunks_per_item),
             "estimate_us": {n: (float(v) if v > 0 else None) for n, v in zip(_lib.SSD_FAMILIES, plan.estimate_us)}}
 
 
