@@ -168,7 +168,8 @@ struct Choice {
 ssd::cost::Problem problem_of(const Params &p, int64_t n_cu)
 {
     ssd::cost::Problem q;
-    q.units = (int64_t)p.batch * p.nheads * (p.headdim / 32) / 4;
+    q.units = ((int64_t)p.batch * p.nheads * (p.headdim / 32) + 3) / 4;
+    q.quads = (int64_t)p.batch * p.ngroups * (((p.nheads / p.ngroups) * (p.headdim / 32) + 3) / 4);
     q.chunks = p.C; q.chunk_size = p.Q; q.dstate = p.dstate;
     q.n_cu = n_cu > 0 ? (int)n_cu : 256;
     return q;
@@ -186,6 +187,16 @@ Choice choose(const Params &p, bool fused, int64_t n_cu, bool few = true)
     if (fused && few && forced == 0 && ssd::cost::few_units(problem_of(p, n_cu))) {
         if (p.states ? pair_supported(p, true) : p.dt_out == ssd::DT_F32 && pair_supported(with_states_in_out(p), true))
             return {F_PAIR, !p.states, false, true};
+    }
+    // Groups whose tiles are no multiple of four: neither the four-tile nor the chain kernel takes the call, and a walk of one
+    // workgroup per tile (token-split) is what is left.  With room for the chunk states the pair goes in front of it from four
+    // chunks on where its estimate is a tenth lower.
+    const int in_group = (p.nheads / p.ngroups) * (p.headdim / 32);
+    if (fused && forced == 0 && in_group % 4 && p.C >= 4) {
+        const ssd::cost::Problem q = problem_of(p, n_cu);
+        if (ssd::cost::ragged_pair_us(q) < 0.9 * ssd::cost::token_split_us(q) &&
+            (p.states ? pair_supported(p) : p.dt_out == ssd::DT_F32 && pair_supported(with_states_in_out(p))))
+            return {F_PAIR, !p.states, false, false};
     }
     // Few state tiles, many chunks, fp32 `out`: the chunk-state launch keeps every compute unit busy where the
     // fused kernels have one workgroup per tile.  It writes the chunk states into `out`, and the streaming
@@ -277,7 +288,7 @@ double estimate_us(const ssd::cost::Problem &q, const Choice &c)
 {
     switch (c.family) {
         case F_FOUR_TILE: return ssd::cost::four_tile_us(q);
-        case F_PAIR: return ssd::cost::pair_us(q);
+        case F_PAIR: return q.quads > q.units ? ssd::cost::ragged_pair_us(q) : ssd::cost::pair_us(q);
         case F_TOKEN_SPLIT: return ssd::cost::token_split_us(q);
         default: return 1e30;
     }
@@ -711,7 +722,7 @@ int ssd_query_fused_plan(const ssd_dims *dims, int has_workspace, int compute_un
     const Choice c = choose(p, true, n_cu);
     if (ssd::mfma_supported(p)) plan->estimate_us[SSD_FAMILY_TOKEN_SPLIT] = (float)ssd::cost::token_split_us(q);
     if (ssd::quad_supported(p)) plan->estimate_us[SSD_FAMILY_FOUR_TILE] = (float)ssd::cost::four_tile_us(q);
-    if (pair_supported(with_states_in_out(p))) plan->estimate_us[SSD_FAMILY_PAIR] = (float)ssd::cost::pair_us(q);
+    if (pair_supported(with_states_in_out(p))) plan->estimate_us[SSD_FAMILY_PAIR] = (float)estimate_us(q, {F_PAIR, false, false, false});
     plan->family = c.family;
     if (ssd::chain_supported(p)) {
         double us = 0.;
@@ -752,6 +763,7 @@ int ssd_query_fused_wants_states(const ssd_tensor *x, const ssd_tensor *B, const
     if (rc) return rc;
     // what the call runs with a fp32 `out`, and whether it still does with the place it would be given
     const Choice c = choose(as_out, true, n_cu), given = p.out ? choose(as_states, true, n_cu) : c;
+    if (p.out && !c.few && rows_preferred(p, n_cu, true)) return 0;
     if (c.family == F_PAIR) {
         if (given.family != F_PAIR || (ssd::chain_supported(as_out) && chain_preferred(as_out, n_cu, packed_form(p)))) return 0;
         // Packed rows so long that a fp32 `out` runs the pair whatever the number of units: these calls have the chain

@@ -26,7 +26,8 @@ namespace ssd {
 namespace cost {
 
 struct Problem {
-    int64_t units;      // groups of four state tiles (32 headdim rows x dstate) that share (batch, group)
+    int64_t units;      // groups of four state tiles (32 headdim rows x dstate) that share (batch, group); tiles / 4, rounded up
+    int64_t quads;      // the same with every group's tiles rounded up to fours: workgroups of the chunk-state launch
     int chunks;         // chunks per sequence
     int chunk_size, dstate;
     int n_cu;           // compute units of the device
@@ -96,6 +97,15 @@ inline double pair_us(const Problem &q)
     const double x_bytes = (double)q.units * q.chunks * 256.0 * q.chunk_size;       // 4 tiles x 32 rows x Q x bf16
     const double s_bytes = (double)q.units * q.chunks * 512.0 * q.dstate;           // 4 tiles x 32 rows x N x fp32
     return 6.0 + (x_bytes + 3.0 * s_bytes) / 5.0e6 * (256.0 / q.n_cu);
+}
+
+// The same where a group's tiles are no multiple of four: the chunk-state launch takes 7.1 us a workgroup's chunk (the
+// four-tile kernel's time on a full device) also for workgroups that are not full, and is followed by the recurrence.
+inline double ragged_pair_us(const Problem &q)
+{
+    const double x_bytes = (double)q.units * q.chunks * 256.0 * q.chunk_size, s_bytes = (double)q.units * q.chunks * 512.0 * q.dstate;
+    const double states = (double)q.quads * q.chunks * 7.1 * work(q) / q.n_cu, bytes = (x_bytes + s_bytes) / 5.0e6 * (256.0 / q.n_cu);
+    return 6.0 + (states > bytes ? states : bytes) + 2.0 * s_bytes / 5.0e6 * (256.0 / q.n_cu);
 }
 
 // Row kernel (ssd_rows.hip): workgroups of kr slices of 16 state rows, one per compute unit, each walking its whole sequence.

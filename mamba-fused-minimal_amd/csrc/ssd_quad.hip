@@ -91,10 +91,11 @@ __global__ void __launch_bounds__(256, 2) quad_kernel(const Params p)
     char *wbuf = xring + kRing * 2048;                                   // 2 slots x Q weights
     char *stage = lds + kRing * NT * 1024 + 4 * wave_lds<NT, SPC>() + wave * kStage;
 
-    // Work item -> (batch, head, row slice); the four items of a workgroup share batch and group (checked on the
-    // host).  Consecutive workgroups sit on the same XCD (workgroups are dealt round-robin over the p.n_xcd XCDs), so
+    // Workgroup -> (batch, group) and four of its state tiles; where a group's tiles are no multiple of four (chunk states
+    // only), the last workgroup's waves without a tile compute the last one again and store nothing.  Consecutive workgroups sit on the same XCD (workgroups are dealt round-robin over the p.n_xcd XCDs), so
     // a batch's B is fetched from HBM by one or two L2 slices only.
-    const int n_wg = p.n_items >> 2, n_seg = CO ? p.n_seg : 1;
+    const int n_pt = p.headdim >> 5, tiles = (p.nheads / p.ngroups) * n_pt, wpg = (tiles + 3) >> 2;
+    const int n_wg = p.batch * p.ngroups * wpg, n_seg = CO ? p.n_seg : 1;
     const int per_xcd = (n_wg * n_seg + p.n_xcd - 1) / p.n_xcd;          // workgroups per XCD
     const int vwg = (int)(blockIdx.x % p.n_xcd) * per_xcd + (int)(blockIdx.x / p.n_xcd);
     if (vwg >= n_wg * n_seg) return;                                     // whole workgroup: no barrier is skipped
@@ -108,14 +109,13 @@ __global__ void __launch_bounds__(256, 2) quad_kernel(const Params p)
         c1 = min(p.C, c0 + cps);
         if (c0 >= c1) return;
     }
-    const int item = 4 * wg + wave;
-    const int n_pt = p.headdim >> 5;
-    const int pt = item % n_pt;
-    const int r1 = item / n_pt;
-    const int h = r1 % p.nheads;
-    const int b = r1 / p.nheads;
+    const int tile = min(4 * (wg % wpg) + wave, tiles - 1);
+    const bool exists = !CO || 4 * (wg % wpg) + wave < tiles;
+    const int pt = tile % n_pt;
+    const int g = (wg / wpg) % p.ngroups;
+    const int h = g * (p.nheads / p.ngroups) + tile / n_pt;
+    const int b = wg / (wpg * p.ngroups);
     const int C = c1, L = p.seqlen;      // chunks at and beyond c1 are not this workgroup's: never requested
-    const int g = h / (p.nheads / p.ngroups);
     const int p0 = pt * 32;
     const int dt_out = F32IO ? (int)DT_F32 : (CO ? p.dt_states : p.dt_out), dt_init = F32IO ? (int)DT_F32 : p.dt_init;
 
@@ -436,7 +436,7 @@ __global__ void __launch_bounds__(256, 2) quad_kernel(const Params p)
             // zero, which drops them -- the waits count a boundary's stores whether or not they reach memory.
             const int cp = c > c0 ? c - 1 : c0;
             store_state(make_rsrc((char *)p.states + (b * p.sst_b + cp * p.sst_c + h * p.sst_h) * esize_of(dt_out),
-                                  c > c0 ? slice_out * esize_of(dt_out) : 0), dt_out, (int)p.sst_p);
+                                  c > c0 && exists ? slice_out * esize_of(dt_out) : 0), dt_out, (int)p.sst_p);
 #pragma unroll
             for (int it = 0; it < NT; ++it)
 #pragma unroll
@@ -532,7 +532,7 @@ __global__ void __launch_bounds__(256, 2) quad_kernel(const Params p)
     }
     if (CO)
         store_state(make_rsrc((char *)p.states + (b * p.sst_b + (C - 1) * p.sst_c + h * p.sst_h) * esize_of(dt_out),
-                              slice_out * esize_of(dt_out)), dt_out, (int)p.sst_p);
+                              exists ? slice_out * esize_of(dt_out) : 0), dt_out, (int)p.sst_p);
     else
         store_state(make_rsrc(p.fin + b * p.sf_b + h * p.sf_h, slice_fin * 4), DT_F32, (int)p.sf_p);
 }
@@ -546,7 +546,6 @@ static bool inputs_ok(const Params &p)
     if (p.headdim % 32 != 0) return false;
     if (p.dstate != 64 && p.dstate != 128) return false;
     if (p.Q != 128 && p.Q != 256) return false;
-    if (((p.nheads / p.ngroups) * (p.headdim / 32)) % 4 != 0) return false;      // 4 tiles of one (batch, group)
     if (!aligned(p.x, 16) || (p.sx_b | p.sx_l | p.sx_h) % 8) return false;
     if (!aligned(p.B, 16) || (p.sB_b | p.sB_l | p.sB_g) % 8) return false;
     if ((int64_t)p.Q * 2 * p.sx_l >= (1LL << 31) || (int64_t)p.Q * 2 * p.sB_l >= (1LL << 31)) return false;
@@ -570,16 +569,16 @@ bool quad_supported(const Params &p)
 {
     using namespace quad;
     if (p.states || !p.out || !p.fin) return false;
-    if (!inputs_ok(p)) return false;
+    if (!inputs_ok(p) || ((p.nheads / p.ngroups) * (p.headdim / 32)) % 4) return false;      // four tiles of one (batch, group)
     if (!rows_ok(p.out, p.dt_out, p.so_b | p.so_c | p.so_h | p.so_p, p.so_p, p.headdim)) return false;
     if (!rows_ok(p.fin, DT_F32, p.sf_b | p.sf_h | p.sf_p, p.sf_p, p.headdim)) return false;
     if (p.init && !rows_ok(p.init, p.dt_init, p.sin_b | p.sin_h | p.sin_p, p.sin_p, p.headdim)) return false;
     return true;
 }
 
-bool quad_inputs_supported(const Params &p) { return quad::inputs_ok(p); }
+bool quad_inputs_supported(const Params &p) { return quad::inputs_ok(p) && ((p.nheads / p.ngroups) * (p.headdim / 32)) % 4 == 0; }
 
-// ... and the chunk-state call (`states` only), under the same conditions.
+// ... and the chunk-state call (`states` only), under the same conditions but for the number of tiles.
 bool quad_chunk_state_supported(const Params &p)
 {
     using namespace quad;
@@ -602,7 +601,7 @@ static hipError_t launch_quad_k(const Params &p, dim3 grid, hipStream_t s)
 template <int NT, int SPC, bool CO>
 static hipError_t launch_quad_t(const Params &p, hipStream_t s)
 {
-    dim3 grid((((p.n_items >> 2) * (CO ? p.n_seg : 1) + p.n_xcd - 1) / p.n_xcd) * p.n_xcd);
+    dim3 grid(((p.n_items * (CO ? p.n_seg : 1) + p.n_xcd - 1) / p.n_xcd) * p.n_xcd);
     const bool f32io = CO ? p.dt_states == DT_F32 : p.dt_out == DT_F32 && (!p.init || p.dt_init == DT_F32);
     if (p.seq) return f32io ? launch_quad_k<NT, SPC, true, true, CO>(p, grid, s) : launch_quad_k<NT, SPC, true, false, CO>(p, grid, s);
     return f32io ? launch_quad_k<NT, SPC, false, true, CO>(p, grid, s) : launch_quad_k<NT, SPC, false, false, CO>(p, grid, s);
@@ -618,10 +617,13 @@ static hipError_t launch_quad_c(const Params &p, hipStream_t s)
     return launch_quad_t<4, 4, CO>(p, s);
 }
 
+// workgroups that hold every state tile once
+static int units_of(const Params &p) { return p.batch * p.ngroups * (((p.nheads / p.ngroups) * (p.headdim / 32) + 3) / 4); }
+
 hipError_t launch_quad(const Params &p_in, hipStream_t s)
 {
     Params p = p_in;
-    p.n_items = p.batch * p.nheads * (p.headdim / 32);
+    p.n_items = units_of(p);
     if (p.n_items <= 0) return hipSuccess;
     if (p.n_cu <= 0) p.n_cu = 256;
     p.n_xcd = p.n_cu >= 32 ? p.n_cu / 32 : 1;       // an XCD is 32 compute units on this part
@@ -635,7 +637,7 @@ int set_quad_segment_chunks(int n) { return g_segment_chunks.exchange(n); }
 hipError_t launch_quad_chunk_state(const Params &p_in, hipStream_t s)
 {
     Params p = p_in;
-    p.n_items = p.batch * p.nheads * (p.headdim / 32);
+    p.n_items = units_of(p);
     if (p.n_items <= 0 || p.C <= 0) return hipSuccess;
     if (p.n_cu <= 0) p.n_cu = 256;
     p.n_xcd = p.n_cu >= 32 ? p.n_cu / 32 : 1;
@@ -648,7 +650,7 @@ hipError_t launch_quad_chunk_state(const Params &p_in, hipStream_t s)
         double best = 0;
         for (int k = 1; k <= p.C; ++k) {
             const int nseg = (p.C + k - 1) / k;
-            const int per_cu = ((p.n_items >> 2) * nseg + p.n_cu - 1) / p.n_cu;
+            const int per_cu = (p.n_items * nseg + p.n_cu - 1) / p.n_cu;
             const double t = per_cu * (k + 0.4);
             if (cps <= 0 || t < best) { best = t; cps = k; }
         }
