@@ -348,8 +348,8 @@ int ssd_fused_cumsum_chunk_state_passing_fwd_ws(const ssd_tensor *x, const ssd_t
  * f32/bf16/f16.  Innermost strides of C, prev_states and y must be 1.  accumulate != 0 adds to what y holds (the
  * intra-chunk half of the scan computed elsewhere) instead of overwriting it.  bf16 C with fp32 or bf16 states,
  * dstate 64/128, chunk size 64/128/256 and headdim % 32 == 0 run on the matrix cores: a fp32 state enters as bf16
- * hi + lo (the reference rounds the state to C's element type), a bf16 state as it is; everything else on a plain
- * FMA kernel (one thread per output element, orders of magnitude slower).  Size limits of the matrix-core kernels: one
+ * hi + lo (the reference rounds the state to C's element type), a bf16 state as it is; everything else on the fp32 matrix
+ * instructions, with fp32 products and sums.  Size limits of the bf16 kernels: one
  * chunk of C rows and one chunk of y rows (chunk_size * row pitch in bytes) must stay below 2 GiB; the sequence length
  * itself is not limited by them.
  */
