@@ -296,6 +296,15 @@ int ssd_query_fused_wants_states(const ssd_tensor *x, const ssd_tensor *B, const
                                  const ssd_tensor *final_states, const ssd_dims *dims);
 
 /*
+ * Whether a fused call on these very arguments needs nothing that a caller would bring along: 1 = ssd_fused_chunk_state_passing_fwd
+ * runs the very kernels that ssd_fused_chunk_state_passing_fwd_ws would with a workspace and SSD_KERNEL_AUTO, and a place for the
+ * chunk states would change nothing (ssd_query_fused_wants_states); 0 = not so; negative = rejected arguments.  Pure host logic.
+ */
+int ssd_query_fused_is_plain(const ssd_tensor *x, const ssd_tensor *B, const ssd_tensor *dt, const ssd_tensor *dA_cumsum,
+                             const ssd_tensor *seq_idx, const ssd_tensor *initial_states, const ssd_tensor *out,
+                             const ssd_tensor *final_states, const ssd_dims *dims);
+
+/*
  * dt preparation and per-chunk cumulative sum, the producer of `dt` and `dA_cumsum` for the three calls above.
  * Replaces _chunk_cumsum_fwd / _chunk_cumsum_fwd_kernel (kernels/ssd_chunk_state.py:176-199, 33-79):
  *   d = float(dt[b,l,h]) (+ dt_bias[h]); d = log1p(exp(d)) where dt_softplus and d <= 20; d = clamp(d, dt_min, dt_max);

@@ -782,6 +782,22 @@ int ssd_query_fused_wants_states(const ssd_tensor *x, const ssd_tensor *B, const
     return c.generic_pair && given.generic_pair && p.C >= 4 && 2 * tiles <= 3 * n_cu ? 1 : 0;
 }
 
+int ssd_query_fused_is_plain(const ssd_tensor *x, const ssd_tensor *B, const ssd_tensor *dt, const ssd_tensor *dA_cumsum,
+                             const ssd_tensor *seq_idx, const ssd_tensor *initial_states, const ssd_tensor *out,
+                             const ssd_tensor *final_states, const ssd_dims *dims)
+{
+    Params p;
+    int rc = fill_fused(p, x, B, dt, dA_cumsum, seq_idx, initial_states, nullptr, out, final_states, dims, 1);
+    if (rc) return rc;
+    const int n_cu = compute_units() > 0 ? compute_units() : 256;
+    if (ssd::chain_supported(p) && g_forced_split.load(std::memory_order_relaxed) == 0 && !rows_preferred(p, n_cu, true) &&
+        chain_preferred(p, n_cu, packed_form(p)))
+        return 0;
+    // (below four chunks a place for chunk states changes nothing)
+    if (p.dt_out == ssd::DT_F32 || p.C < 4) return 1;
+    return ssd_query_fused_wants_states(x, B, dt, dA_cumsum, seq_idx, initial_states, out, final_states, dims) == 0 ? 1 : 0;
+}
+
 int ssd_chunk_cumsum_fwd(const ssd_tensor *dt, const ssd_tensor *A, const ssd_tensor *dt_bias, const ssd_tensor *dt_out,
                          const ssd_tensor *dA_cumsum, int32_t batch, int32_t seqlen, int32_t nheads, int32_t chunk_size,
                          int dt_softplus, float dt_min, float dt_max, void *stream)

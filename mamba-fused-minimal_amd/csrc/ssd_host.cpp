@@ -2,9 +2,19 @@
 // ctypes.  Describing nine tensors as ssd_tensor structs field by field from Python takes longer than the kernels of a
 // small call do (13 us a fused call, of 27); here the sizes, strides and pointers are read off the tensor objects.
 // Nothing is checked or kept here: shapes are the wrappers' business (ssd_amd/ops.py), everything else the library's.
+//
+// The *_call functions are a wrapper's whole ordinary call in one: plain tensors of the shapes, types and strides that need no
+// conversion, outputs allocated here, on the current device and stream.  They return None, and have done nothing, wherever
+// anything is out of the ordinary -- other shapes or types, tensor subclasses, several devices, a call that the kernel with a
+// kept workspace would serve or that gains from room for chunk states -- and the wrapper goes its general way, which also
+// says what is wrong.  A small fused call (2 x 384 tokens x 13 heads) costs the host 12.5 us through the general way and 7 us
+// through this one, which is what it takes: its kernel runs 6 us.
 #include <Python.h>
 
+#include <torch/csrc/Dtype.h>
 #include <torch/csrc/autograd/python_variable.h>
+
+#include <ATen/ops/empty.h>
 
 #include <string>
 
@@ -246,9 +256,240 @@ PyObject *wants_states(PyObject *, PyObject *const *a, Py_ssize_t n)
     });
 }
 
+// ---- whole ordinary calls -------------------------------------------------------------------------------------------
+
+struct OutOfTheOrdinary {};      // the general way, then
+
+bool ours(at::ScalarType t) { return t == at::kFloat || t == at::kBFloat16 || t == at::kHalf; }
+
+// A plain dense tensor of `dim` dimensions, none of them empty, on GPU `device`; its last dimension contiguous where asked.
+const at::Tensor &plain(PyObject *o, int64_t dim, int64_t device, bool inner = true)
+{
+    if (!THPVariable_CheckExact(o)) throw OutOfTheOrdinary();
+    const at::Tensor &v = THPVariable_Unpack(o);
+    if (!v.is_cuda() || v.get_device() != device || v.layout() != at::kStrided || v.dim() != dim || v.numel() == 0 ||
+        (inner && v.stride(dim - 1) != 1))
+        throw OutOfTheOrdinary();
+    return v;
+}
+
+void need(bool ok) { if (!ok) throw OutOfTheOrdinary(); }
+
+template <class... N> bool sized(const at::Tensor &v, N... n)
+{
+    const int64_t want[] = {(int64_t)n...};
+    for (size_t i = 0; i < sizeof...(n); ++i)
+        if (v.size(i) != want[i]) return false;
+    return true;
+}
+
+at::Tensor made(at::IntArrayRef sizes, at::ScalarType type, const at::Tensor &like)
+{
+    return at::empty(sizes, like.options().dtype(type).requires_grad(false).memory_format(c10::nullopt));
+}
+
+ssd_tensor described(const at::Tensor &v)
+{
+    ssd_tensor t{};
+    t.dtype = v.scalar_type() == at::kInt ? 0 : v.scalar_type() == at::kFloat ? SSD_F32 : v.scalar_type() == at::kBFloat16 ? SSD_BF16 : SSD_F16;
+    t.data = v.data_ptr();
+    const auto strides = v.strides();
+    for (size_t i = 0; i < strides.size(); ++i) t.stride[i] = strides[i];
+    return t;
+}
+
+at::ScalarType type_of(PyObject *o)
+{
+    need(THPDtype_Check(o));
+    const at::ScalarType t = ((THPDtype *)o)->scalar_type;
+    need(ours(t));
+    return t;
+}
+
+// seq_idx (b, L) or None
+ssd_tensor sequences(PyObject *o, int64_t b, int64_t L, int64_t device)
+{
+    if (o == Py_None) return ssd_tensor{};
+    const at::Tensor &v = plain(o, 2, device, false);
+    need(v.scalar_type() == at::kInt && sized(v, b, L));
+    return described(v);
+}
+
+PyObject *pair_of(const at::Tensor &a, const at::Tensor &b)
+{
+    PyObject *x = THPVariable_Wrap(a);
+    PyObject *y = x ? THPVariable_Wrap(b) : nullptr;
+    PyObject *t = y ? PyTuple_Pack(2, x, y) : nullptr;
+    Py_XDECREF(x);
+    Py_XDECREF(y);
+    return t;
+}
+
+template <class F>
+PyObject *ordinary(Py_ssize_t got, Py_ssize_t want, F &&f)
+{
+    return guarded(got, want, [&]() -> PyObject * {
+        try {
+            return f();
+        } catch (const OutOfTheOrdinary &) {
+            Py_RETURN_NONE;
+        }
+    });
+}
+
+struct Inputs {
+    ssd_tensor x, B, dt, dA, seq;
+    ssd_dims d;
+    const at::Tensor *xv;
+};
+
+Inputs inputs(PyObject *Bo, PyObject *xo, PyObject *dto, PyObject *dAo, PyObject *seqo, int64_t device)
+{
+    const at::Tensor &x = plain(xo, 4, device), &B = plain(Bo, 4, device), &dt = plain(dto, 4, device, false), &dA = plain(dAo, 4, device, false);
+    const int64_t b = x.size(0), L = x.size(1), H = x.size(2), G = B.size(2), C = dt.size(2), Q = dt.size(3);
+    need(ours(x.scalar_type()) && B.scalar_type() == x.scalar_type() && dt.scalar_type() == at::kFloat && dA.scalar_type() == at::kFloat);
+    need(H % G == 0 && B.size(0) == b && B.size(1) == L && sized(dt, b, H, C, Q) && sized(dA, b, H, C, Q) && C == (L + Q - 1) / Q);
+    need(b <= INT32_MAX && L <= INT32_MAX && H <= INT32_MAX && x.size(3) <= INT32_MAX && B.size(3) <= INT32_MAX && C <= INT32_MAX && Q <= INT32_MAX);
+    return Inputs{described(x), described(B), described(dt), described(dA), sequences(seqo, b, L, device),
+                  ssd_dims{(int32_t)b, (int32_t)L, (int32_t)H, (int32_t)x.size(3), (int32_t)B.size(3), (int32_t)G, (int32_t)Q, (int32_t)C}, &x};
+}
+
+// B, x, dt, dA_cumsum, out_dtype, initial_states, seq_idx, most (state tile, chunk) pairs, device, stream -> (out, final_states) or None
+PyObject *fused_call(PyObject *, PyObject *const *a, Py_ssize_t n)
+{
+    return ordinary(n, 10, [&]() -> PyObject * {
+        const int64_t most = number(a[7]), device = number(a[8]);
+        void *const stream = pointer(a[9]);
+        const at::ScalarType out_type = type_of(a[4]);
+        const Inputs in = inputs(a[0], a[1], a[2], a[3], a[6], device);
+        const ssd_dims &d = in.d;
+        // beyond, the general way's kept workspace may have to grow
+        need((int64_t)d.batch * d.nheads * ((d.headdim + 31) / 32) * d.nchunks <= most);
+        ssd_tensor init{};
+        if (a[5] != Py_None) {
+            const at::Tensor &v = plain(a[5], 4, device);
+            need(ours(v.scalar_type()) && sized(v, d.batch, d.nheads, d.headdim, d.dstate));
+            init = described(v);
+        }
+        // contiguous outputs at a made-up, aligned address, as the allocator will give them
+        const int64_t N = d.dstate, P = d.headdim, H = d.nheads, C = d.nchunks;
+        void *const somewhere = (void *)(uintptr_t)4096;
+        const int code = out_type == at::kFloat ? SSD_F32 : out_type == at::kBFloat16 ? SSD_BF16 : SSD_F16;
+        ssd_tensor out{somewhere, code, 0, {C * H * P * N, H * P * N, P * N, N, 1}}, fin{somewhere, SSD_F32, 0, {H * P * N, P * N, N, 1, 0}};
+        need(ssd_query_fused_is_plain(&in.x, &in.B, &in.dt, &in.dA, &in.seq, &init, &out, &fin, &d) == 1);
+        const at::Tensor out_v = made({d.batch, C, H, P, N}, out_type, *in.xv), fin_v = made({d.batch, H, P, N}, at::kFloat, *in.xv);
+        out.data = out_v.data_ptr();
+        fin.data = fin_v.data_ptr();
+        need(unlocked([&] {
+            return ssd_fused_chunk_state_passing_fwd(&in.x, &in.B, &in.dt, &in.dA, &in.seq, &init, nullptr, &out, &fin, &d, 1, stream);
+        }) == SSD_OK);
+        return pair_of(out_v, fin_v);
+    });
+}
+
+// B, x, dt, dA_cumsum, seq_idx, states_in_fp32, device, stream -> states or None
+PyObject *chunk_state_call(PyObject *, PyObject *const *a, Py_ssize_t n)
+{
+    return ordinary(n, 8, [&]() -> PyObject * {
+        const bool f32 = number(a[5]) != 0;
+        const int64_t device = number(a[6]);
+        void *const stream = pointer(a[7]);
+        const Inputs in = inputs(a[0], a[1], a[2], a[3], a[4], device);
+        const ssd_dims &d = in.d;
+        const at::Tensor v = made({d.batch, d.nchunks, d.nheads, d.headdim, d.dstate}, f32 ? at::kFloat : in.xv->scalar_type(), *in.xv);
+        const ssd_tensor states = described(v);
+        need(unlocked([&] { return ssd_chunk_state_fwd(&in.x, &in.B, &in.dt, &in.dA, &in.seq, &states, &d, 1, stream); }) == SSD_OK);
+        return THPVariable_Wrap(v);
+    });
+}
+
+// states, dA_chunk, initial_states, seq_idx, chunk_size (0 without seq_idx), out_dtype (None: that of states), device, stream
+// -> (out, final_states) or None
+PyObject *state_passing_call(PyObject *, PyObject *const *a, Py_ssize_t n)
+{
+    return ordinary(n, 8, [&]() -> PyObject * {
+        const int64_t Q = number(a[4]), device = number(a[6]);
+        void *const stream = pointer(a[7]);
+        const at::Tensor &s = plain(a[0], 4, device), &da = plain(a[1], 3, device, false);
+        const int64_t b = s.size(0), C = s.size(1), H = s.size(2), dim = s.size(3);
+        need(ours(s.scalar_type()) && da.scalar_type() == at::kFloat && sized(da, b, H, C));
+        need(b <= INT32_MAX && C <= INT32_MAX && H <= INT32_MAX && dim <= INT32_MAX && Q <= INT32_MAX);
+        ssd_tensor init{}, seq{};
+        if (a[2] != Py_None) {
+            const at::Tensor &v = plain(a[2], 3, device);
+            need(ours(v.scalar_type()) && sized(v, b, H, dim));
+            init = described(v);
+        }
+        int64_t L = 0;
+        if (a[3] != Py_None) {
+            L = plain(a[3], 2, device, false).size(1);
+            need(L <= INT32_MAX && Q > 0);
+            seq = sequences(a[3], b, L, device);
+        }
+        const at::ScalarType out_type = a[5] == Py_None ? s.scalar_type() : type_of(a[5]);
+        const at::Tensor out_v = made({b, C, H, dim}, out_type, s), fin_v = made({b, H, dim}, at::kFloat, s);
+        const ssd_tensor t = described(s), d = described(da), out = described(out_v), fin = described(fin_v);
+        need(unlocked([&] {
+            return ssd_state_passing_fwd(&t, &d, &init, &seq, &out, &fin, (int32_t)b, (int32_t)C, (int32_t)H, (int32_t)dim, (int32_t)L,
+                                         a[3] != Py_None ? (int32_t)Q : 0, stream);
+        }) == SSD_OK);
+        return pair_of(out_v, fin_v);
+    });
+}
+
+// dt, A, dt_bias, chunk_size, dt_softplus, dt_min, dt_max, device, stream -> (dA_cumsum, dt_out) or None
+PyObject *chunk_cumsum_call(PyObject *, PyObject *const *a, Py_ssize_t n)
+{
+    return ordinary(n, 9, [&]() -> PyObject * {
+        need(PyLong_Check(a[3]));
+        const int64_t Q = number(a[3]), device = number(a[7]);
+        const int softplus = (int)number(a[4]);
+        const float lo = (float)real(a[5]), hi = (float)real(a[6]);
+        void *const stream = pointer(a[8]);
+        const at::Tensor &dt = plain(a[0], 3, device, false), &A = plain(a[1], 1, device, false);
+        const int64_t b = dt.size(0), L = dt.size(1), H = dt.size(2);
+        need(ours(dt.scalar_type()) && ours(A.scalar_type()) && A.size(0) == H && Q > 0 && Q <= INT32_MAX);
+        need(b <= INT32_MAX && L <= INT32_MAX && H <= INT32_MAX);
+        ssd_tensor bias{};
+        if (a[2] != Py_None) {
+            const at::Tensor &v = plain(a[2], 1, device, false);
+            need(ours(v.scalar_type()) && v.size(0) == H);
+            bias = described(v);
+        }
+        const int64_t C = (L + Q - 1) / Q;
+        const at::Tensor dt_v = made({b, H, C, Q}, at::kFloat, dt), da_v = made({b, H, C, Q}, at::kFloat, dt);
+        const ssd_tensor t = described(dt), At = described(A), out = described(dt_v), da = described(da_v);
+        need(unlocked([&] { return ssd_chunk_cumsum_fwd(&t, &At, &bias, &out, &da, (int32_t)b, (int32_t)L, (int32_t)H, (int32_t)Q, softplus, lo, hi, stream); }) ==
+             SSD_OK);
+        return pair_of(da_v, dt_v);
+    });
+}
+
+// C, prev_states, dA_cumsum, seq_idx, out_dtype (None: that of C), device, stream -> y or None
+PyObject *scan_states_call(PyObject *, PyObject *const *a, Py_ssize_t n)
+{
+    return ordinary(n, 7, [&]() -> PyObject * {
+        const int64_t device = number(a[5]);
+        void *const stream = pointer(a[6]);
+        const at::Tensor &c = plain(a[0], 4, device), &s = plain(a[1], 5, device), &da = plain(a[2], 4, device, false);
+        const int64_t b = c.size(0), L = c.size(1), G = c.size(2), N = c.size(3), C = s.size(1), H = s.size(2), P = s.size(3), Q = da.size(3);
+        need(ours(c.scalar_type()) && ours(s.scalar_type()) && da.scalar_type() == at::kFloat);
+        need(H % G == 0 && s.size(0) == b && s.size(4) == N && sized(da, b, H, C, Q) && C == (L + Q - 1) / Q);
+        need(b <= INT32_MAX && L <= INT32_MAX && H <= INT32_MAX && P <= INT32_MAX && N <= INT32_MAX && C <= INT32_MAX && Q <= INT32_MAX);
+        const ssd_tensor seq = sequences(a[3], b, L, device);
+        const at::Tensor y = made({b, L, H, P}, a[4] == Py_None ? c.scalar_type() : type_of(a[4]), c);
+        const ssd_tensor ct = described(c), st = described(s), dt = described(da), yt = described(y);
+        const ssd_dims d{(int32_t)b, (int32_t)L, (int32_t)H, (int32_t)P, (int32_t)N, (int32_t)G, (int32_t)Q, (int32_t)C};
+        need(unlocked([&] { return ssd_chunk_scan_states_fwd(&ct, &st, &dt, &seq, &yt, &d, 0, stream); }) == SSD_OK);
+        return THPVariable_Wrap(y);
+    });
+}
+
 #define SSD_METHOD(name) {#name, (PyCFunction)(void (*)(void))name, METH_FASTCALL, nullptr}
 PyMethodDef methods[] = {SSD_METHOD(chunk_state), SSD_METHOD(state_passing), SSD_METHOD(fused), SSD_METHOD(fused_scan),
                          SSD_METHOD(chunk_cumsum), SSD_METHOD(chunk_scan_states), SSD_METHOD(wants_states),
+                         SSD_METHOD(fused_call), SSD_METHOD(chunk_state_call), SSD_METHOD(state_passing_call), SSD_METHOD(chunk_cumsum_call),
+                         SSD_METHOD(scan_states_call),
                          {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_ssd_host", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
 

@@ -17,7 +17,7 @@ _DTYPES = {torch.float32: SSD_F32, torch.bfloat16: SSD_BF16, torch.float16: SSD_
 EXPORTS = ("ssd_version", "ssd_status_string", "ssd_chunk_state_fwd", "ssd_state_passing_fwd",
            "ssd_fused_chunk_state_passing_fwd", "ssd_fused_chunk_state_passing_fwd_ws", "ssd_fused_workspace_bytes", "ssd_fused_workspace_bytes_for",
            "ssd_fused_workspace_status", "ssd_fused_workspace_status_of", "ssd_set_chain_xcds", "ssd_measure_traffic_floor", "ssd_measure_traffic_floor_part", "ssd_fused_scan_workspace_bytes", "ssd_fused_chunk_state_passing_scan_fwd", "ssd_fused_chunk_state_passing_fwd_static", "ssd_fused_static_status",
-           "ssd_fused_cumsum_chunk_state_passing_fwd", "ssd_fused_cumsum_chunk_state_passing_fwd_ws", "ssd_query_path", "ssd_query_fused_plan", "ssd_query_fused_rows", "ssd_query_fused_wants_states", "ssd_chunk_cumsum_fwd", "ssd_chunk_scan_states_fwd", "ssd_set_scan_kernel", "ssd_set_token_split", "ssd_set_segment_chunks")
+           "ssd_fused_cumsum_chunk_state_passing_fwd", "ssd_fused_cumsum_chunk_state_passing_fwd_ws", "ssd_query_path", "ssd_query_fused_plan", "ssd_query_fused_rows", "ssd_query_fused_is_plain", "ssd_query_fused_wants_states", "ssd_chunk_cumsum_fwd", "ssd_chunk_scan_states_fwd", "ssd_set_scan_kernel", "ssd_set_token_split", "ssd_set_segment_chunks")
 
 
 class SsdTensor(ctypes.Structure):
@@ -102,6 +102,8 @@ def load():
     lib.ssd_query_fused_plan.restype = ctypes.c_int
     lib.ssd_query_fused_plan.argtypes = [D, ctypes.c_int, ctypes.c_int, ctypes.POINTER(SsdFusedPlan)]
     lib.ssd_query_fused_wants_states.restype = ctypes.c_int
+    lib.ssd_query_fused_is_plain.restype = ctypes.c_int
+    lib.ssd_query_fused_is_plain.argtypes = [T, T, T, T, T, T, T, T, D]
     lib.ssd_query_fused_wants_states.argtypes = [T, T, T, T, T, T, T, T, D]
     lib.ssd_chunk_cumsum_fwd.restype = ctypes.c_int
     lib.ssd_chunk_cumsum_fwd.argtypes = [T, T, T, T, T, i32, i32, i32, i32, ctypes.c_int, ctypes.c_float, ctypes.c_float, vp]

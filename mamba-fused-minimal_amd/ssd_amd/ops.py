@@ -27,6 +27,15 @@ def _stream(t):
 _raw_stream = torch._C._cuda_getCurrentRawStream
 
 
+def _ordinary(t, call, *args):
+    """call(*args, device, stream) of the extension module: a wrapper's ordinary call in one.  None, and nothing has happened,
+    where anything about it is out of the ordinary (csrc/ssd_host.cpp): the wrapper's general way follows."""
+    if not t.is_cuda:
+        return None
+    device = torch._C._cuda_getDevice()
+    return call(*args, device, _raw_stream(device))
+
+
 def _on_device(t, call, *args):
     """call(*args, stream handle) with t's device current."""
     index = t.device.index
@@ -138,6 +147,11 @@ def _fused_scan_workspace_need(device, sizes, with_out, chunks_per_item):
     return int(_lib.load().ssd_fused_scan_workspace_bytes(_lib.dims_arg(*sizes), with_out, chunks_per_item))
 
 
+# (state tile, chunk) pairs whose flags fit the smallest workspace that is kept: a call of no more of them that needs no
+# workspace leaves the kept one alone.
+_WORKSPACE_PAIRS = (1 << 16) // 4 - _lib.SSD_WORKSPACE_HEADER_INTS
+
+
 def _own_workspace(x, nbytes):
     """-> the _Kept of x's device and current stream, holding at least nbytes (None under stream capture)."""
     if torch.cuda.is_current_stream_capturing():
@@ -220,6 +234,10 @@ def _prep_inputs(B, x, dt, dA_cumsum, seq_idx):
 
 
 def _chunk_state_fwd(B, x, dt, dA_cumsum, seq_idx=None, states=None, states_in_fp32=True):
+    if states is None:
+        done = _ordinary(x, _lib.host().chunk_state_call, B, x, dt, dA_cumsum, seq_idx, 1 if states_in_fp32 else 0)
+        if done is not None:
+            return done
     return _chunk_state_impl(B, x, dt, dA_cumsum, seq_idx, states, states_in_fp32, True)
 
 
@@ -248,6 +266,10 @@ def _chunk_state_impl(B, x, dt, dA_cumsum, seq_idx, states, states_in_fp32, _cla
 
 def _state_passing_fwd(states, dA_chunk_cumsum, initial_states=None, seq_idx=None, chunk_size=None,
                        out_dtype=None):
+    done = _ordinary(states, _lib.host().state_passing_call, states, dA_chunk_cumsum, initial_states, seq_idx,
+                     chunk_size if isinstance(chunk_size, int) else 0, out_dtype)
+    if done is not None:
+        return done
     batch, nchunks, nheads, dim = states.shape
     assert dA_chunk_cumsum.shape == (batch, nheads, nchunks)
     if initial_states is not None:
@@ -293,6 +315,11 @@ def _fused_chunk_state_state_passing_fwd(B, x, dt, dA_cumsum, out_dtype, initial
     ``_workspace`` (an int32 tensor to use instead of the wrapper's own, which it keeps per device and stream and whose
     fill launch it saves from the second call on) with ``_epoch`` (ssd_fused_opts.epoch for that tensor) are test and
     tuning hooks."""
+    if states is None and _clamp is True and _kernel == 0 and _spin_limit == 0 and _workspace is None and _chunks_per_item == 0:
+        wanted = out_dtype if out_dtype is not None else torch.float32 if states_in_fp32 else B.dtype
+        done = _ordinary(x, _lib.host().fused_call, B, x, dt, dA_cumsum, wanted, initial_states, seq_idx, _WORKSPACE_PAIRS)
+        if done is not None:
+            return done
     batch, seqlen, nheads, headdim = x.shape
     _, _, nchunks, chunk_size = dt.shape
     _, _, ngroups, dstate = B.shape
@@ -423,6 +450,9 @@ def _chunk_cumsum_fwd(dt, A, chunk_size, dt_bias=None, dt_softplus=False, dt_lim
     """dt preparation + per-chunk cumulative sum of dt * A; same call surface as the reference's
     kernels/ssd_chunk_state.py:176-199.  dt (batch, seqlen, nheads) -> (dA_cumsum, dt_out), both
     (batch, nheads, nchunks, chunk_size) fp32."""
+    done = _ordinary(dt, _lib.host().chunk_cumsum_call, dt, A, dt_bias, chunk_size, int(bool(dt_softplus)), float(dt_limit[0]), float(dt_limit[1]))
+    if done is not None:
+        return done
     batch, seqlen, nheads = dt.shape
     assert A.shape == (nheads,)
     if dt_bias is not None:
@@ -519,6 +549,10 @@ def _chunk_scan_states_fwd(C, prev_states, dA_cumsum, seq_idx=None, out=None, ou
     state passing; dA_cumsum (batch, nheads, nchunks, chunk_size).  Returns y (batch, seqlen, nheads, headdim) of
     ``out_dtype`` (default: C's, as the reference's ``out`` takes x's); with ``out=`` the result goes there, and with
     ``accumulate=True`` it is added to what ``out`` holds (the intra-chunk half of the scan)."""
+    if out is None and not accumulate:
+        done = _ordinary(C, _lib.host().scan_states_call, C, prev_states, dA_cumsum, seq_idx, out_dtype)
+        if done is not None:
+            return done
     batch, seqlen, ngroups, dstate = C.shape
     _, nchunks, nheads, headdim, _ = prev_states.shape
     chunk_size = dA_cumsum.shape[-1]
