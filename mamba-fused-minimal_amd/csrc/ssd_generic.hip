@@ -1,18 +1,26 @@
-// SSD chunk-state contraction (optionally with the recurrence) on the fp32 matrix instructions, for whatever the bf16
-// kernels do not take: fp32 and fp16 inputs, any headdim, dstate, chunk size and alignment.  The weighted x and B enter
-// v_mfma_f32_16x16x4_f32 as fp32 values and every sum is fp32, so fp32 inputs keep fp32 accuracy.
+// SSD chunk-state contraction (optionally with the recurrence) for whatever the bf16 kernels do not take: fp32 and fp16
+// inputs, any headdim, dstate, chunk size and alignment, with the accuracy of fp32 products and sums.
 //
-// Where its time goes: the fp32 matrix instructions (256 flop per clock and compute unit, a sixteenth of bf16's) are the
-// largest part -- fp32, batch 2 x 2048 tokens x 24 heads x 64 x 128: 1.6 GFLOP, 10 us, and 41 MB, 8 us; 21 us measured (an
-// FMA kernel that staged both operands through LDS: 92 us); fp16, batch 8 x 3001 x 48 heads: 18.9 GFLOP in 187 us.  The
-// matrix units are busy 56 % of that fp32 launch; a wave waits 64 % of its clocks to issue, with three of them on a SIMD, and
-// 19 % in s_waitcnt, and the rest of the launch is where the waves of a SIMD start, or add up and store, together.  So the
-// operands must cost next to no issue slots: a lane loads A consecutive headdim elements of one token's x row and S
-// consecutive dstate elements of its B row with one load each, and that *is* the operand layout -- lane i of a 16-lane group
-// stands for rows A i .. A i + A-1 and columns S i .. S i + S-1 of the tile, the four lane groups for four consecutive tokens,
-// and matrix instruction (r, s) multiplies the r-th element of every x vector with the s-th of every B vector.  No LDS on the
-// way in, no barrier in the loop, whole rows per load; the accumulators of one lane are S consecutive columns, so rows leave
-// as vectors as well.
+// The fp32 matrix instructions (256 flop per clock and compute unit) are a sixteenth of bf16's, so an operand enters as the
+// sum of bf16 values: the product x * w and an fp32 B as three (all 24 bits), an f16 B as two, a bf16 B as itself, and
+// v_mfma_f32_16x16x32_bf16 multiplies all pairs of parts but those below 2^-24 of the largest: 6, 5 or 3 instructions of 16 clocks
+// where the fp32 ones take 256.  Each adds 32 products at a time, so the sums round less often: error against 64 bits 0.58 -
+// 0.75e-7 where the fp32 instructions left 0.66 - 1.3e-7 (fp32, fp16 and odd sizes, fast and slow decays).  Where a sum is not finite
+// (an infinite input, or one that rounds to an infinite bf16) the fp32 instructions do the wave's tokens again.
+//
+// What bounds it: the vector instructions that split the operands -- 6 to 8 per element, about as many clocks as the matrix
+// instructions take, and the two hardly overlap on a SIMD --, and for small calls a wave's start and the adding up at the end.
+// Chunk states, fp32 matrix instructions / this: fp16, 2 x 3001 tokens x 24 heads x 64 x 128 31.5 / 24.3 us, 8 x 3001 x 48 188 / 120;
+// fp32, 2 x 2048 x 24 20.4 / 18.6; 1024 x 8 x 64 x 64 8.6 / 6.3.  A lane loads A consecutive headdim elements of eight tokens' x
+// rows and S consecutive dstate elements of their B rows, and its eight tokens of one row or column *are* the operand layout: lane i
+// of a 16-lane group stands for rows A i .. A i + A-1 and columns S i .. S i + S-1 of the tile, the four lane groups for eight
+// consecutive tokens each, and matrix instruction (r, s) multiplies the r-th elements of the x vectors with the s-th of the B
+// vectors.  No LDS on the way in, no barrier in the loop, whole rows per load; the accumulators of one lane are S consecutive
+// columns, so rows leave as vectors as well.
+//
+// The walk over a sequence's chunks (FUSED: one chunk, or a 16-bit out without room for chunk states) keeps the fp32 matrix
+// instructions: with the parts of the operands beside the running state a 64 x 64 tile leaves one wave a SIMD, and it was
+// slower (fp16, 8 x 3000 x 48 x 64 x 128 234 / 242 us, 8 x 102 x 76 x 128 x 128 47 / 64, 8 x 2000 x 60 x 40 x 40 in chunks of 100 114 / 134).
 //
 // One workgroup owns a (16 A) x (16 S) tile of one (batch, head) and chunk; its SPLIT = 4 waves take a quarter of the
 // chunk's tokens each and add up through LDS, after which wave v holds accumulator q = v of every instruction.  In
@@ -85,13 +93,41 @@ __device__ __forceinline__ void store_state(void *base, int64_t off, int dt, con
 }
 
 constexpr int kWaves = 4;
-constexpr int kWindow = 64;      // tokens whose weights a wave computes at once, one per lane
-// matrix steps of four tokens whose rows are loaded together, a group ahead of their use: a group's matrix instructions
+constexpr int kWindow = 64;      // walk: tokens whose weights a wave computes at once, one per lane
+// walk: matrix steps of four tokens whose rows are loaded together, a group ahead of their use: a group's matrix instructions
 // (32 clocks each) have to last for a load's way from memory
 constexpr int group_of(int tiles) { return tiles >= 12 ? 4 : 2; }
+constexpr int kStep = 32;        // tokens of a bf16 matrix instruction
 
+// Eight fp32 values as the sum of PARTS bf16 ones each (three hold all 24 bits of a value, two the 11 bits of an f16), every
+// part the rest rounded to nearest.
+using tile::bf16x8;
+template <int PARTS>
+__device__ __forceinline__ void split(const float (&v)[8], bf16x8 (&parts)[PARTS])
+{
+    float rest[8];
+#pragma unroll
+    for (int t = 0; t < 8; ++t) rest[t] = v[t];
+#pragma unroll
+    for (int q = 0; q < PARTS; ++q) {
+        tile::u32x4 packed;
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+            uint32_t two = tile::pack_bf16(rest[2 * t], rest[2 * t + 1]);
+            asm volatile("" : "+v"(two));      // keeps the compiler from converting a second time
+            packed[t] = two;
+            if (q + 1 < PARTS) {
+                rest[2 * t] -= __builtin_bit_cast(float, two << 16);
+                rest[2 * t + 1] -= __builtin_bit_cast(float, two & 0xffff0000u);
+            }
+        }
+        parts[q] = __builtin_bit_cast(bf16x8, packed);
+    }
+}
+// parts of an element of B: a bf16 is one, an f16 two, an fp32 three
+template <typename T> constexpr int kBParts = sizeof(T) == 4 ? 3 : std::is_same<T, _Float16>::value ? 2 : 1;
 template <int A, int S, typename T, int SPLIT, bool FUSED>
-__global__ void __launch_bounds__(64 * kWaves, FUSED ? 2 : 3) generic_kernel(const Params p)
+__global__ void __launch_bounds__(64 * kWaves, 2) generic_kernel(const Params p)
 {
     // partial tiles: accumulator q of the wave that owns it, from each of the three others
     constexpr int SV = S == 3 ? 4 : S;
@@ -160,6 +196,8 @@ __global__ void __launch_bounds__(64 * kWaves, FUSED ? 2 : 3) generic_kernel(con
 #pragma unroll
             for (int s = 0; s < S; ++s) acc[r][s] = f32x4{0.f, 0.f, 0.f, 0.f};
 
+        if constexpr (FUSED) {
+        // the walk: fp32 matrix instructions, steps of four tokens, one per lane group
         for (int w0 = k_begin; w0 < k_end; w0 += kWindow) {
             const int steps = (min(kWindow, k_end - w0) + 3) >> 2;
             const T *xw = xc + (int64_t)(w0 + sub) * p.sx_l, *Bw = Bc + (int64_t)(w0 + sub) * p.sB_l;
@@ -212,6 +250,118 @@ __global__ void __launch_bounds__(64 * kWaves, FUSED ? 2 : 3) generic_kernel(con
                         for (int s = 0; s < S; ++s) acc[r][s] = __builtin_amdgcn_mfma_f32_16x16x4f32(xs[r], bs[s], acc[r][s], 0, 0, 0);
                 }
             }
+        }
+        } else {
+        // Steps of 32 tokens: lane group `sub` holds the tokens 8 sub + t, t = 0 .. 7, of its rows and columns.  The rows of the
+        // next step are on their way while a step is multiplied, the inputs of the weights (one token per lane) a window of
+        // two steps ahead.
+        const int steps = k_begin < k_end ? (k_end - k_begin + kStep - 1) / kStep : 0;
+        Row<A, T> xr[8];
+        Row<S, T> br[8];
+        auto place = [&](int st, int t) {
+            const int k = k_begin + st * kStep + 8 * sub + t;
+            return (int64_t)(k < k_end ? k : 0);      // elsewhere: the chunk's first token, not used
+        };
+        auto load_x = [&](int st) {
+#pragma unroll
+            for (int t = 0; t < 8; ++t) xr[t] = load_row<A>(xc + place(st, t) * p.sx_l);
+        };
+        auto load_B = [&](int st) {
+#pragma unroll
+            for (int t = 0; t < 8; ++t) br[t] = load_row<S>(Bc + place(st, t) * p.sB_l);
+        };
+        float da_k = 0.f, dt_k = 0.f;
+        int32_t id_k = 0;
+        auto load_weights = [&](int window) {
+            const int kl = min(k_begin + window * 2 * kStep + lane, k_end - 1);      // lanes past the end repeat the last token; nobody asks them
+            da_k = dab[c * p.sda_c + (int64_t)kl * p.sda_k];
+            dt_k = dtb[c * p.sdt_c + (int64_t)kl * p.sdt_k];
+            id_k = sqb ? sqb[(int64_t)(t0 + kl) * p.ssq_l] : 0;
+        };
+        auto weight = [&](int window) {      // zero for tokens past the end
+            float ex = last - da_k;
+            if (p.clamp) ex = fminf(ex, 0.f);
+            const float w = __expf(ex) * dt_k;
+            return id_k != id_last || k_begin + window * 2 * kStep + lane >= k_end ? 0.f : w;
+        };
+        // row r of the step's x rows times the weights, column s of its B rows, as fp32 values (tokens past the end: zero times
+        // whatever the first token holds)
+        auto products = [&](int st, float w, auto r, float (&v)[8]) {
+#pragma unroll
+            for (int t = 0; t < 8; ++t) v[t] = element<decltype(r)::value>(xr[t]) * __shfl(w, (st * kStep + 8 * sub + t) & 63);
+        };
+        auto columns = [&](auto s, float (&v)[8]) {
+#pragma unroll
+            for (int t = 0; t < 8; ++t) v[t] = element<decltype(s)::value>(br[t]);
+        };
+        if (steps > 0) {
+            load_x(0);
+            load_B(0);
+            load_weights(0);
+        }
+        float w = 0.f;
+        for (int st = 0; st < steps; ++st) {
+            if ((st & 1) == 0) {
+                w = weight(st >> 1);
+                load_weights((st >> 1) + 1);
+            }
+            const int next = min(st + 1, steps - 1);      // behind the last step: that one again, not used
+            bf16x8 xp[A][3];
+            static_for<A>([&](auto r) {
+                float v[8];
+                products(st, w, r, v);
+                split<3>(v, xp[r.value]);
+            });
+            load_x(next);
+            static_for<S>([&](auto s) {
+                float v[8];
+                columns(s, v);
+                bf16x8 bp[kBParts<T>];
+                split<kBParts<T>>(v, bp);
+                if constexpr (s.value == S - 1) load_B(next);
+#pragma unroll
+                for (int q = kBParts<T> - 1; q >= 0; --q)       // the smallest products first; those below 2^-24 of the largest not at all
+#pragma unroll
+                    for (int u = 2 - q; u >= 0; --u)
+#pragma unroll
+                        for (int r = 0; r < A; ++r) acc[r][s.value] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xp[r][u], bp[q], acc[r][s.value], 0, 0, 0);
+            });
+        }
+        // An infinite value, or one that rounds to an infinite bf16, leaves NaN in its rest, and so does one in the place of a token
+        // past the end: where a sum is not finite this wave's tokens are added up once more by the fp32 instructions.
+        bool finite = true;
+#pragma unroll
+        for (int r = 0; r < A; ++r)
+#pragma unroll
+            for (int s = 0; s < S; ++s)
+#pragma unroll
+                for (int q = 0; q < 4; ++q) finite &= __builtin_fabsf(acc[r][s][q]) < __builtin_inff();
+        if (!__all(finite)) {
+#pragma unroll
+            for (int r = 0; r < A; ++r)
+#pragma unroll
+                for (int s = 0; s < S; ++s) acc[r][s] = f32x4{0.f, 0.f, 0.f, 0.f};
+            for (int st = 0; st < steps; ++st) {
+                load_x(st);
+                load_B(st);
+                load_weights(st >> 1);
+                w = weight(st >> 1);
+                static_for<A>([&](auto r) {
+                    float xs[8];
+                    products(st, w, r, xs);
+                    static_for<S>([&](auto s) {
+                        float bs[8];
+                        columns(s, bs);
+#pragma unroll
+                        for (int t = 0; t < 8; ++t)
+                            if (k_begin + st * kStep + 8 * sub + t >= k_end) xs[t] = bs[t] = 0.f;
+#pragma unroll
+                        for (int t = 0; t < 8; ++t)
+                            acc[r.value][s.value] = __builtin_amdgcn_mfma_f32_16x16x4f32(xs[t], bs[t], acc[r.value][s.value], 0, 0, 0);
+                    });
+                });
+            }
+        }
         }
 
         if constexpr (SPLIT == 1) {
@@ -329,12 +479,12 @@ hipError_t launch_generic(const Params &p_in, bool fused, hipStream_t s)
     generic::Shape k{1, 1, generic::kWaves, 0};
     int64_t items = 0;
     const int64_t n_cu = p.n_cu > 0 ? p.n_cu : 256;
-    // One wave per tile where a quarter of a chunk is too little (chunk 64, batch 2 x 1900 tokens x 15 heads x 48 x 96:
-    // 13.5 against 16.6 us; chunk 100: 16.9 against 14.1) and where 64 x 64 tiles alone give every SIMD six waves (fp16,
-    // batch 8 x 3001 x 48 heads x 64 x 128: chunk 256 187 against 198 us, chunk 128 203 against 247; half of it, four and a
-    // half waves: 105 against 101).
+    // One wave per tile where a quarter of a chunk is too little (chunk 64) and where 64 x 64 tiles alone give every SIMD two
+    // waves, all there is room for: quarters / one wave, us: fp32, 3 x 15232 tokens x 8 heads x 64 x 64, chunk 128 (2.8 a SIMD)
+    // 65 / 47; 8 x 520 x 22 x 128 x 128 (2.1) 38 / 31; fp16, 8 x 3001 x 48 (9) 120 / 121; 2 x 3001 x 24 (1.1) 24 / 28;
+    // fp32, 2 x 2048 x 24 (0.75) 18.6 / 22.8.
     const int64_t big_tiles = (int64_t)p.batch * p.nheads * p.C * ((p.headdim + 63) / 64) * ((p.dstate + 63) / 64);
-    if (!fused && (p.Q <= 64 || big_tiles >= 24 * n_cu)) k.split = 1;
+    if (!fused && (p.Q <= 64 || big_tiles >= 8 * n_cu)) k.split = 1;
     // the largest tile (operands loaded once per 16 A x 16 S) that still gives every compute unit four waves
     static const int caps[][2] = {{4, 4}, {4, 2}, {2, 2}};
     for (const auto &cap : caps) {

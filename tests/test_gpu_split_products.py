@@ -1,0 +1,65 @@
+"""Chunk states of fp32, fp16 and odd-sized inputs as products of bf16 parts: the error against 64 bits stays that of fp32
+sums, whatever the magnitudes, at the edges of steps (32 tokens), quarters and tiles; what is not finite goes the fp32 way."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def ops():
+    import ssd_amd
+    from ssd_amd import _lib
+    _lib.load()
+    assert torch.cuda.is_available(), "these tests need the MI355X"
+    return ssd_amd
+
+
+def _exact(x, B, dt, dA, Q):
+    b, L, H, P = x.shape
+    out = []
+    for c in range(-(-L // Q)):
+        t0, t1 = c * Q, min(L, c * Q + Q)
+        w = torch.exp(torch.clamp(dA[:, :, c, -1:].double() - dA[:, :, c, :t1 - t0].double(), max=0.0)) * dt[:, :, c, :t1 - t0].double()
+        xw = (x[:, t0:t1].double().permute(0, 2, 3, 1) * w[:, :, None]).contiguous()
+        out.append(torch.matmul(xw, B[:, t0:t1].double().repeat_interleave(H // B.shape[2], 2).transpose(1, 2).contiguous()))
+    return torch.stack(out, 1)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16], ids=str)
+@pytest.mark.parametrize("L,Q", [(1, 40), (31, 40), (33, 40), (95, 40), (127, 127), (129, 129), (200, 100), (515, 257), (700, 300)])
+@pytest.mark.parametrize("P,N,H", [(20, 24, 2), (65, 17, 3), (64, 96, 40)])
+def test_error_is_that_of_fp32_sums(ops, dtype, L, Q, P, N, H):
+    g = torch.Generator().manual_seed(L + P)
+    C = -(-L // Q)
+    # magnitudes over twelve (f16: six) orders beside each other
+    spread = lambda *s: (torch.randn(s, generator=g) * 10.0 ** (torch.rand(s, generator=g) * (6 if dtype == torch.float16 else 12) - 4)).to(dtype)  # noqa: E731
+    dt, dA = torch.rand(1, H, C, Q, generator=g), -torch.rand(1, H, C, Q, generator=g).cumsum(-1) * 0.05
+    for make in (spread, lambda *s: torch.randn(s, generator=g).to(dtype)):
+        x, B = make(1, L, H, P), make(1, L, 1, N)
+        got = ops._chunk_state_fwd(B.cuda(), x.cuda(), dt.cuda(), dA.cuda())
+        want = _exact(x, B, dt, dA, Q)
+        # weights and products rounded to fp32 (exp's argument included: |dA| up to 7), L sums of them
+        bound = torch.matmul(x.double().abs().permute(0, 2, 3, 1), B.double().abs().transpose(1, 2).contiguous()).amax()
+        err = (got.double().cpu() - want)
+        assert float(err.norm() / want.norm()) < 4e-6 and float(err.abs().amax()) <= 2e-5 * float(bound)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16], ids=str)
+def test_what_is_not_finite_stays_where_it_is(ops, dtype):
+    L, Q, H, P, N = 300, 100, 3, 40, 24
+    g = torch.Generator().manual_seed(3)
+    x, B = torch.randn(1, L, H, P, generator=g).to(dtype), torch.randn(1, L, 1, N, generator=g).to(dtype)
+    dt, dA = torch.rand(1, H, 3, Q, generator=g) + 0.1, -torch.rand(1, H, 3, Q, generator=g).cumsum(-1) * 0.05
+    clean = ops._chunk_state_fwd(B.cuda(), x.cuda(), dt.cuda(), dA.cuda())
+    x[0, 100, 1, 7], x[0, 230, 2, 11] = float("inf"), float("nan")        # the first token of a chunk too: what padding reads
+    B[0, 20, 0, 5] = -float("inf")
+    got = ops._chunk_state_fwd(B.cuda(), x.cuda(), dt.cuda(), dA.cuda())
+    assert bool((got[0, 1, 1, 7].isinf() & (got[0, 1, 1, 7].sign() == B[0, 100, 0].sign().cuda())).all())
+    assert bool(got[0, 2, 2, 11].isnan().all()) and bool(got[0, 0, :, :, 5].isinf().all())
+    got[0, 1, 1, 7], got[0, 2, 2, 11], got[0, 0, :, :, 5] = clean[0, 1, 1, 7], clean[0, 2, 2, 11], clean[0, 0, :, :, 5]
+    torch.testing.assert_close(got, clean, rtol=1e-5, atol=1e-5)
+    if dtype == torch.float32:        # rounds to an infinite bf16, is none
+        x, B = torch.full((1, 1, 1, 2), 3.4e38), torch.full((1, 1, 1, 2), 0.5)
+        one = ops._chunk_state_fwd(B.cuda(), x.cuda(), torch.ones(1, 1, 1, 1, device="cuda"), torch.zeros(1, 1, 1, 1, device="cuda"))
+        torch.testing.assert_close(one.cpu(), torch.full((1, 1, 1, 2, 2), 1.7e38))
