@@ -764,6 +764,10 @@ int ssd_query_fused_wants_states(const ssd_tensor *x, const ssd_tensor *B, const
     // what the call runs with a fp32 `out`, and whether it still does with the place it would be given
     const Choice c = choose(as_out, true, n_cu), given = p.out ? choose(as_states, true, n_cu) : c;
     if (p.out && !c.few && rows_preferred(p, n_cu, true)) return 0;
+    // the scan's state half without passed states on few chunks; planes that are not one row stay with the chain kernel
+    if (!p.out && g_forced_split.load(std::memory_order_relaxed) == 0 && ssd::chain_supported(as_out) &&
+        (!p.init || p.sin_p == p.dstate) && ssd::cost::scan_in_two(problem_of(p, n_cu)))
+        return 1;
     if (c.family == F_PAIR) {
         if (given.family != F_PAIR || (ssd::chain_supported(as_out) && chain_preferred(as_out, n_cu, packed_form(p)))) return 0;
         // Packed rows so long that a fp32 `out` runs the pair whatever the number of units: these calls have the chain

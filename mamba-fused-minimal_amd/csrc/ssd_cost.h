@@ -199,5 +199,24 @@ inline bool few_units_packed(const Problem &q, PackedForm form)
     return chunks / 160.0 + per_cu / 4.6 <= work(q);
 }
 
+// The scan's state half without passed states: the chain kernel multiplies each entering state by its chunk's C rows, one launch
+// that keeps the states on chip but does everything in one instruction stream per SIMD; with room for the states the fused
+// call and the scan's own kernel run one after the other, each on the kernel that suits it.  One launch / two, bf16 y, us:
+//     units x chunks (dstate 128, chunk 256)     8 x 1 (64, 128)   23.0 /  11.1        80 x  8    76.7 /  61.0
+//                                               40 x 2             37.3 /  18.4       160 x  8   107.3 /  95.7
+//                                               20 x 3             38.1 /  18.0        40 x 16    76.9 /  70.4
+//                                              192 x 2             42.0 /  37.5        96 x 16   115.9 / 122.0   (not taken)
+//                                              320 x 3             90.8 /  81.2        80 x 32   198.2 / 229.0   (not taken)
+//                                               40 x 8             52.2 /  40.5       160 x 32   342.7 / 358.8   (not taken)
+//     dstate 64:  48 x 16   64.1 / 55.2     chunk 128:  96 x 8   54.8 / 45.3     four sequences a row:  160 x 8   109.3 / 98.8
+// and level from there on: 320 x 4 105.7 / 107.3, 960 x 1 82.6 / 78.7 (fp32 y: 85.4 / 87.0; elsewhere two are ahead by a little more
+// with it).  The line: up to eight chunks while units or units x chunks stay within what was measured, sixteen up to 48 units; the
+// room is then 84 MB at most for dstate 128.
+inline bool scan_in_two(const Problem &q)
+{
+    if (q.chunks > 8) return q.chunks <= 16 && q.units <= 48;
+    return q.units <= 160 || (q.units <= 320 && q.units * q.chunks <= 960);
+}
+
 }  // namespace cost
 }  // namespace ssd

@@ -63,11 +63,11 @@ def _states_room(x, batch, nchunks, nheads, headdim, dstate):
 
 
 def _room_wanted(sizes, x, B, dt, dA_cumsum, seq_idx, initial_states, out, final_states):
-    """Room for the chunk states of a fused call on these tensors where it gains from that (ssd_query_fused_wants_states;
-    never below four chunks): chunk states + recurrence is then the faster way, and neither a 16-bit nor an absent ``out``
-    is a place for them."""
+    """Room for the chunk states of a fused call on these tensors where it gains from that (ssd_query_fused_wants_states; with an
+    ``out`` never below four chunks): chunk states + recurrence, or the fused call in front of the scan's own kernel, is then
+    the faster way, and neither a 16-bit nor an absent ``out`` is a place for them."""
     batch, _, nheads, headdim, dstate, _, _, nchunks = sizes
-    if nchunks < 4:
+    if nchunks < 4 and out is not None:
         return None
     index = x.device.index
     if index == torch.cuda.current_device():
