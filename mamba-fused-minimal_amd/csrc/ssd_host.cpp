@@ -360,11 +360,13 @@ PyObject *fused_call(PyObject *, PyObject *const *a, Py_ssize_t n)
     return ordinary(n, 10, [&]() -> PyObject * {
         const int64_t most = number(a[7]), device = number(a[8]);
         void *const stream = pointer(a[9]);
+        // The two refusals that ordinary calls meet return: a throw costs 3 us, and more the first time.  Beyond `most`, the general
+        // way's kept workspace may have to grow.
+        const at::Tensor &xv = plain(a[1], 4, device);
+        if (xv.size(0) * xv.size(2) * ((xv.size(3) + 31) / 32) * plain(a[2], 4, device, false).size(2) > most) Py_RETURN_NONE;
         const at::ScalarType out_type = type_of(a[4]);
         const Inputs in = inputs(a[0], a[1], a[2], a[3], a[6], device);
         const ssd_dims &d = in.d;
-        // beyond, the general way's kept workspace may have to grow
-        need((int64_t)d.batch * d.nheads * ((d.headdim + 31) / 32) * d.nchunks <= most);
         ssd_tensor init{};
         if (a[5] != Py_None) {
             const at::Tensor &v = plain(a[5], 4, device);
@@ -376,7 +378,7 @@ PyObject *fused_call(PyObject *, PyObject *const *a, Py_ssize_t n)
         void *const somewhere = (void *)(uintptr_t)4096;
         const int code = out_type == at::kFloat ? SSD_F32 : out_type == at::kBFloat16 ? SSD_BF16 : SSD_F16;
         ssd_tensor out{somewhere, code, 0, {C * H * P * N, H * P * N, P * N, N, 1}}, fin{somewhere, SSD_F32, 0, {H * P * N, P * N, N, 1, 0}};
-        need(ssd_query_fused_is_plain(&in.x, &in.B, &in.dt, &in.dA, &in.seq, &init, &out, &fin, &d) == 1);
+        if (ssd_query_fused_is_plain(&in.x, &in.B, &in.dt, &in.dA, &in.seq, &init, &out, &fin, &d) != 1) Py_RETURN_NONE;
         const at::Tensor out_v = made({d.batch, C, H, P, N}, out_type, *in.xv), fin_v = made({d.batch, H, P, N}, at::kFloat, *in.xv);
         out.data = out_v.data_ptr();
         fin.data = fin_v.data_ptr();

@@ -151,6 +151,11 @@ def _fused_scan_workspace_need(device, sizes, with_out, chunks_per_item):
 # workspace leaves the kept one alone.
 _WORKSPACE_PAIRS = (1 << 16) // 4 - _lib.SSD_WORKSPACE_HEADER_INTS
 
+# Elements of x up to which a fused call is tried as an ordinary one: with more the GPU takes three times as long as the host, and
+# most such calls run on the kernel with a workspace, where the refused attempt cost a first call on new inputs 4 - 8 us
+# (4 x 8192 x 80 heads: 210 us without, 221 with it; 8 x 2048 x 24 heads, 25 M elements, taken: 66 without, 46 with it).
+_ORDINARY_ELEMENTS = 1 << 25
+
 
 def _own_workspace(x, nbytes):
     """-> the _Kept of x's device and current stream, holding at least nbytes (None under stream capture)."""
@@ -315,7 +320,8 @@ def _fused_chunk_state_state_passing_fwd(B, x, dt, dA_cumsum, out_dtype, initial
     ``_workspace`` (an int32 tensor to use instead of the wrapper's own, which it keeps per device and stream and whose
     fill launch it saves from the second call on) with ``_epoch`` (ssd_fused_opts.epoch for that tensor) are test and
     tuning hooks."""
-    if states is None and _clamp is True and _kernel == 0 and _spin_limit == 0 and _workspace is None and _chunks_per_item == 0:
+    if (states is None and _clamp is True and _kernel == 0 and _spin_limit == 0 and _workspace is None and _chunks_per_item == 0 and
+            x.numel() <= _ORDINARY_ELEMENTS):
         wanted = out_dtype if out_dtype is not None else torch.float32 if states_in_fp32 else B.dtype
         done = _ordinary(x, _lib.host().fused_call, B, x, dt, dA_cumsum, wanted, initial_states, seq_idx, _WORKSPACE_PAIRS)
         if done is not None:
