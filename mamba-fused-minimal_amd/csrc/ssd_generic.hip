@@ -482,17 +482,20 @@ hipError_t launch_generic(const Params &p_in, bool fused, hipStream_t s)
     // One wave per tile where a quarter of a chunk is too little (chunk 64) and where 64 x 64 tiles alone give every SIMD two
     // waves, all there is room for: quarters / one wave, us: fp32, 3 x 15232 tokens x 8 heads x 64 x 64, chunk 128 (2.8 a SIMD)
     // 65 / 47; 8 x 520 x 22 x 128 x 128 (2.1) 38 / 31; fp16, 8 x 3001 x 48 (9) 120 / 121; 2 x 3001 x 24 (1.1) 24 / 28;
-    // fp32, 2 x 2048 x 24 (0.75) 18.6 / 22.8.
+    // fp32, 2 x 2048 x 24 (0.75) 18.6 / 22.8.  A quarter of a chunk of 128 is one step of 32 tokens, so there from 2.5 tiles a
+    // compute unit: fp32, 2 x 2048 x 24 (6) 23.3 / 19.6, 5357 x 8 (2.6) 14.9 / 13.9; fp16 22.3 / 18.3, 13.6 / 13.3; bf16, 2 x 3000 x 15 x
+    // 48 x 96 in chunks of 100 (7) 21.7 / 16.7; 5000 x 7 x 48 x 96 (2.2) 10.3 / 11.0; fp32, 5357 x 8 x 64 x 64 (1.3) 10.2 / 13.2.
     const int64_t big_tiles = (int64_t)p.batch * p.nheads * p.C * ((p.headdim + 63) / 64) * ((p.dstate + 63) / 64);
-    if (!fused && (p.Q <= 64 || big_tiles >= 8 * n_cu)) k.split = 1;
-    // the largest tile (operands loaded once per 16 A x 16 S) that still gives every compute unit four waves
+    if (!fused && (p.Q <= 64 || big_tiles >= 8 * n_cu || (p.Q <= 128 && 2 * big_tiles >= 5 * n_cu))) k.split = 1;
+    // the largest tile (operands loaded once per 16 A x 16 S) that still gives every compute unit four waves; with one wave a
+    // tile the largest there is beyond chunks of 64 (5357 x 8 above as 64 x 32: 15.0)
     static const int caps[][2] = {{4, 4}, {4, 2}, {2, 2}};
     for (const auto &cap : caps) {
         k.a = generic::per_lane(p.headdim, cap[0]);
         k.sv = generic::per_lane(p.dstate, cap[1]);
         const int64_t n_pt = (p.headdim + 16 * k.a - 1) / (16 * k.a), n_nt = (p.dstate + 16 * k.sv - 1) / (16 * k.sv);
         items = (int64_t)p.batch * p.nheads * n_pt * n_nt * (fused ? 1 : p.C);
-        if (items * k.split >= n_cu * generic::kWaves) break;
+        if (items * k.split >= n_cu * generic::kWaves || (k.split == 1 && p.Q > 64)) break;
     }
     if (items <= 0) return hipSuccess;
     if (items > 0x7fffffffLL - 64) return hipErrorInvalidValue;

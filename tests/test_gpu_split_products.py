@@ -27,7 +27,7 @@ def _exact(x, B, dt, dA, Q):
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16], ids=str)
-@pytest.mark.parametrize("L,Q", [(1, 40), (31, 40), (33, 40), (95, 40), (127, 127), (129, 129), (200, 100), (515, 257), (700, 300)])
+@pytest.mark.parametrize("L,Q", [(1, 40), (31, 40), (33, 40), (95, 40), (127, 127), (129, 129), (200, 100), (515, 257), (700, 300), (1700, 100)])
 @pytest.mark.parametrize("P,N,H", [(20, 24, 2), (65, 17, 3), (64, 96, 40)])
 def test_error_is_that_of_fp32_sums(ops, dtype, L, Q, P, N, H):
     g = torch.Generator().manual_seed(L + P)
