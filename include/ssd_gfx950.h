@@ -279,7 +279,9 @@ int ssd_query_fused_plan(const ssd_dims *dims, int has_workspace, int compute_un
  * slices per workgroup, 0 where the call runs what ssd_query_fused_plan says, or a negative status.  It takes bf16 x / B with
  * headdim % 16 == 0, dstate 64 or 128, chunk_size % 128 == 0, any number of heads; x rows whose heads lie within the token
  * pitch; fp32 or 16-bit out.  ssd_fused_chunk_state_passing_fwd_ws insists on it with opts->kernel = SSD_KERNEL_ROWS and
- * opts->chunks_per_item = the slices (SSD_ERR_SHAPE where it does not apply; the other calls refuse that value).
+ * opts->chunks_per_item = the slices (SSD_ERR_SHAPE where it does not apply; the other calls refuse that value).  The library
+ * by itself runs it only in place of the other bf16 kernels (headdim % 32 == 0, chunk_size 128 or 256): x times its weight has
+ * 16 bits in all of them and 24 in the kernel for the remaining sizes.
  */
 int ssd_query_fused_rows(const ssd_dims *dims, int has_workspace, int compute_units);
 

@@ -325,9 +325,13 @@ bool chain_preferred(const Params &p, int n_cu, ssd::cost::PackedForm form)
 // Slices per workgroup of the row kernel where a fused call runs on it, else 0.  workspace: the chain kernel is a candidate.
 // Where few units go to chunk states + recurrence the call does so in front of this kernel too (2 x 2048 x 24 heads: 22 us
 // against 21, 1 x 1536 x 24: 15 against 13).
+// Only calls that the other bf16 kernels take as well: headdim 48, chunks of 384 and the like would run here too, but their own
+// kernel (F_GENERIC) carries x * w in 24 bits where this one has 16, and as chunk states + recurrence it fills the chip where a
+// workgroup here walks a whole row (65536 x 4 heads x 48 x 128, chunk 128: 137 us there, 679 here; 131072 x 2 x 64, chunk 384: 114,
+// 1323).
 int rows_preferred(const Params &p, int n_cu, bool workspace)
 {
-    if (g_forced_split.load(std::memory_order_relaxed) != 0 || !ssd::rows_supported(p)) return 0;
+    if (g_forced_split.load(std::memory_order_relaxed) != 0 || !ssd::rows_supported(p) || !ssd::mfma_supported(p)) return 0;
     const ssd::cost::Problem q = problem_of(p, n_cu);
     double us = 0.;
     const int64_t slices = (int64_t)(p.nheads / p.ngroups) * (p.headdim / 16), groups = (int64_t)p.batch * p.ngroups;

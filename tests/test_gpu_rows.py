@@ -67,9 +67,9 @@ def test_rows_kernel(ops, oracle, kw, kr):
 # 128 rows and more to a compute unit, a second round of workgroups, few units, long rows: the other families
 @pytest.mark.parametrize("kw,rows", [
     (dict(b=8, L=2048, H=24), 3), (dict(b=1, L=4096, H=80), 2), (dict(b=4, L=2048, H=80), 5), (dict(b=4, L=8192, H=64), 4),
-    (dict(b=2, L=640, H=30, P=48), 1), (dict(b=1, L=1000, H=50, Q=384), 1), (dict(b=3, L=1100, H=26, P=128, N=64, G=2), 3),
+    (dict(b=3, L=1100, H=26, P=128, N=64, G=2), 3),
     (dict(b=8, L=2048, H=48), 0), (dict(b=4, L=8192, H=80), 0), (dict(b=1, L=2048, H=24), 0), (dict(b=2, L=8192, H=48), 0),
-    (dict(b=1, L=1024, H=80, P=40), 0), (dict(b=1, L=1024, H=80, Q=64), 0),
+    (dict(b=1, L=1024, H=80, P=40), 0), (dict(b=1, L=1024, H=80, Q=64), 0), (dict(b=2, L=640, H=30, P=48), 0), (dict(b=1, L=1000, H=50, Q=384), 0),
 ], ids=lambda v: "-".join(f"{k}{x}" for k, x in v.items()) if isinstance(v, dict) else str(v))
 def test_calls_left_to_the_library(ops, oracle, kw, rows):
     args = dict(P=64, N=128, G=1, Q=256, init=True, nseq=3)
@@ -104,3 +104,33 @@ def test_calls_left_to_the_library(ops, oracle, kw, rows):
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(g_out, o) and torch.equal(g_fin, f)
+
+
+# headdim 48 and 80, chunks of 384, initial states at an odd address: not sizes of the other bf16 kernels, the call stays with
+# the kernel that multiplies in 24 bits
+@pytest.mark.parametrize("kw", [dict(b=2, L=700, H=30, P=48, Q=128), dict(b=1, L=1400, H=40, P=80), dict(b=1, L=1000, H=50, P=64, Q=384),
+                                dict(b=4, L=700, H=48, P=64, odd_init=True)], ids=lambda kw: "-".join(f"{k}{v}" for k, v in kw.items()))
+def test_sizes_off_the_tilings_keep_their_products(ops, kw):
+    args = dict(N=128, Q=256, odd_init=False)
+    args.update(kw)
+    b, L, H, P, N, Q = (args[k] for k in "bLHPNQ")
+    C, g = -(-L // Q), torch.Generator().manual_seed(L)
+    x, B = torch.randn(b, L, H, P, generator=g).to(torch.bfloat16), torch.randn(b, L, 1, N, generator=g).to(torch.bfloat16)
+    dt, dA = torch.rand(b, H, C, Q, generator=g) + 0.5, -torch.rand(b, H, C, Q, generator=g).cumsum(-1) * 2.0 ** -12
+    init = torch.randn(b, H, P, N, generator=g)
+    want, state = [], init.double()
+    for c in range(C):
+        t0, t1 = c * Q, min(L, c * Q + Q)
+        want.append(state)
+        w = torch.exp(dA[:, :, c, -1:].double() - dA[:, :, c, :t1 - t0].double()) * dt[:, :, c, :t1 - t0].double()
+        xw = (x[:, t0:t1].double().permute(0, 2, 3, 1) * w[:, :, None]).contiguous()
+        state = torch.exp(dA[:, :, c, -1].double())[..., None, None] * state + torch.matmul(xw, B[:, t0:t1].double().transpose(1, 2).contiguous())
+    ginit = torch.empty(b * H * P * N + 1, device="cuda")[1:].view(init.shape) if args["odd_init"] else torch.empty(init.shape, device="cuda")
+    ginit.copy_(init)
+    print(f"[rows off tilings] {kw}", flush=True)
+    out, fin = ops._fused_chunk_state_state_passing_fwd(B.cuda(), x.cuda(), dt.cuda(), dA.cuda(), torch.float32, initial_states=ginit)
+    # Sums of up to 384 products one after the other leave sqrt(384 / 2) * 2^-24 / sqrt(3) = 5e-7 of their size, of 32 at a time less;
+    # the weights add 1e-7.  x * w in 16 bits alone is at 2^-18 / sqrt(3) = 2e-6.
+    for got, ref in ((out, torch.stack(want, 1)), (fin, state)):
+        err = float((got.double().cpu() - ref).norm() / ref.norm())
+        assert err < 6e-7, err

@@ -80,3 +80,13 @@ def test_room_is_bounded_and_a_call_does_without_it(monkeypatch):
     monkeypatch.setattr(impl.torch, "empty", lambda *args, **kw: pytest.fail("more than the bound was asked for"))
     limit = impl._STATES_ROOM_BYTES // (4 * 8 * 64 * 128)
     assert impl._states_room(x, 1, limit + 1, 8, 64, 128) is None
+
+
+def test_sizes_off_the_bf16_tilings_are_not_the_row_kernels():
+    # headdim 48 and 80, chunks of 384, initial states at an odd address: the row kernel could, with 16 bits of x * w where their own
+    # kernel has 24, so they keep that one and with a 16-bit out its room for chunk states
+    for b, L, H, P, Q in ((1, 65536, 4, 48, 128), (1, 131072, 16, 80, 128), (1, 131072, 2, 64, 384), (1, 4096, 8, 48, 256), (2, 640, 30, 48, 256)):
+        for workspace in (False, True):
+            assert ops.fused_plan(b, L, H, P, 128, 1, Q, workspace=workspace, compute_units=256)["rows"] == 0
+    assert _wants(L=4096, H=8, P=48) and _wants(L=8192, H=2, Q=384) and _wants(b=2, L=4096, H=16, P=80, Q=128)
+    assert _wants(b=2, L=2048, H=24, init=torch.empty(2 * 24 * 64 * 128 + 1)[1:].view(2, 24, 64, 128))
