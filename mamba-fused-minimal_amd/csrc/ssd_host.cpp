@@ -283,9 +283,19 @@ template <class... N> bool sized(const at::Tensor &v, N... n)
     return true;
 }
 
+// Memory may have to be mapped, or cached blocks flushed, before an output is there: other Python threads go on meanwhile, as
+// they do inside torch.empty.  Where there is none the general way asks again and raises torch.OutOfMemoryError.
 at::Tensor made(at::IntArrayRef sizes, at::ScalarType type, const at::Tensor &like)
 {
-    return at::empty(sizes, like.options().dtype(type).requires_grad(false).memory_format(c10::nullopt));
+    struct Released {
+        PyThreadState *const state = PyEval_SaveThread();
+        ~Released() { PyEval_RestoreThread(state); }
+    } released;
+    try {
+        return at::empty(sizes, like.options().dtype(type).requires_grad(false).memory_format(c10::nullopt));
+    } catch (const c10::OutOfMemoryError &) {
+        throw OutOfTheOrdinary();
+    }
 }
 
 ssd_tensor described(const at::Tensor &v)

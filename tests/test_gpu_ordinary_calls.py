@@ -122,3 +122,18 @@ def test_out_of_the_ordinary(ops, oracle, both):
         graph.replay()
         torch.cuda.synchronize()
         _same(got, want)
+
+
+def test_no_memory_is_torchs_own_error(ops):
+    # outputs of 4 TiB and more over inputs of a few elements: no kernel is launched
+    b, L, H, P, N = 1, 1 << 20, 128, 64, 128
+    one = lambda *shape, dtype=torch.float32: torch.zeros((1,) * (len(shape) - 1) + shape[-1:], dtype=dtype, device="cuda").expand(shape)  # noqa: E731
+    x, B, dt, states = one(b, L, H, P, dtype=torch.bfloat16), one(b, L, 1, N, dtype=torch.bfloat16), one(b, H, L, 1), one(b, L, H, P * N)
+    few = dict(x=one(1, 1 << 16, 8, 64, dtype=torch.bfloat16), B=one(1, 1 << 16, 1, 1 << 26, dtype=torch.bfloat16), dt=one(1, 8, 64, 1 << 10))
+    for call in (lambda: ops._chunk_state_fwd(B, x, dt, dt), lambda: ops._state_passing_fwd(states, one(b, H, L)),
+                 lambda: ops._chunk_cumsum_fwd(one(b, 1 << 30, 1 << 10), one(1 << 10), 256),
+                 lambda: ops._chunk_scan_states_fwd(one(1, 1 << 30, 1, 64), one(1, 1 << 22, 64, 64, 64), one(1, 64, 1 << 22, 256), out_dtype=torch.float32),
+                 lambda: ops._fused_chunk_state_state_passing_fwd(few["B"], few["x"], few["dt"], few["dt"], torch.float32)):
+        with pytest.raises(torch.OutOfMemoryError):
+            call()
+    torch.cuda.empty_cache()
