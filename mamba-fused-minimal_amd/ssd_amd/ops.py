@@ -28,12 +28,13 @@ _raw_stream = torch._C._cuda_getCurrentRawStream
 
 
 def _ordinary(t, call, *args):
-    """call(*args, device, stream) of the extension module: a wrapper's ordinary call in one.  None, and nothing has happened,
-    where anything about it is out of the ordinary (csrc/ssd_host.cpp): the wrapper's general way follows."""
+    """The extension module's function ``call`` (a name: tensors elsewhere need no module) with (*args, device, stream): a
+    wrapper's ordinary call in one.  None, and nothing has happened, where anything about it is out of the ordinary
+    (csrc/ssd_host.cpp): the wrapper's general way follows."""
     if not t.is_cuda:
         return None
     device = torch._C._cuda_getDevice()
-    return call(*args, device, _raw_stream(device))
+    return getattr(_lib.host(), call)(*args, device, _raw_stream(device))
 
 
 def _on_device(t, call, *args):
@@ -240,7 +241,7 @@ def _prep_inputs(B, x, dt, dA_cumsum, seq_idx):
 
 def _chunk_state_fwd(B, x, dt, dA_cumsum, seq_idx=None, states=None, states_in_fp32=True):
     if states is None:
-        done = _ordinary(x, _lib.host().chunk_state_call, B, x, dt, dA_cumsum, seq_idx, 1 if states_in_fp32 else 0)
+        done = _ordinary(x, "chunk_state_call", B, x, dt, dA_cumsum, seq_idx, 1 if states_in_fp32 else 0)
         if done is not None:
             return done
     return _chunk_state_impl(B, x, dt, dA_cumsum, seq_idx, states, states_in_fp32, True)
@@ -271,7 +272,7 @@ def _chunk_state_impl(B, x, dt, dA_cumsum, seq_idx, states, states_in_fp32, _cla
 
 def _state_passing_fwd(states, dA_chunk_cumsum, initial_states=None, seq_idx=None, chunk_size=None,
                        out_dtype=None):
-    done = _ordinary(states, _lib.host().state_passing_call, states, dA_chunk_cumsum, initial_states, seq_idx,
+    done = _ordinary(states, "state_passing_call", states, dA_chunk_cumsum, initial_states, seq_idx,
                      chunk_size if isinstance(chunk_size, int) else 0, out_dtype)
     if done is not None:
         return done
@@ -323,7 +324,7 @@ def _fused_chunk_state_state_passing_fwd(B, x, dt, dA_cumsum, out_dtype, initial
     if (states is None and _clamp is True and _kernel == 0 and _spin_limit == 0 and _workspace is None and _chunks_per_item == 0 and
             x.numel() <= _ORDINARY_ELEMENTS):
         wanted = out_dtype if out_dtype is not None else torch.float32 if states_in_fp32 else B.dtype
-        done = _ordinary(x, _lib.host().fused_call, B, x, dt, dA_cumsum, wanted, initial_states, seq_idx, _WORKSPACE_PAIRS)
+        done = _ordinary(x, "fused_call", B, x, dt, dA_cumsum, wanted, initial_states, seq_idx, _WORKSPACE_PAIRS)
         if done is not None:
             return done
     batch, seqlen, nheads, headdim = x.shape
@@ -456,7 +457,7 @@ def _chunk_cumsum_fwd(dt, A, chunk_size, dt_bias=None, dt_softplus=False, dt_lim
     """dt preparation + per-chunk cumulative sum of dt * A; same call surface as the reference's
     kernels/ssd_chunk_state.py:176-199.  dt (batch, seqlen, nheads) -> (dA_cumsum, dt_out), both
     (batch, nheads, nchunks, chunk_size) fp32."""
-    done = _ordinary(dt, _lib.host().chunk_cumsum_call, dt, A, dt_bias, chunk_size, int(bool(dt_softplus)), float(dt_limit[0]), float(dt_limit[1]))
+    done = _ordinary(dt, "chunk_cumsum_call", dt, A, dt_bias, chunk_size, int(bool(dt_softplus)), float(dt_limit[0]), float(dt_limit[1]))
     if done is not None:
         return done
     batch, seqlen, nheads = dt.shape
@@ -556,7 +557,7 @@ def _chunk_scan_states_fwd(C, prev_states, dA_cumsum, seq_idx=None, out=None, ou
     ``out_dtype`` (default: C's, as the reference's ``out`` takes x's); with ``out=`` the result goes there, and with
     ``accumulate=True`` it is added to what ``out`` holds (the intra-chunk half of the scan)."""
     if out is None and not accumulate:
-        done = _ordinary(C, _lib.host().scan_states_call, C, prev_states, dA_cumsum, seq_idx, out_dtype)
+        done = _ordinary(C, "scan_states_call", C, prev_states, dA_cumsum, seq_idx, out_dtype)
         if done is not None:
             return done
     batch, seqlen, ngroups, dstate = C.shape

@@ -338,3 +338,25 @@ def test_workspace_status_decoding():
     assert st(h) == 0
     for code in (-7, -8, -9, -10):
         assert lib.ssd_status_string(code).decode() not in ("unknown status", "")
+
+
+def test_arguments_are_checked_without_the_extension_module(monkeypatch):
+    # tensors that are not on a GPU: the wrappers' own errors, also where nothing is built
+    import ssd_amd as ops
+    from ssd_amd import _lib
+
+    def missing():
+        raise ImportError("not built")
+    monkeypatch.setattr(_lib, "host", missing)
+    x, B, dt = torch.zeros(1, 256, 2, 64), torch.zeros(1, 256, 1, 128), torch.zeros(1, 2, 1, 256)
+    states = torch.zeros(1, 1, 2, 64, 128)
+    for wrong, right in ((lambda: ops._chunk_state_fwd(B[:, :-1], x, dt, dt), lambda: ops._chunk_state_fwd(B, x, dt, dt)),
+                         (lambda: ops._state_passing_fwd(states.flatten(-2), dt[:, :1, :, 0]), lambda: ops._state_passing_fwd(states.flatten(-2), dt[..., 0])),
+                         (lambda: ops._fused_chunk_state_state_passing_fwd_concurrent(B, x, dt, dt[..., :-1], None),
+                          lambda: ops._fused_chunk_state_state_passing_fwd_concurrent(B, x, dt, dt, None)),
+                         (lambda: ops._chunk_cumsum_fwd(x[..., 0], torch.zeros(3), 256), lambda: ops._chunk_cumsum_fwd(x[..., 0], torch.zeros(2), 256)),
+                         (lambda: ops._chunk_scan_states_fwd(B[..., :-1], states, dt), lambda: ops._chunk_scan_states_fwd(B, states, dt))):
+        with pytest.raises(AssertionError):
+            wrong()
+        with pytest.raises(RuntimeError, match="must live on a gfx950"):
+            right()
