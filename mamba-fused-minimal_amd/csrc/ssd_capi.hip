@@ -342,11 +342,13 @@ int rows_preferred(const Params &p, int n_cu, bool workspace)
         if (!p.seq || ssd::cost::few_units_packed(q, packed_form(p))) return 0;
         c = choose(p, true, q.n_cu, false);
     }
+    us /= ssd::cost::rows_margin(q, kr);
     if (us >= estimate_us(q, c)) return 0;
     if (workspace && ssd::chain_supported(p)) {
         double chain = 0.;
         ssd::cost::chain_chunks_per_item(q, &chain);
         if (us >= chain) return 0;
+        if (p.seq && !ssd::cost::rows_packed(q, kr, p.dt_out == ssd::DT_F32) && chain_preferred(p, n_cu, packed_form(p))) return 0;
     }
     return kr;
 }

@@ -120,9 +120,10 @@ inline double rows_us(const Problem &q, int kr)
 // Slices per workgroup of the row kernel, 0 where it is no candidate.  slices: 16-row slices of a (batch, group); groups:
 // (batch, group) pairs.  There is a workgroup per compute unit at most: a second round of workgroups costs as much as the
 // first (8 x 2048 x 48 heads: 66 us, the others 57).  A workgroup reads the same few columns of x to the end, so long rows
-// depend on how those columns fall on the memory channels, and a third of the workgroups finish up to a fifth late: up to 5120
-// tokens the kernel is ahead wherever its estimate is, beyond that only with four slices at dstate 128 or with chunks of
-// 128.  Inputs from memory, the faster of the others against this kernel, us (slices):
+// depend on how those columns fall on the memory channels, and a third of the workgroups finish up to a fifth late.  Up to 5120
+// tokens the kernel is ahead wherever its estimate is (rows_margin), beyond that only with four slices at dstate 128 or with chunks
+// of 128, and there in groups of 16 slices and more: below, too few workgroups share a group's B (12 x 10730).  Inputs from memory, the faster of the others
+// against this kernel, us (slices):
 //     8 x 2048 x 24 heads       48.4 /  35.9 (3)      4 x 8192 x 64                   143.5 / 132.7 (4)
 //     2 x 2048 x 80             49.0 /  34.9 (3)      4 x 8192 x 80                   175.7 / 177.1 (5)   (not taken)
 //     1 x 4096 x 80             53.9 /  46.3 (2)      1 x 8192 x 80                    70.9 /  85.9 (2)   (not taken)
@@ -130,17 +131,43 @@ inline double rows_us(const Problem &q, int kr)
 //     4 x 2048 x 80             56.3 /  48.5 (5)      4 x 8192 x 80, chunk 128        249.2 / 228.5 (5)
 //     8 x 2048 x 24, chunk 128  64.9 /  42.7 (3)      4 x 8192 x 80, dstate 64        130.2 / 137.0 (5)   (not taken)
 //     8 x 2048 x 24, dstate 64  34.7 /  28.9 (3)      8 x 3729 x 24, 8 groups, dstate 64, chunk 128   75.7 / 54.7 (3)
+//     2 x 4608 x 52             53.8 /  47.4 (2)      12 x 10730 x 32 x 32, 8 groups, chunk 128      238.8 / 248.0 (4)   (not taken)
+//     1 x 5120 x 64             52.5 /  43.0 (1)      1 x 5120 x 80                    53.1 /  56.2 (2)   (not taken)
 inline int rows_slices(const Problem &q, int64_t slices, int64_t groups, int most, double *us)
 {
     int best = 0;
-    const bool long_rows = (int64_t)q.chunks * q.chunk_size > 5120;
-    for (int kr = 1; kr <= most; ++kr) {
+    const int64_t tokens = (int64_t)q.chunks * q.chunk_size;
+    for (int kr = 1; kr <= most && kr <= slices; ++kr) {
         if (groups * ceil_div(slices, kr) > q.n_cu) continue;
-        if (long_rows && !(kr >= 4 && (q.chunk_size == 128 || (kr == 4 && q.dstate == 128)))) continue;
+        if (tokens > 5120 && !(slices >= 16 && kr >= 4 && (q.chunk_size == 128 || (kr == 4 && q.dstate == 128)))) continue;
         const double t = rows_us(q, kr);
         if (!best || t < *us) { best = kr; *us = t; }
     }
     return best;
+}
+
+// How far below the other families' the row kernel's estimate has to be.  With dstate 64 and few chunks theirs are up to a fifth
+// too high, and four and five slices pay their start (other family / row kernel, us: 4 x 512 x 51 heads, chunk 128, 12.8 / 14.1;
+// 1338 x 113 x 128 22.6 / 23.6; 3 x 486 x 66, 2 groups, chunk 128, 12.9 / 13.3); two slices of long rows take longer than their
+// estimate (1 x 5120 x 80, 0.90 of the chain kernel's, 53.1 / 56.2; 1 x 5120 x 128, 0.84, 66.7 / 55.9).
+inline double rows_margin(const Problem &q, int kr)
+{
+    if (q.dstate == 64) return q.chunks <= 6 && kr >= 4 ? 0.9 : 1.0;
+    return kr == 2 && q.chunk_size > 128 && (int64_t)q.chunks * q.chunk_size > 4608 ? 0.88 : 1.0;
+}
+
+// Packed sequences (seq_idx) where the chain kernel would have the call: the estimate knows nothing of its chains being cut, so
+// with a sequence start in every chunk it is ahead of narrow workgroups, which walk the whole row all the same.  Chain / row
+// kernel (slices), us, a start in every chunk:
+//     1 x 5120 x 64, fp32 out    37.3 / 44.1 (1)      8 x 4352 x 10, bf16 out         38.7 /  41.9 (2)      (neither taken)
+//     2 x 3840 x 28, 2 groups    24.5 / 34.3 (1)      6 x 4608 x 12 x 128             56.2 /  66.3 (3)      (neither taken)
+//     12 x 3340 x 12 x 32, dstate 64, chunk 128   27.0 / 30.7 (2)      4 x 4096 x 48     58.1 /  62.7 (3)      (neither taken)
+//     6 x 2560 x 28              53.4 / 40.0 (3)      12 x 2329 x 12, 2 groups        41.4 /  39.4 (3)
+//     4 x 4608 x 44, chunk 128   91.2 / 86.3 (3)      8 x 4449 x 22, bf16 out         69.0 /  62.0 (3)
+//     4 x 8192 x 64             134.2 / 129.6 (4)     12 x 3307 x 16, 2 groups, chunk 128   78.9 / 63.0 (4)
+inline bool rows_packed(const Problem &q, int kr, bool out_f32)
+{
+    return kr >= 4 || (kr == 3 && (q.chunk_size == 128 || !out_f32 || (int64_t)q.chunks * q.chunk_size <= 3072));
 }
 
 // Few units: the pair, whatever the estimates say (they are fits to 24 and more heads and know the recurrence as a pure

@@ -100,11 +100,13 @@ def test_estimates_are_within_a_quarter_of_the_measurement_where_a_family_is_pic
 
 def test_the_benchmark_configurations_keep_their_kernels():
     # b=4 L=8192 H=80, the packed b=1 L=32768 H=80 and the grouped b=1 L=131072 H=128: chain kernel, four chunks per item;
-    # b=8 L=2048 H=24: token-split
+    # b=8 L=2048 H=24: the row kernel with three slices, where that does not go token-split
     for b, L, H, G in ((4, 8192, 80, 1), (1, 32768, 80, 1), (1, 131072, 128, 8)):
         plan = ops.fused_plan(b, L, H, 64, 128, G, 256)
         assert (plan["family"], plan["chunks_per_item"]) == ("chain", 4), plan
-    assert ops.fused_plan(8, 2048, 24, 64, 128, 1, 256)["family"] == "token_split"
+        assert plan["rows"] == 0
+    plan = ops.fused_plan(8, 2048, 24, 64, 128, 1, 256)
+    assert (plan["rows"], plan["family"]) == (3, "token_split")
 
 
 def test_without_a_workspace_the_chain_kernel_is_never_planned():
@@ -126,3 +128,84 @@ def test_sizes_the_fast_kernels_do_not_cover_fall_to_the_generic_family():
     assert plan["family"] == "generic" and plan["estimate_us"]["chain"] is None
     with pytest.raises(Exception):
         ops.fused_plan(1, 1024, 7, 64, 128, 2, 256)          # nheads % ngroups
+
+
+# The row kernel against what the call ran before it: batch, seqlen, nheads, headdim, dstate, ngroups, chunk, bits of out, a sequence
+# start in every chunk, microseconds without it, with it (inputs from memory, random shapes: where it lost, and some where it did not).
+ROWS = [
+    (1, 513, 34, 32, 128, 2, 256, 16, 0, 12.4, 8.9), (1, 619, 30, 128, 128, 1, 256, 32, 1, 12.4, 9.9),
+    (1, 757, 11, 64, 128, 1, 256, 16, 0, 12.3, 8.9), (1, 1338, 113, 128, 64, 1, 256, 16, 0, 22.6, 23.6),
+    (1, 2048, 80, 64, 128, 1, 256, 32, 1, 29.3, 26.0), (1, 2560, 96, 64, 128, 1, 256, 16, 1, 33.6, 29.7),
+    (1, 3189, 48, 128, 64, 1, 128, 32, 0, 45.1, 35.4), (1, 3891, 88, 128, 128, 8, 128, 32, 0, 85.4, 70.2),
+    (1, 4267, 43, 128, 128, 1, 256, 32, 1, 39.3, 43.5), (1, 5120, 64, 64, 128, 1, 256, 32, 1, 37.3, 44.1),
+    (1, 5120, 80, 64, 128, 1, 256, 32, 0, 53.1, 56.2), (1, 5120, 80, 64, 128, 1, 256, 32, 1, 38.8, 56.2),
+    (1, 5120, 128, 64, 128, 1, 256, 32, 1, 68.2, 55.6), (2, 565, 128, 64, 128, 8, 256, 16, 1, 24.8, 18.9),
+    (2, 1536, 32, 64, 128, 2, 256, 32, 1, 22.4, 17.2), (2, 1536, 37, 128, 128, 1, 256, 32, 1, 33.5, 26.5),
+    (2, 1792, 48, 64, 128, 8, 256, 32, 0, 26.0, 23.6), (2, 3072, 64, 32, 128, 8, 128, 16, 1, 30.2, 31.8),
+    (2, 3840, 28, 64, 128, 2, 256, 32, 1, 24.5, 34.3), (2, 4096, 80, 64, 128, 1, 256, 32, 1, 55.8, 61.3),
+    (2, 4608, 52, 64, 128, 1, 256, 32, 1, 40.8, 47.5), (3, 486, 66, 64, 64, 2, 128, 16, 0, 12.9, 13.3),
+    (3, 1536, 42, 32, 128, 2, 256, 32, 1, 21.6, 17.0), (3, 3072, 12, 128, 64, 1, 128, 32, 1, 26.5, 28.0),
+    (3, 3072, 14, 128, 128, 1, 128, 16, 1, 31.5, 33.4), (3, 3840, 18, 64, 128, 1, 256, 32, 1, 24.4, 33.2),
+    (3, 3873, 84, 64, 128, 1, 128, 32, 1, 107.2, 85.0), (3, 4608, 15, 128, 128, 1, 256, 16, 1, 39.0, 42.5),
+    (3, 5011, 12, 128, 128, 1, 256, 32, 1, 39.4, 49.0), (4, 512, 51, 64, 64, 1, 128, 32, 0, 12.8, 14.1),
+    (4, 512, 51, 64, 64, 1, 128, 32, 1, 13.1, 14.2), (4, 768, 6, 32, 128, 1, 256, 32, 0, 12.0, 8.8),
+    (4, 2216, 16, 64, 128, 8, 256, 32, 1, 32.0, 25.1), (4, 3328, 72, 32, 64, 1, 256, 32, 1, 35.7, 37.6),
+    (4, 4096, 48, 64, 128, 1, 256, 32, 1, 58.1, 62.7), (4, 5888, 94, 32, 128, 2, 256, 16, 0, 100.8, 111.3),
+    (4, 5888, 94, 32, 128, 2, 256, 16, 1, 101.6, 114.3), (4, 8817, 48, 64, 128, 8, 128, 16, 1, 172.1, 148.5),
+    (6, 512, 8, 128, 64, 8, 128, 32, 1, 12.3, 10.6), (6, 768, 18, 32, 128, 1, 128, 16, 1, 16.7, 11.2),
+    (6, 1280, 24, 64, 128, 8, 256, 32, 0, 30.3, 24.6), (6, 2304, 11, 128, 64, 1, 128, 32, 1, 36.1, 30.1),
+    (6, 2304, 16, 64, 64, 8, 128, 32, 1, 35.9, 27.0), (6, 2324, 7, 128, 128, 1, 128, 32, 1, 30.5, 32.2),
+    (6, 2574, 10, 64, 128, 1, 256, 32, 1, 35.9, 26.6), (6, 4427, 7, 128, 128, 1, 256, 16, 1, 38.9, 42.5),
+    (6, 4608, 12, 128, 128, 1, 256, 32, 1, 56.2, 66.3), (6, 4864, 14, 64, 64, 2, 256, 16, 1, 39.7, 35.9),
+    (6, 18176, 24, 64, 128, 8, 256, 16, 0, 314.6, 340.3), (6, 18176, 24, 64, 128, 8, 256, 16, 1, 320.3, 345.6),
+    (8, 1280, 16, 128, 128, 8, 256, 16, 0, 42.5, 26.2), (8, 2048, 24, 64, 128, 1, 256, 32, 1, 48.9, 35.3),
+    (8, 4352, 10, 64, 128, 1, 256, 16, 1, 38.7, 41.9), (8, 4411, 13, 128, 64, 1, 256, 32, 1, 63.9, 55.8),
+    (12, 1280, 5, 64, 64, 1, 256, 32, 1, 13.9, 12.1), (12, 1790, 22, 64, 128, 1, 256, 16, 0, 44.0, 36.6),
+    (12, 2816, 6, 64, 128, 1, 128, 16, 1, 30.7, 31.7), (12, 3307, 16, 64, 128, 2, 128, 32, 0, 80.5, 62.6),
+    (12, 3307, 16, 64, 128, 2, 128, 32, 1, 78.9, 63.0), (12, 3340, 12, 32, 64, 1, 128, 32, 1, 27.0, 30.7),
+    (12, 4352, 4, 64, 64, 1, 128, 32, 0, 38.3, 32.1), (12, 4352, 4, 64, 64, 1, 128, 32, 1, 26.0, 32.6),
+    (12, 4660, 4, 64, 64, 1, 128, 32, 1, 27.5, 36.8), (12, 10730, 32, 32, 128, 8, 128, 32, 0, 238.8, 248.0),
+    (12, 10730, 32, 32, 128, 8, 128, 32, 1, 225.5, 248.1), (16, 2816, 8, 64, 128, 1, 256, 16, 0, 36.3, 31.6),
+    (16, 4096, 5, 64, 128, 1, 256, 32, 0, 52.0, 43.1), (16, 4570, 7, 128, 128, 1, 256, 16, 1, 77.1, 62.1),
+    (16, 6411, 9, 64, 128, 1, 128, 32, 1, 180.0, 119.5),
+]
+
+
+def _tensor(shape, code):
+    """A contiguous tensor of that shape at an aligned address that nobody reads."""
+    from ssd_amd import _lib
+    t = _lib.SsdTensor(data=4096, dtype=code)
+    step = 1
+    for i in reversed(range(len(shape))):
+        t.stride[i] = step
+        step *= shape[i]
+    return t
+
+
+def _runs_rows(b, L, H, P, N, G, Q, bits, packed):
+    """Whether the fused call on such tensors, with a workspace, runs the row kernel."""
+    from ssd_amd import _lib
+    if not ops.fused_plan(b, L, H, P, N, G, Q, compute_units=256)["rows"]:
+        return False
+    C, none = -(-L // Q), _lib.tensor_arg(None)
+    bf, f32 = _lib.SSD_BF16, _lib.SSD_F32
+    plain = _lib.load().ssd_query_fused_is_plain(
+        _tensor((b, L, H, P), bf), _tensor((b, L, G, N), bf), _tensor((b, H, C, Q), f32), _tensor((b, H, C, Q), f32),
+        _tensor((b, L), 0) if packed else none, none, _tensor((b, C, H, P, N), f32 if bits == 32 else bf), _tensor((b, H, P, N), f32),
+        _lib.dims_arg(b, L, H, P, N, G, Q, C))
+    return plain == 1
+
+
+def test_the_row_kernel_is_not_taken_where_it_lost():
+    taken = [row for row in ROWS if _runs_rows(*row[:9])]
+    for row in taken:
+        assert row[10] <= 1.03 * row[9], row
+    ahead = [row for row in ROWS if row[9] > 1.08 * row[10]]
+    assert len([row for row in ahead if row in taken]) >= 0.9 * len(ahead)
+
+
+def test_the_row_kernel_on_long_rows_needs_slices_enough():
+    # groups of two slices, whose workgroups would be half empty, and of eight
+    for args in ((4, 16384, 32, 32, 128, 32, 256), (2, 32768, 64, 32, 128, 64, 256), (12, 10730, 32, 32, 128, 8, 128)):
+        for workspace in (False, True):
+            assert ops.fused_plan(*args, workspace=workspace, compute_units=256)["rows"] == 0
