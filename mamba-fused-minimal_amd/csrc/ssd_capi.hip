@@ -190,26 +190,25 @@ Choice choose(const Params &p, bool fused, int64_t n_cu, bool few = true)
     }
     // Groups whose tiles are no multiple of four: neither the four-tile nor the chain kernel takes the call, and a walk of one
     // workgroup per tile (token-split) is what is left.  With room for the chunk states the pair goes in front of it from four
-    // chunks on where its estimate is a tenth lower.
+    // chunks on where its estimate is a tenth lower, and nowhere else: the rules below it were drawn for full workgroups.
     const int in_group = (p.nheads / p.ngroups) * (p.headdim / 32);
-    if (fused && forced == 0 && in_group % 4 && p.C >= 4) {
-        const ssd::cost::Problem q = problem_of(p, n_cu);
-        if (ssd::cost::ragged_pair_us(q) < 0.9 * ssd::cost::token_split_us(q) &&
-            (p.states ? pair_supported(p) : p.dt_out == ssd::DT_F32 && pair_supported(with_states_in_out(p))))
-            return {F_PAIR, !p.states, false, false};
-    }
+    const bool ragged = in_group % 4 != 0;
+    if (fused && forced == 0 && ragged && p.C >= 4 && ssd::mfma_supported(p) && ssd::cost::ragged_pair_ahead(problem_of(p, n_cu)) &&
+        (p.states ? pair_supported(p) : p.dt_out == ssd::DT_F32 && pair_supported(with_states_in_out(p))))
+        return {F_PAIR, !p.states, false, false};
     // Few state tiles, many chunks, fp32 `out`: the chunk-state launch keeps every compute unit busy where the
     // fused kernels have one workgroup per tile.  It writes the chunk states into `out`, and the streaming
     // recurrence turns them into the passed states in place (b=1 L=32768 H=80: 330 us against 425 us).
-    if (fused && !p.states && forced == 0 && tiles < 2 * n_cu && (int64_t)tiles * p.C >= 32 * n_cu &&
+    if (fused && !p.states && forced == 0 && !ragged && tiles < 2 * n_cu && (int64_t)tiles * p.C >= 32 * n_cu &&
         p.dt_out == ssd::DT_F32 && pair_supported(with_states_in_out(p)))
         return {F_PAIR, true, false, false};
     // The caller wants the per-chunk states as well: the chunk-state launch of the four-tile kernel, which keeps
     // every compute unit busy whatever the number of tiles, then the streaming recurrence over what it wrote
     // (b=1 L=32768 H=80: 336 us against 496 us for the token-split kernel doing both at once).
-    if (fused && p.states && (forced == 1 || (forced == 0 && (int64_t)tiles * p.C >= 32 * n_cu)) && pair_supported(p))
+    if (fused && p.states && (forced == 1 || (forced == 0 && !ragged && (int64_t)tiles * p.C >= 32 * n_cu)) && pair_supported(p))
         return {F_PAIR, false, false, false};
-    if (!fused && (forced == 1 || (forced == 0 && (int64_t)tiles * p.C >= 8 * n_cu)) && ssd::quad_chunk_state_supported(p))
+    if (!fused && (forced == 1 || (forced == 0 && (int64_t)tiles * p.C >= 8 * n_cu && ssd::cost::quads_filled(in_group, p.dstate, p.Q))) &&
+        ssd::quad_chunk_state_supported(p))
         return {F_FOUR_TILE, false, false, false};
     if (ssd::mfma_supported(p)) return {F_TOKEN_SPLIT, false, false, false};
     if (fused && forced == 0 && !p.states && p.dt_out == ssd::DT_F32 && generic_pair_supported(with_states_in_out(p)))

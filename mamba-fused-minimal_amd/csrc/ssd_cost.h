@@ -108,6 +108,27 @@ inline double ragged_pair_us(const Problem &q)
     return 6.0 + (states > bytes ? states : bytes) + 2.0 * s_bytes / 5.0e6 * (256.0 / q.n_cu);
 }
 
+// ... against the walk of one workgroup per tile, whose chunks take a third longer in rows of more than 32.  On 110 random shapes
+// the pair was ahead wherever its estimate is a tenth lower, by 1.3 to 3.4 times; between that and the other side of the line it
+// lost up to a third.  Walk / pair, us (tiles of a group): 4 x 8448 tokens x 30 heads x 32 in 2 groups (15) 97.9 / 58.3;
+// 8 x 22528 x 8 x 64 in 8 groups (2) 288 / 216; 2 x 20480 x 40 in 8 groups (10) 259 / 187; on the other side 8 x 31195 x 16 x 32 in 16 groups (1),
+// bf16 out, 387 / 390; 8 x 8923 x 28 in 4 groups (14), dstate 64, bf16 out, 122 / 144.
+inline bool ragged_pair_ahead(const Problem &q)
+{
+    return ragged_pair_us(q) < 0.9 * token_split_us(q) * (q.chunks > 32 ? 4.0 / 3.0 : 1.0);
+}
+
+// Chunk states: whether workgroups of four tiles, the last of each group partly filled, are ahead of one workgroup per tile.  A wave
+// without a tile of its own multiplies all the same, so four fifths of them have to have one, and at dstate 64 with chunks of 128 a
+// workgroup's start is too much for what it does.  One per tile / four-tile, us (tiles of a group, dstate, chunk): 7, 128, 256 22.9 / 18.8;
+// 13 22.5 / 18.7; 50, 128, 128 116 / 97; 6 23.0 / 23.4; 9 161 / 163; 3 183 / 193; 2 57.7 / 66.7; 1 84 / 104; 7, 64, 256 33.6 / 29.7;
+// 9 110 / 122; 7, 64, 128 10.1 / 11.1; 50 20.2 / 23.5; 1 27 / 48.
+inline bool quads_filled(int64_t tiles, int dstate, int chunk_size)
+{
+    if (tiles % 4 == 0) return true;
+    return 5 * tiles >= 16 * ceil_div(tiles, 4) && (dstate > 64 || chunk_size > 128);
+}
+
 // Row kernel (ssd_rows.hip): workgroups of kr slices of 16 state rows, one per compute unit, each walking its whole sequence.
 // Per chunk and relative to dstate 128, chunk 256 (measured 0.61 at chunk 128, 0.75 at dstate 64, 0.45 at both):
 inline double rows_us(const Problem &q, int kr)

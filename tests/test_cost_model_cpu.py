@@ -209,3 +209,21 @@ def test_the_row_kernel_on_long_rows_needs_slices_enough():
     for args in ((4, 16384, 32, 32, 128, 32, 256), (2, 32768, 64, 32, 128, 64, 256), (12, 10730, 32, 32, 128, 8, 128)):
         for workspace in (False, True):
             assert ops.fused_plan(*args, workspace=workspace, compute_units=256)["rows"] == 0
+
+
+# Groups whose tiles are no multiple of four, the walk of one workgroup per tile against chunk states + recurrence, measured in turn
+# (fp32 or 16-bit out):
+# batch, seqlen, nheads, headdim, dstate, ngroups, chunk, walk, pair
+RAGGED = [
+    (8, 16384, 8, 64, 128, 8, 256, 211.9, 156.9), (8, 22528, 8, 64, 128, 8, 256, 288.4, 216.2), (4, 8448, 30, 32, 128, 2, 256, 97.9, 58.3),
+    (1, 36315, 56, 32, 128, 4, 256, 378.8, 111.8), (2, 20480, 40, 64, 128, 8, 256, 258.5, 186.5), (16, 13696, 4, 32, 128, 4, 128, 236.4, 118.1),
+    (4, 16384, 32, 32, 128, 32, 256, 206.4, 233.1), (2, 32768, 64, 32, 128, 64, 256, 402.2, 459.4), (8, 31195, 16, 32, 128, 16, 256, 386.7, 390.3),
+    (6, 18176, 24, 64, 128, 8, 256, 314.6, 340.3), (4, 5888, 94, 32, 128, 2, 256, 100.8, 111.3), (8, 8923, 28, 64, 64, 4, 256, 122.3, 144.1),
+    (8, 19419, 32, 32, 64, 16, 128, 267.3, 325.2), (8, 1664, 84, 32, 128, 4, 128, 80.8, 100.2), (4, 1627, 176, 32, 64, 16, 128, 54.0, 64.9),
+]
+
+
+def test_groups_off_the_four_tiles_take_the_pair_where_it_is_ahead():
+    for *args, walk, pair in RAGGED:
+        plan = ops.fused_plan(*args, workspace=False, compute_units=256)
+        assert plan["family"] == ("pair" if pair < 0.8 * walk else "token_split"), (args, plan)

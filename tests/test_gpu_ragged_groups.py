@@ -58,7 +58,10 @@ def test_ragged_groups(ops, oracle, kw):
 
 # 36 chunks of 25 heads and more: the pair; below the row kernel or the walk
 @pytest.mark.parametrize("kw,family", [(dict(b=2, L=9216, H=25), "pair"), (dict(b=3, L=5200, H=9, G=3, Q=128, nseq=4), "pair"),
-                                       (dict(b=8, L=700, H=33), "token_split")])
+                                       (dict(b=8, L=700, H=33), "token_split"),
+                                       # groups of one, two and three tiles, with chunk states enough to fill the chip
+                                       (dict(b=8, L=9000, H=8, P=32, G=8), "pair"), (dict(b=4, L=9000, H=8, G=8), "pair"),
+                                       (dict(b=8, L=2500, H=8, P=96, G=8, N=64, Q=128, nseq=3), "token_split")])
 def test_calls_left_to_the_library(ops, oracle, kw, family):
     args = dict(P=64, N=128, G=1, Q=256, init=True, nseq=0)
     args.update(kw)
@@ -69,6 +72,12 @@ def test_calls_left_to_the_library(ops, oracle, kw, family):
     x, B, dt, dA, init, seq = (mv(d[k]) for k in ("x", "B", "dt", "dA_cumsum", "initial_states", "seq_idx"))
     print(f"[ragged auto] {kw}", flush=True)
     want_out, want_fin = oracle.fused_ref(d["B"], d["x"], d["dt"], d["dA_cumsum"], initial_states=d["initial_states"], seq_idx=d["seq_idx"])
+    states = ops._chunk_state_fwd(B, x, dt, dA, seq_idx=seq)
+    torch.testing.assert_close(states.cpu(), oracle.chunk_state_ref(d["B"], d["x"], d["dt"], d["dA_cumsum"], seq_idx=d["seq_idx"]), rtol=2e-3, atol=1e-3)
+    given = torch.empty_like(states)
+    out, fin = ops._fused_chunk_state_state_passing_fwd(B, x, dt, dA, torch.float32, initial_states=init, seq_idx=seq, states=given)
+    torch.testing.assert_close(given, states, rtol=2e-3, atol=1e-3)
+    torch.testing.assert_close(out.cpu(), want_out, rtol=2e-3, atol=1e-3)
     for dtype in (torch.float32, torch.bfloat16):
         out, fin = ops._fused_chunk_state_state_passing_fwd(B, x, dt, dA, dtype, initial_states=init, seq_idx=seq)
         torch.testing.assert_close(out.float().cpu(), want_out, rtol=2e-3 if dtype == torch.float32 else 2.0 ** -7, atol=1e-3)
