@@ -771,7 +771,7 @@ int ssd_query_fused_wants_states(const ssd_tensor *x, const ssd_tensor *B, const
     if (p.out && !c.few && rows_preferred(p, n_cu, true)) return 0;
     // the scan's state half without passed states on few chunks; planes that are not one row stay with the chain kernel
     if (!p.out && g_forced_split.load(std::memory_order_relaxed) == 0 && ssd::chain_supported(as_out) &&
-        (!p.init || p.sin_p == p.dstate) && ssd::cost::scan_in_two(problem_of(p, n_cu)))
+        (!p.init || p.sin_p == p.dstate) && ssd::cost::scan_in_two(problem_of(p, n_cu), p.seq != nullptr))
         return 1;
     if (c.family == F_PAIR) {
         if (given.family != F_PAIR || (ssd::chain_supported(as_out) && chain_preferred(as_out, n_cu, packed_form(p)))) return 0;

@@ -260,8 +260,13 @@ inline bool few_units_packed(const Problem &q, PackedForm form)
 // and level from there on: 320 x 4 105.7 / 107.3, 960 x 1 82.6 / 78.7 (fp32 y: 85.4 / 87.0; elsewhere two are ahead by a little more
 // with it).  The line: up to eight chunks while units or units x chunks stay within what was measured, sixteen up to 48 units; the
 // room is then 84 MB at most for dstate 128.
-inline bool scan_in_two(const Problem &q)
+// Packed sequences cut the one launch's chains: where its items of two chunks are one round of workgroups it then takes the
+// same time whatever the work, and two launches are ahead only up to one and a half unit-chunks a compute unit (a start in every
+// chunk, inputs from memory: 40 x 8 46.4 / 44.2, 192 x 2 42.9 / 39.6, 80 x 5 45.8 / 47.2, 40 x 10 47.7 / 54.0, 72 x 6 44.7 / 50.5,
+// 40 x 12 48.5 / 60.0; dstate 64 40 x 10 37.9 / 40.3; two rounds: 160 x 3 55.0 / 46.4, 80 x 8 74.8 / 62.6, 160 x 6 76.7 / 77.7).
+inline bool scan_in_two(const Problem &q, bool packed)
 {
+    if (packed && q.units * ceil_div(q.chunks, 2) <= q.n_cu && 2 * q.units * q.chunks > 3 * (int64_t)q.n_cu) return false;
     if (q.chunks > 8) return q.chunks <= 16 && q.units <= 48;
     return q.units <= 160 || (q.units <= 320 && q.units * q.chunks <= 960);
 }

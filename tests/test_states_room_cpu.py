@@ -90,3 +90,13 @@ def test_sizes_off_the_bf16_tilings_are_not_the_row_kernels():
             assert ops.fused_plan(b, L, H, P, 128, 1, Q, workspace=workspace, compute_units=256)["rows"] == 0
     assert _wants(L=4096, H=8, P=48) and _wants(L=8192, H=2, Q=384) and _wants(b=2, L=4096, H=16, P=80, Q=128)
     assert _wants(b=2, L=2048, H=24, init=torch.empty(2 * 24 * 64 * 128 + 1)[1:].view(2, 24, 64, 128))
+
+
+@pytest.mark.parametrize("H,chunks,packed,two", [
+    (80, 8, True, True), (80, 8, False, True), (80, 9, True, True), (80, 10, True, False), (80, 10, False, True),      # one round: 1.5 unit-chunks a unit
+    (160, 4, True, True), (160, 5, True, False), (160, 6, True, False), (160, 6, False, True), (96, 9, True, False), (80, 12, True, False),
+    (80, 13, True, True), (160, 8, True, True), (96, 12, True, True), (96, 12, False, True), (104, 12, False, False),  # two rounds
+])
+def test_scan_without_passed_states_in_two_launches(H, chunks, packed, two):
+    seq = torch.zeros(1, 256 * chunks, dtype=torch.int32) if packed else None
+    assert _wants(L=256 * chunks, H=H, out=None, seq=seq) == two
