@@ -271,5 +271,31 @@ inline bool scan_in_two(const Problem &q, bool packed)
     return q.units <= 160 || (q.units <= 320 && q.units * q.chunks <= 960);
 }
 
+// Chunk states of the sizes and types that the bf16 kernels do not take (ssd_generic.hip): a wave per tile or a quarter of a chunk per
+// wave, and whether the operands enter as bf16 parts.  a x sv: elements per lane of the largest tile (of 16 a x 16 sv); tiles: 64 x
+// 64 tiles per compute unit, all chunks counted.
+struct GenericWay { bool quarters, parts; };
+
+inline GenericWay generic_way(int Q, int a, int sv, bool two_bytes, int dstate, double tiles)
+{
+    const bool largest = a == 4 && sv == 4, square3 = a == 3 && sv == 3;
+    if (a > 1 && sv > 1) {
+        if (Q <= 64) return {false, two_bytes && Q == 64 && a * sv >= 8 && !square3};
+        bool wave = false;
+        if (tiles >= 24)
+            wave = two_bytes ? (a * sv >= 8 && !square3) || Q >= 128 : Q >= (largest ? 100 : 256) && a * sv >= 9;
+        else if (tiles >= 8)
+            wave = a * sv >= (two_bytes ? 8 : 9);
+        else if (tiles >= (two_bytes && largest ? 3 : 4))
+            wave = Q <= 160 && a * sv >= 12;
+        if (wave) return {false, true};
+        if (tiles < 24) {
+            const bool even = a != 3 && sv != 3;
+            if (two_bytes ? (largest && Q >= 100) || (even && a * sv >= 8 && Q >= 256) : largest && dstate > 64 && Q >= 256) return {true, true};
+        }
+    }
+    return {Q > 64 && tiles < 24, false};
+}
+
 }  // namespace cost
 }  // namespace ssd

@@ -18,10 +18,10 @@
 // vectors.  No LDS on the way in, no barrier in the loop, whole rows per load; the accumulators of one lane are S consecutive
 // columns, so rows leave as vectors as well.
 //
-// Tiles too small to repay the splitting (parts_pay) and the walk over a sequence's chunks (FUSED: one chunk, or a 16-bit out
-// without room for chunk states) keep the fp32 matrix instructions, the walk because with the parts beside the running state a
-// 64 x 64 tile leaves one wave a SIMD: fp32 instructions / parts (fp16, 8 x 3000 x 48 x 64 x 128 234 / 242 us, 8 x 102 x 76 x 128 x 128
-// 47 / 64, 8 x 2000 x 60 x 40 x 40 in chunks of 100 114 / 134).
+// Tiles and chunks too small to repay the splitting (PARTS, generic_way in ssd_cost.h) and the walk over a sequence's chunks (FUSED: one chunk, or
+// a 16-bit out without room for chunk states) keep the fp32 matrix instructions, the walk because with the parts beside the
+// running state a 64 x 64 tile leaves one wave a SIMD: fp32 instructions / parts (fp16, 8 x 3000 x 48 x 64 x 128 234 / 242 us,
+// 8 x 102 x 76 x 128 x 128 47 / 64, 8 x 2000 x 60 x 40 x 40 in chunks of 100 114 / 134).
 //
 // One workgroup owns a (16 A) x (16 S) tile of one (batch, head) and chunk; its SPLIT = 4 waves take a quarter of the
 // chunk's tokens each and add up through LDS, after which wave v holds accumulator q = v of every instruction.  In
@@ -31,6 +31,7 @@
 // neighbours also compute.  Both store them, the same bits: a sum's order does not depend on the wave or lane that forms it.
 //
 // Reference semantics: kernels/ssd_chunk_state.py:97-173, kernels/ssd_state_passing.py:27-84.
+#include "ssd_cost.h"
 #include "ssd_tile.h"
 
 namespace ssd {
@@ -127,18 +128,7 @@ __device__ __forceinline__ void split(const float (&v)[8], bf16x8 (&parts)[PARTS
 }
 // parts of an element of B: a bf16 is one, an f16 two, an fp32 three
 template <typename T> constexpr int kBParts = sizeof(T) == 4 ? 3 : std::is_same<T, _Float16>::value ? 2 : 1;
-// Whether a tile of A x S products per element pair repays the splitting of A + S operands.  Chunk states, fp32 instructions / parts,
-// us: 8 x 3680 tokens x 12 heads, chunk 64 or 100, bf16, 16 x 96 23.2 / 24.9, 40 x 24 22.6 / 18.6, 48 x 40 25.6 / 21.8; fp32, 16 x 96
-// 21.6 / 24.3, 48 x 24 17.7 / 18.9, 48 x 40 26.2 / 21.3; 2 x 1900 x 8, chunk 100, a quarter a wave, fp32, 96 x 40 9.9 / 11.9, fp16, 48 x
-// 96 10.4 / 11.3, bf16, 80 x 96 14.4 / 15.8.  One column block: 8 x 7360 x 12 x 40 x 16, bf16, fused 50 / 56.
-template <int A, int S, typename T, int SPLIT>
-constexpr bool parts_pay()
-{
-    if (A == 1 || S == 1) return false;
-    return SPLIT == 1 ? sizeof(T) != 4 || S > 2 : A != 3 && S != 3;
-}
-
-template <int A, int S, typename T, int SPLIT, bool FUSED>
+template <int A, int S, typename T, int SPLIT, bool FUSED, bool PARTS>
 __global__ void __launch_bounds__(64 * kWaves, 2) generic_kernel(const Params p)
 {
     // partial tiles: accumulator q of the wave that owns it, from each of the three others
@@ -208,7 +198,7 @@ __global__ void __launch_bounds__(64 * kWaves, 2) generic_kernel(const Params p)
 #pragma unroll
             for (int s = 0; s < S; ++s) acc[r][s] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-        if constexpr (FUSED || !parts_pay<A, S, T, SPLIT>()) {
+        if constexpr (!PARTS) {
         // fp32 matrix instructions, steps of four tokens, one per lane group
         for (int w0 = k_begin; w0 < k_end; w0 += kWindow) {
             const int steps = (min(kWindow, k_end - w0) + 3) >> 2;
@@ -445,15 +435,25 @@ __global__ void __launch_bounds__(64 * kWaves, 2) generic_kernel(const Params p)
     }
 }
 
-struct Shape { int a, sv, split; int64_t grid; };
+struct Shape { int a, sv, split; bool parts; int64_t grid; };
 
 template <int A, int S, typename T>
 hipError_t launch(const Params &p, bool fused, const Shape &k, hipStream_t s)
 {
     const dim3 grid((unsigned)k.grid), block(64 * kWaves);
-    if (fused) hipLaunchKernelGGL((generic_kernel<A, S, T, kWaves, true>), grid, block, 0, s, p);
-    else if (k.split == 1) hipLaunchKernelGGL((generic_kernel<A, S, T, 1, false>), grid, block, 0, s, p);
-    else hipLaunchKernelGGL((generic_kernel<A, S, T, kWaves, false>), grid, block, 0, s, p);
+    if (fused) {
+        hipLaunchKernelGGL((generic_kernel<A, S, T, kWaves, true, false>), grid, block, 0, s, p);
+        return hipGetLastError();
+    }
+    if constexpr (A > 1 && S > 1) {
+        if (k.parts) {
+            if (k.split == 1) hipLaunchKernelGGL((generic_kernel<A, S, T, 1, false, true>), grid, block, 0, s, p);
+            else hipLaunchKernelGGL((generic_kernel<A, S, T, kWaves, false, true>), grid, block, 0, s, p);
+            return hipGetLastError();
+        }
+    }
+    if (k.split == 1) hipLaunchKernelGGL((generic_kernel<A, S, T, 1, false, false>), grid, block, 0, s, p);
+    else hipLaunchKernelGGL((generic_kernel<A, S, T, kWaves, false, false>), grid, block, 0, s, p);
     return hipGetLastError();
 }
 
@@ -488,32 +488,25 @@ int per_lane(int size, int cap)
 hipError_t launch_generic(const Params &p_in, bool fused, hipStream_t s)
 {
     Params p = p_in;
-    generic::Shape k{1, 1, generic::kWaves, 0};
+    generic::Shape k{1, 1, generic::kWaves, false, 0};
     int64_t items = 0;
     const int64_t n_cu = p.n_cu > 0 ? p.n_cu : 256;
-    // One wave per tile where a quarter of a chunk is too little (chunk 64) and where 64 x 64 tiles alone give every SIMD two
-    // waves, all there is room for: quarters / one wave, us: fp32, 3 x 15232 tokens x 8 heads x 64 x 64, chunk 128 (2.8 a SIMD)
-    // 65 / 47; 8 x 520 x 22 x 128 x 128 (2.1) 38 / 31; fp16, 8 x 3001 x 48 (9) 120 / 121; 2 x 3001 x 24 (1.1) 24 / 28;
-    // fp32, 2 x 2048 x 24 (0.75) 18.6 / 22.8.  A quarter of a chunk of 128 is one step of 32 tokens, so there from 2.5 whole tiles a
-    // compute unit, 6 that are not (2 x 1900 x 8 x 80 x 96, 4.75, 14.4 with quarters of fp32 instructions, 15.8 with one wave): fp32, 2 x 2048 x 24 (6) 23.3 / 19.6, 5357 x 8 (2.6) 14.9 / 13.9; fp16 22.3 / 18.3, 13.6 / 13.3; bf16, 2 x 3000 x 15 x
-    // 48 x 96 in chunks of 100 (7) 21.7 / 16.7; 5000 x 7 x 48 x 96 (2.2) 10.3 / 11.0; fp32, 5357 x 8 x 64 x 64 (1.3) 10.2 / 13.2.
-    const int64_t big_tiles = (int64_t)p.batch * p.nheads * p.C * ((p.headdim + 63) / 64) * ((p.dstate + 63) / 64);
-    const bool whole = p.headdim % 64 == 0 && p.dstate % 64 == 0;
-    const int cols = generic::per_lane(p.dstate, 4);
-    // Tiles of fp32 instructions are not short of work in a quarter before six waves a SIMD (bf16, 8 x 3680 x 12 x 48 x 16, chunk 128
-    // (14) 15.0 / 16.0; 8 x 3680 x 12 x 16 x 96, chunk 100 (28) 30.4 / 24.1).
-    const bool parts = generic::per_lane(p.headdim, 4) > 1 && cols > (p.dt_in == DT_F32 ? 2 : 1);
-    if (!fused && (p.Q <= 64 || big_tiles >= (parts ? 8 : 24) * n_cu || (parts && p.Q <= 128 && 2 * big_tiles >= (whole ? 5 : 12) * n_cu)))
-        k.split = 1;
-    // the largest tile (operands loaded once per 16 A x 16 S) that still gives every compute unit four waves; with one wave a
-    // tile the largest there is beyond chunks of 64 (5357 x 8 above as 64 x 32: 15.0)
+    if (!fused) {
+        const int64_t tiles = (int64_t)p.batch * p.nheads * p.C * ((p.headdim + 63) / 64) * ((p.dstate + 63) / 64);
+        const cost::GenericWay w = cost::generic_way(p.Q, generic::per_lane(p.headdim, 4), generic::per_lane(p.dstate, 4), p.dt_in != DT_F32,
+                                                     p.dstate, (double)tiles / n_cu);
+        k.split = w.quarters ? generic::kWaves : 1;
+        k.parts = w.parts;
+    }
+    // the largest tile (operands loaded once per 16 A x 16 S) that still gives every compute unit four waves; with parts, one wave a
+    // tile, the largest there is beyond chunks of 64 (5357 x 8 x 64 x 128, chunk 128, as 64 x 32: 15.0 us, 13.9)
     static const int caps[][2] = {{4, 4}, {4, 2}, {2, 2}};
     for (const auto &cap : caps) {
         k.a = generic::per_lane(p.headdim, cap[0]);
         k.sv = generic::per_lane(p.dstate, cap[1]);
         const int64_t n_pt = (p.headdim + 16 * k.a - 1) / (16 * k.a), n_nt = (p.dstate + 16 * k.sv - 1) / (16 * k.sv);
         items = (int64_t)p.batch * p.nheads * n_pt * n_nt * (fused ? 1 : p.C);
-        if (items * k.split >= n_cu * generic::kWaves || (k.split == 1 && p.Q > 64)) break;
+        if (items * k.split >= n_cu * generic::kWaves || (k.parts && k.split == 1 && p.Q > 64)) break;
     }
     if (items <= 0) return hipSuccess;
     if (items > 0x7fffffffLL - 64) return hipErrorInvalidValue;
