@@ -21,6 +21,8 @@
 // global side, and the operand reads (16 lanes = 16 rows, same piece) then touch 16 different bank groups.
 #include "ssd_tile.h"
 
+#include <algorithm>
+
 namespace ssd {
 
 namespace scan {
@@ -496,10 +498,10 @@ __device__ __forceinline__ float element(const Raw<2> &r, int j, bool bf)
 // for itself: 5609 and 4773 us.
 // CB, SB: bytes of an element of C and of the states; which 16-bit type is uniform.
 template <int CB, int SB, int PB, int MB>
-__global__ void __launch_bounds__(256, 2) scan_states_any_kernel(const ScanParams p, int token_tiles, int row_tiles, int64_t items)
+__global__ void __launch_bounds__(256, 2) scan_states_any_kernel(const ScanParams p, int token_tiles, int row_tiles, int64_t first_item, int64_t items)
 {
     const int lane = threadIdx.x & 63, i16 = lane & 15, kg = lane >> 4;
-    int64_t item = (int64_t)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    int64_t item = first_item + (int64_t)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     if (item >= items) return;
     const int tt = (int)(item % token_tiles); item /= token_tiles;
     const int pt = (int)(item % row_tiles); item /= row_tiles;
@@ -693,11 +695,17 @@ static hipError_t launch_scan_any_k(const ScanParams &p, int row_tiles, hipStrea
     const int64_t units = (int64_t)p.batch * p.C * p.nheads * row_tiles;
     const bool small = units * ((p.Q + 63) / 64) < 1024;
     const int tiles = small ? (p.Q + 15) / 16 : (p.Q + 63) / 64;
-    const int64_t items = units * tiles, blocks = (items + 3) / 4;
-    if (blocks > 0x7fffffffLL) return hipErrorInvalidValue;
-    if (small) hipLaunchKernelGGL((scan::scan_states_any_kernel<CB, SB, PB, 1>), dim3((unsigned)blocks), dim3(256), 0, s, p, tiles, row_tiles, items);
-    else hipLaunchKernelGGL((scan::scan_states_any_kernel<CB, SB, PB, 4>), dim3((unsigned)blocks), dim3(256), 0, s, p, tiles, row_tiles, items);
-    return hipGetLastError();
+    const int64_t items = units * tiles;
+    // a launch holds fewer than 2^32 threads: short chunks of many heads (chunk 1, 2^20 tokens x 64 heads) are more waves than that
+    constexpr int64_t kMostBlocks = 1 << 23;
+    for (int64_t first = 0; first < items; first += 4 * kMostBlocks) {
+        const dim3 grid((unsigned)std::min((items - first + 3) / 4, kMostBlocks));
+        if (small) hipLaunchKernelGGL((scan::scan_states_any_kernel<CB, SB, PB, 1>), grid, dim3(256), 0, s, p, tiles, row_tiles, first, items);
+        else hipLaunchKernelGGL((scan::scan_states_any_kernel<CB, SB, PB, 4>), grid, dim3(256), 0, s, p, tiles, row_tiles, first, items);
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return e;
+    }
+    return hipSuccess;
 }
 
 template <int CB, int SB>

@@ -48,3 +48,15 @@ def test_scan_any(ops, oracle, c_type, s_type, b, L, H, P, N, G, Q, nseq):
     assert torch.equal(yv, y + 0.5) and bool((out[..., 0] == 0.5).all())
     for dtype in (torch.float16, torch.bfloat16):
         assert torch.equal(ops._chunk_scan_states_fwd(mv(C), mv(prev), mv(dA), seq_idx=mv(seq), out_dtype=dtype), y.to(dtype))
+
+
+def test_more_waves_than_one_launch_holds(ops):
+    # chunks of one token: a wave per (token, head), 2^26 of them and some; the state that enters a chunk is its only factor
+    L, H = (1 << 20) + 3, 64
+    g = torch.Generator(device="cuda").manual_seed(5)
+    C = torch.randn(1, L, 1, 1, generator=g, device="cuda")
+    prev = torch.randn(1, L, H, 1, 1, generator=g, device="cuda")
+    dA = torch.zeros(1, H, L, 1, device="cuda")
+    print("[scan any] 2^26 waves", flush=True)
+    y = ops._chunk_scan_states_fwd(C, prev, dA)
+    assert torch.equal(y, C[:, :, 0, :, None] * prev[..., 0])          # one product each: rounded once
