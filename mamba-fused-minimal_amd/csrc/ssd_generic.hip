@@ -6,7 +6,7 @@
 // v_mfma_f32_16x16x32_bf16 multiplies all pairs of parts but those below 2^-24 of the largest: 6, 5 or 3 instructions of 16 clocks
 // where the fp32 ones take 256.  Each adds 32 products at a time, so the sums round less often: error against 64 bits 0.58 -
 // 0.75e-7 where the fp32 instructions left 0.66 - 1.3e-7 (fp32, fp16 and odd sizes, fast and slow decays).  Where a sum is not finite
-// (an infinite input, or one that rounds to an infinite bf16) the fp32 instructions do the wave's tokens again.
+// (an infinite input, or one too large for its parts, kLift) the fp32 instructions do the wave's tokens again.
 //
 // What bounds it: the vector instructions that split the operands -- 6 to 8 per element, about as many clocks as the matrix
 // instructions take, and the two hardly overlap on a SIMD --, and for small calls a wave's start and the adding up at the end.
@@ -28,7 +28,8 @@
 // fused mode it walks the chunks with the state in registers.  Short chunks leave a quarter too little to do between
 // a wave's start and the adding up: there a wave owns a tile by itself (SPLIT = 1).  Rows and columns past the edge of an
 // odd headdim or dstate are not loaded: the last lanes' vectors move up to end at the edge and repeat rows that their
-// neighbours also compute.  Both store them, the same bits: a sum's order does not depend on the wave or lane that forms it.
+// neighbours also compute.  Both store them, the same bits: a sum's order does not depend on the wave or lane that forms it.  (Not
+// where only one of the two has done its tokens again in fp32: either sum is then stored, both with the accuracy stated above.)
 //
 // Reference semantics: kernels/ssd_chunk_state.py:97-173, kernels/ssd_state_passing.py:27-84.
 #include "ssd_cost.h"
@@ -128,6 +129,11 @@ __device__ __forceinline__ void split(const float (&v)[8], bf16x8 (&parts)[PARTS
 }
 // parts of an element of B: a bf16 is one, an f16 two, an fp32 three
 template <typename T> constexpr int kBParts = sizeof(T) == 4 ? 3 : std::is_same<T, _Float16>::value ? 2 : 1;
+// Three parts hold 24 bits only down to 2^-109, below that the last one is subnormal: x * w and an fp32 B are split 2^24 times as
+// large, which reaches down to the smallest normal fp32 value, and the sums are scaled back.
+constexpr float kLift = 0x1p24f;
+template <typename T> constexpr float kBLift = kBParts<T> == 3 ? kLift : 1.f;
+
 template <int A, int S, typename T, int SPLIT, bool FUSED, bool PARTS>
 __global__ void __launch_bounds__(64 * kWaves, 2) generic_kernel(const Params p)
 {
@@ -304,7 +310,7 @@ __global__ void __launch_bounds__(64 * kWaves, 2) generic_kernel(const Params p)
         float w = 0.f;
         for (int st = 0; st < steps; ++st) {
             if ((st & 1) == 0) {
-                w = weight(st >> 1);
+                w = kLift * weight(st >> 1);
                 load_weights((st >> 1) + 1);
             }
             const int next = min(st + 1, steps - 1);      // behind the last step: that one again, not used
@@ -318,6 +324,9 @@ __global__ void __launch_bounds__(64 * kWaves, 2) generic_kernel(const Params p)
             static_for<S>([&](auto s) {
                 float v[8];
                 columns(s, v);
+                if constexpr (kBLift<T> != 1.f)
+#pragma unroll
+                    for (int t = 0; t < 8; ++t) v[t] *= kBLift<T>;
                 bf16x8 bp[kBParts<T>];
                 split<kBParts<T>>(v, bp);
                 if constexpr (s.value == S - 1) load_B(next);
@@ -329,15 +338,18 @@ __global__ void __launch_bounds__(64 * kWaves, 2) generic_kernel(const Params p)
                         for (int r = 0; r < A; ++r) acc[r][s.value] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xp[r][u], bp[q], acc[r][s.value], 0, 0, 0);
             });
         }
-        // An infinite value, or one that rounds to an infinite bf16, leaves NaN in its rest, and so does one in the place of a token
-        // past the end: where a sum is not finite this wave's tokens are added up once more by the fp32 instructions.
+        // An infinite value, or one that is infinite 2^24 times as large or as a bf16, leaves NaN in its rest, and so does one in the place
+        // of a token past the end: where a sum is not finite this wave's tokens are added up once more by the fp32 instructions.
         bool finite = true;
 #pragma unroll
         for (int r = 0; r < A; ++r)
 #pragma unroll
             for (int s = 0; s < S; ++s)
 #pragma unroll
-                for (int q = 0; q < 4; ++q) finite &= __builtin_fabsf(acc[r][s][q]) < __builtin_inff();
+                for (int q = 0; q < 4; ++q) {
+                    finite &= __builtin_fabsf(acc[r][s][q]) < __builtin_inff();
+                    acc[r][s][q] *= 1.f / (kLift * kBLift<T>);
+                }
         if (!__all(finite)) {
 #pragma unroll
             for (int r = 0; r < A; ++r)

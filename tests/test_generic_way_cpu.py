@@ -87,3 +87,11 @@ def test_without_parts_the_fp32_instructions_go_as_they_did(way):
     # one wave a tile in chunks up to 64 and from 24 tiles on, quarters elsewhere
     assert way([("fp32", 40, 40, Q, t) for Q, t in ((32, 1), (64, 30), (65, 1), (100, 23.9), (100, 24))]) == [(0, 0), (0, 0), (1, 0), (0, 1), (0, 0)]
     assert way([("fp16", 16, 128, Q, t) for Q, t in ((64, 3), (128, 12), (256, 30))]) == [(0, 0), (1, 0), (0, 0)]      # one row block
+
+
+def test_sizes_that_are_tested_with_parts_run_them(way):
+    # headdim, dstate, chunk and 64 x 64 tiles over 256 compute units of tests/test_gpu_split_products.py -> (quarters, parts)
+    fp32 = [(64, 128, 257, 70 * 3 * 2), (64, 128, 257, 33 * 2 * 2), (63, 127, 257, 2 * 2 * 2), (64, 128, 100, 80 * 7 * 2), (48, 63, 100, 90 * 13), (48, 40, 100, 90 * 23)]
+    two = [(64, 64, 257, 90 * 3), (31, 63, 257, 2 * 2), (64, 63, 64, 100 * 11), (32, 63, 100, 90 * 23), (64, 63, 100, 110 * 7)]
+    assert way([("fp32", P, N, Q, t / 256) for P, N, Q, t in fp32]) == [(1, 1), (1, 1), (1, 1), (0, 1), (0, 1), (0, 1)]
+    assert way([("fp16", P, N, Q, t / 256) for P, N, Q, t in two]) == [(1, 1), (1, 1), (0, 1), (0, 1), (0, 1)]

@@ -63,3 +63,29 @@ def test_what_is_not_finite_stays_where_it_is(ops, dtype):
         x, B = torch.full((1, 1, 1, 2), 3.4e38), torch.full((1, 1, 1, 2), 0.5)
         one = ops._chunk_state_fwd(B.cuda(), x.cuda(), torch.ones(1, 1, 1, 1, device="cuda"), torch.zeros(1, 1, 1, 1, device="cuda"))
         torch.testing.assert_close(one.cpu(), torch.full((1, 1, 1, 2, 2), 1.7e38))
+
+
+# Sizes that run the products of parts (tests/test_generic_way_cpu.py holds the rule to them): tiles of 64 x 64, 64 x 32, 48 x 48 and
+# smaller ones, a quarter of a chunk or a whole one per wave, ragged last chunks, odd edges.
+PARTS_FP32 = [(515, 257, 64, 128, 70), (300, 257, 64, 128, 33), (300, 257, 63, 127, 2), (700, 100, 64, 128, 80), (1210, 100, 48, 63, 90), (2300, 100, 48, 40, 90)]
+PARTS_16 = [(515, 257, 64, 64, 90), (300, 257, 31, 63, 2), (700, 64, 64, 63, 100), (2300, 100, 32, 63, 90), (700, 100, 64, 63, 110)]
+PARTS = [(torch.float32, *v) for v in PARTS_FP32] + [(t, *v) for t in (torch.float16, torch.bfloat16) for v in PARTS_16]
+
+
+@pytest.mark.parametrize("dtype,L,Q,P,N,H", PARTS, ids=str)
+def test_every_product_of_parts_counts(ops, dtype, L, Q, P, N, H):
+    # Weights that are powers of two, so that nothing but the products and their sums rounds: measured 0.5e-7 of the norm, and 1.3e-6
+    # or more with one of the products of parts left out.  The weights reach to where a third bf16 part would be subnormal and to
+    # where the sums would be infinite on their way (the fp32 instructions then); so does an fp32 B.
+    g = torch.Generator(device="cuda").manual_seed(L + P)
+    C = -(-L // Q)
+    x = torch.randn(1, L, H, P, generator=g, device="cuda").to(dtype)
+    B = torch.randn(1, L, 1, N, generator=g, device="cuda").to(dtype)
+    dA = torch.zeros(1, H, C, Q, device="cuda")
+    for e, e_B in ((0, 0), (-118, 0), (106, 0)) + (((0, -118), (0, 106), (60, -118)) if dtype == torch.float32 else ()):
+        dt, Bs = torch.full((1, H, C, Q), 2.0 ** e, device="cuda"), B * 2.0 ** e_B
+        print(f"[parts] {dtype} {(L, Q, P, N, H)} 2^{e} 2^{e_B}", flush=True)
+        got = ops._chunk_state_fwd(Bs, x, dt, dA)
+        want = _exact(x, Bs, dt, dA, Q)
+        err = float((got.double() - want).norm() / want.norm())
+        assert err < 4e-7, (e, e_B, err)
