@@ -89,3 +89,24 @@ def test_every_product_of_parts_counts(ops, dtype, L, Q, P, N, H):
         want = _exact(x, Bs, dt, dA, Q)
         err = float((got.double() - want).norm() / want.norm())
         assert err < 4e-7, (e, e_B, err)
+
+
+@pytest.mark.parametrize("dtype,L,Q,P,N,H", PARTS, ids=str)
+def test_what_is_not_finite_stays_where_it_is_on_every_tile(ops, dtype, L, Q, P, N, H):
+    g = torch.Generator(device="cuda").manual_seed(L + P)
+    C = -(-L // Q)
+    x = torch.randn(1, L, H, P, generator=g, device="cuda").to(dtype)
+    B = torch.randn(1, L, 1, N, generator=g, device="cuda").to(dtype)
+    dt = torch.rand(1, H, C, Q, generator=g, device="cuda") + 0.1
+    dA = -torch.rand(1, H, C, Q, generator=g, device="cuda").cumsum(-1) * 0.05
+    clean = ops._chunk_state_fwd(B, x, dt, dA)
+    last = (C - 1) * Q                                    # the last chunk's first token: what padding reads
+    x[0, last, 1, P - 1], x[0, Q - 1, 0, 3], B[0, Q // 2, 0, N - 1] = float("inf"), float("nan"), -float("inf")
+    print(f"[parts not finite] {dtype} {(L, Q, P, N, H)}", flush=True)
+    got = ops._chunk_state_fwd(B, x, dt, dA)
+    assert bool((got[0, C - 1, 1, P - 1].isinf() & (got[0, C - 1, 1, P - 1].sign() == B[0, last, 0].sign())).all())
+    assert bool(got[0, 0, 0, 3].isnan().all()) and bool(got[0, 0, 1:, :, N - 1].isinf().all())
+    for at in ((0, C - 1, 1, P - 1), (0, 0, 0, 3), (0, 0, slice(None), slice(None), N - 1)):
+        got[at] = clean[at]
+    # sums of up to Q products in two orders: Q 2^-24 of their magnitudes, which are of order one, at most
+    torch.testing.assert_close(got, clean, rtol=1e-5, atol=Q * 2.0 ** -22)
