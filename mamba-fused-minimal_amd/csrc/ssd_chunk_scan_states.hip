@@ -637,7 +637,8 @@ bool scan_states_mfma_supported(const ScanParams &p)
     // byte offsets inside one descriptor are 32-bit; the descriptors of C and y cover one chunk
     if ((int64_t)p.Q * p.sC_l * 2 >= 0x7fffffffLL || (int64_t)p.Q * p.so_l * (p.dt_out == DT_F32 ? 4 : 2) >= 0x7fffffffLL) return false;
     if ((int64_t)p.headdim * p.sst_p * 4 >= 0x7fffffffLL) return false;
-    return (int64_t)p.batch * p.C * p.nheads * (p.headdim / 32) < 0x7fffffffLL;
+    // one launch of 256 threads a workgroup: fewer than 2^32 of them
+    return (int64_t)p.batch * p.C * p.nheads * (p.headdim / (p.headdim % 64 == 0 ? 64 : 32)) < (1 << 24);
 }
 
 template <int NK, int PB, int MB, bool PLAIN, bool S16 = false>

@@ -35,6 +35,8 @@
 #include "ssd_cost.h"
 #include "ssd_tile.h"
 
+#include <algorithm>
+
 namespace ssd {
 namespace generic {
 
@@ -135,7 +137,7 @@ constexpr float kLift = 0x1p24f;
 template <typename T> constexpr float kBLift = kBParts<T> == 3 ? kLift : 1.f;
 
 template <int A, int S, typename T, int SPLIT, bool FUSED, bool PARTS>
-__global__ void __launch_bounds__(64 * kWaves, 2) generic_kernel(const Params p)
+__global__ void __launch_bounds__(64 * kWaves, 2) generic_kernel(const Params p, int first_group)
 {
     // partial tiles: accumulator q of the wave that owns it, from each of the three others
     constexpr int SV = S == 3 ? 4 : S;
@@ -149,7 +151,7 @@ __global__ void __launch_bounds__(64 * kWaves, 2) generic_kernel(const Params p)
     // Consecutive workgroups land on consecutive XCDs: give each XCD a contiguous run of tiles, so that the tiles that
     // share x (the column tiles of a head) and B (the heads of a group) share an L2.
     const int per_xcd = gridDim.x >> 3;
-    int item = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
+    int item = first_group + (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
     if (SPLIT == 1) item = item * kWaves + wv;
     if (item >= p.n_items) return;
     const int n_pt = (p.headdim + 16 * A - 1) / (16 * A), n_nt = (p.dstate + 16 * S - 1) / (16 * S);
@@ -449,24 +451,28 @@ __global__ void __launch_bounds__(64 * kWaves, 2) generic_kernel(const Params p)
 
 struct Shape { int a, sv, split; bool parts; int64_t grid; };
 
+// A launch holds fewer than 2^32 threads: short chunks of many heads (chunk 1, 2^20 tokens x 64 heads) are more workgroups than that.
+constexpr int64_t kMostGroups = 1 << 23;
+
+template <int A, int S, typename T, int SPLIT, bool FUSED, bool PARTS>
+hipError_t launch_k(const Params &p, const Shape &k, hipStream_t s)
+{
+    for (int64_t first = 0; first < k.grid; first += kMostGroups) {
+        const dim3 grid((unsigned)std::min(k.grid - first, kMostGroups));
+        hipLaunchKernelGGL((generic_kernel<A, S, T, SPLIT, FUSED, PARTS>), grid, dim3(64 * kWaves), 0, s, p, (int)first);
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return e;
+    }
+    return hipSuccess;
+}
+
 template <int A, int S, typename T>
 hipError_t launch(const Params &p, bool fused, const Shape &k, hipStream_t s)
 {
-    const dim3 grid((unsigned)k.grid), block(64 * kWaves);
-    if (fused) {
-        hipLaunchKernelGGL((generic_kernel<A, S, T, kWaves, true, false>), grid, block, 0, s, p);
-        return hipGetLastError();
-    }
-    if constexpr (A > 1 && S > 1) {
-        if (k.parts) {
-            if (k.split == 1) hipLaunchKernelGGL((generic_kernel<A, S, T, 1, false, true>), grid, block, 0, s, p);
-            else hipLaunchKernelGGL((generic_kernel<A, S, T, kWaves, false, true>), grid, block, 0, s, p);
-            return hipGetLastError();
-        }
-    }
-    if (k.split == 1) hipLaunchKernelGGL((generic_kernel<A, S, T, 1, false, false>), grid, block, 0, s, p);
-    else hipLaunchKernelGGL((generic_kernel<A, S, T, kWaves, false, false>), grid, block, 0, s, p);
-    return hipGetLastError();
+    if (fused) return launch_k<A, S, T, kWaves, true, false>(p, k, s);
+    if constexpr (A > 1 && S > 1)
+        if (k.parts) return k.split == 1 ? launch_k<A, S, T, 1, false, true>(p, k, s) : launch_k<A, S, T, kWaves, false, true>(p, k, s);
+    return k.split == 1 ? launch_k<A, S, T, 1, false, false>(p, k, s) : launch_k<A, S, T, kWaves, false, false>(p, k, s);
 }
 
 template <int A, int S>

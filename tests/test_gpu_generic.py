@@ -115,3 +115,13 @@ def test_a_row_does_not_depend_on_where_it_lies(ops, oracle, kw):
     for out, fin in calls:
         assert same(out) and same(fin)
     assert torch.equal(calls[1][0], calls[2][0]) and torch.equal(calls[1][1], calls[2][1])
+
+
+def test_more_workgroups_than_one_launch_holds(ops):
+    # chunks of one token: a tile per (token, head), four to a workgroup, 2^26 of them and some; one product each, rounded once
+    L, H = (1 << 20) + 3, 64
+    g = torch.Generator(device="cuda").manual_seed(5)
+    x, B = torch.randn(1, L, H, 1, generator=g, device="cuda"), torch.randn(1, L, 1, 1, generator=g, device="cuda")
+    dt, dA = torch.ones(1, H, L, 1, device="cuda"), torch.zeros(1, H, L, 1, device="cuda")
+    print("[generic] 2^26 tiles", flush=True)
+    assert torch.equal(ops._chunk_state_fwd(B, x, dt, dA)[..., 0], x * B)
