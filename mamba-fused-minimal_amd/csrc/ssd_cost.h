@@ -272,29 +272,46 @@ inline bool scan_in_two(const Problem &q, bool packed)
 }
 
 // Chunk states of the sizes and types that the bf16 kernels do not take (ssd_generic.hip): a wave per tile or a quarter of a chunk per
-// wave, and whether the operands enter as bf16 parts.  a x sv: elements per lane of the largest tile (of 16 a x 16 sv); tiles: 64 x
-// 64 tiles per compute unit, all chunks counted.
+// wave, and whether the operands enter as bf16 parts.  a x sv: elements per lane of the largest tile (of 16 a x 16 sv); b_parts: of an
+// element of B (fp32 3, f16 2, bf16 1); tiles: 64 x 64 tiles per compute unit, all chunks counted.
+// Without parts: a wave per tile in chunks up to 64 and from 24 tiles on.  Parts are ahead as a wave per tile where tiles are plenty --
+// the earlier the larger the tile, which splits fewer operands per product, and the fewer parts B has --, and in quarters where a
+// chunk is long or tiles are few.  Lines through 3400 timings (18 tiles, 3 types, chunks of 64 to 256, 1/4 to 40 tiles); fp32
+// instructions / a wave per tile / quarters, us (type, headdim x dstate, chunk, tiles):
+//     fp16 64 x 64, 64, 4      16.5 / 13.9 / 20.1      bf16 48 x 96, 64, 6       13.6 / 12.8 / 19.1      fp32 64 x 64, 64, 12     28.8 / 30.0 / 51.2
+//     fp16 64 x 64, 128, 3     15.6 / 14.4 / 15.5      fp16 64 x 64, 128, 1      10.4 / 12.9 / 9.4       fp32 64 x 128, 128, 4    20.1 / 16.7 / 19.5
+//     fp16 48 x 48, 128, 4     16.4 / 16.7 / 17.0      fp16 48 x 48, 128, 8      25.3 / 20.9 / 28.9      fp32 48 x 48, 128, 8     23.3 / 23.3 / 31.9
+//     fp32 64 x 128, 256, 2    20.0 / 21.2 / 18.8      fp16 64 x 32, 256, 4      22.2 / 24.3 / 19.4      fp32 64 x 32, 128, 24    56.5 / 59.3 / 84.0
+// Of those 3400 calls 10 run more than 3 % longer than with fp32 instructions throughout, by 10 % at most (6 us at 1/4 tile).
 struct GenericWay { bool quarters, parts; };
 
-inline GenericWay generic_way(int Q, int a, int sv, bool two_bytes, int dstate, double tiles)
+inline GenericWay generic_way(int Q, int a, int sv, int b_parts, int dstate, double tiles)
 {
-    const bool largest = a == 4 && sv == 4, square3 = a == 3 && sv == 3;
-    if (a > 1 && sv > 1) {
-        if (Q <= 64) return {false, two_bytes && Q == 64 && a * sv >= 8 && !square3};
-        bool wave = false;
-        if (tiles >= 24)
-            wave = two_bytes ? (a * sv >= 8 && !square3) || Q >= 128 : Q >= (largest ? 100 : 256) && a * sv >= 9;
-        else if (tiles >= 8)
-            wave = a * sv >= (two_bytes ? 8 : 9);
-        else if (tiles >= (two_bytes && largest ? 3 : 4))
-            wave = Q <= 160 && a * sv >= 12;
-        if (wave) return {false, true};
-        if (tiles < 24) {
-            const bool even = a != 3 && sv != 3;
-            if (two_bytes ? (largest && Q >= 100) || (even && a * sv >= 8 && Q >= 256) : largest && dstate > 64 && Q >= 256) return {true, true};
-        }
+    const int m = a * sv;
+    const bool bf16 = b_parts == 1, two_bytes = b_parts < 3, largest = m == 16, longer = Q > 160;
+    const GenericWay fp32 = {Q > 64 && tiles < 24, false}, wave = {false, true}, quarters = {true, true};
+    // one row or column block splits as many operands as it has products; fp32 splits both in three
+    if (a == 1 || sv == 1 || (!two_bytes && sv == 2)) return fp32;
+    if (Q <= 64) {
+        if (Q < 64) return bf16 && largest && Q >= 32 ? wave : fp32;
+        if (bf16) return m != 6 || tiles < 16 ? wave : fp32;
+        if (two_bytes) return m >= 8 && (m != 9 || tiles < 16) ? wave : fp32;
+        return (largest && tiles >= 3.5 && tiles < 7) || (m == 9 && dstate > 64 && tiles >= 5.5 && tiles < 16) ? wave : fp32;
     }
-    return {Q > 64 && tiles < 24, false};
+    if (tiles >= 24) {      // the fp32 instructions go a wave per tile too
+        const int shortest = two_bytes && m >= 8 && m != 9 ? 65 : largest ? 100 : two_bytes || m >= 8 ? 128 : 256;
+        return Q >= shortest ? wave : fp32;
+    }
+    double first = 7;
+    if (two_bytes) first = m >= 12 ? (longer ? 5 : 2.5) : m >= 8 ? (longer ? 7 : 5) : bf16 && m == 4 && !longer ? 5.5 : 7;
+    else if (largest) first = longer ? 5.5 : 3.5;
+    else if (m == 12 || (m == 9 && Q <= 128)) first = 5.5;
+    if (tiles >= first) return wave;
+    if (!two_bytes) return largest && longer && (dstate > 64 || tiles < 2.5) ? quarters : fp32;
+    if (longer) return m >= 8 || bf16 ? quarters : fp32;
+    if (largest) return tiles >= (bf16 ? 0.75 : 1) ? quarters : fp32;
+    // a quarter of one whole step of 32 tokens
+    return Q >= 96 && Q <= 128 && tiles >= 1 && (m == 12 || (m == 8 && (bf16 || tiles < 3.5))) ? quarters : fp32;
 }
 
 }  // namespace cost

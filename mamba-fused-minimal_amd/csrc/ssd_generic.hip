@@ -511,7 +511,7 @@ hipError_t launch_generic(const Params &p_in, bool fused, hipStream_t s)
     const int64_t n_cu = p.n_cu > 0 ? p.n_cu : 256;
     if (!fused) {
         const int64_t tiles = (int64_t)p.batch * p.nheads * p.C * ((p.headdim + 63) / 64) * ((p.dstate + 63) / 64);
-        const cost::GenericWay w = cost::generic_way(p.Q, generic::per_lane(p.headdim, 4), generic::per_lane(p.dstate, 4), p.dt_in != DT_F32,
+        const cost::GenericWay w = cost::generic_way(p.Q, generic::per_lane(p.headdim, 4), generic::per_lane(p.dstate, 4), p.dt_in == DT_F32 ? 3 : p.dt_in == DT_F16 ? 2 : 1,
                                                      p.dstate, (double)tiles / n_cu);
         k.split = w.quarters ? generic::kWaves : 1;
         k.parts = w.parts;

@@ -67,7 +67,7 @@ def test_what_is_not_finite_stays_where_it_is(ops, dtype):
 
 # Sizes that run the products of parts (tests/test_generic_way_cpu.py holds the rule to them): tiles of 64 x 64, 64 x 32, 48 x 48 and
 # smaller ones, a quarter of a chunk or a whole one per wave, ragged last chunks, odd edges.
-PARTS_FP32 = [(515, 257, 64, 128, 70), (300, 257, 64, 128, 33), (300, 257, 63, 127, 2), (700, 100, 64, 128, 80), (1210, 100, 48, 63, 90), (2300, 100, 48, 40, 90)]
+PARTS_FP32 = [(515, 257, 64, 128, 70), (300, 257, 64, 128, 33), (300, 257, 63, 127, 2), (700, 100, 64, 128, 80), (1510, 100, 48, 63, 90), (2300, 100, 48, 40, 90)]
 PARTS_16 = [(515, 257, 64, 64, 90), (300, 257, 31, 63, 2), (700, 64, 64, 63, 100), (2300, 100, 32, 63, 90), (700, 100, 64, 63, 110)]
 PARTS = [(torch.float32, *v) for v in PARTS_FP32] + [(t, *v) for t in (torch.float16, torch.bfloat16) for v in PARTS_16]
 
