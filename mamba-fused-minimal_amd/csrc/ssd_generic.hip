@@ -342,17 +342,17 @@ __global__ void __launch_bounds__(64 * kWaves, 2) generic_kernel(const Params p,
         }
         // An infinite value, or one that is infinite 2^24 times as large or as a bf16, leaves NaN in its rest, and so does one in the place
         // of a token past the end: where a sum is not finite this wave's tokens are added up once more by the fp32 instructions.
-        bool finite = true;
+        float odd[4] = {0.f, 0.f, 0.f, 0.f};      // zero times every sum: NaN where one is not finite
 #pragma unroll
         for (int r = 0; r < A; ++r)
 #pragma unroll
             for (int s = 0; s < S; ++s)
 #pragma unroll
                 for (int q = 0; q < 4; ++q) {
-                    finite &= __builtin_fabsf(acc[r][s][q]) < __builtin_inff();
+                    odd[q] = __builtin_fmaf(acc[r][s][q], 0.f, odd[q]);
                     acc[r][s][q] *= 1.f / (kLift * kBLift<T>);
                 }
-        if (!__all(finite)) {
+        if (!__all(odd[0] + odd[1] + odd[2] + odd[3] == 0.f)) {
 #pragma unroll
             for (int r = 0; r < A; ++r)
 #pragma unroll
