@@ -146,7 +146,8 @@ int ssd_fused_chunk_state_passing_fwd(const ssd_tensor *x, const ssd_tensor *B, 
  * workspace: device memory, 4-byte aligned, at least ssd_fused_workspace_bytes(dims) -- with bf16 `out`: 16-byte
  * aligned and at least ssd_fused_workspace_bytes_for(dims, SSD_BF16, chunks_per_item), see below --; the call clears what it uses
  * (a small fill launch, no memset node), so the memory may hold anything and may be reused by later calls on the
- * same stream (a caller that keeps a workspace to itself can save the fill launch: `epoch` below).  Two calls whose kernels may overlap (different streams) need workspaces of their own.
+ * same stream (a caller that keeps a workspace to itself can save the fill launch: `epoch` below).  Two calls whose kernels
+ * may overlap (different streams) need workspaces of their own.
  * kernel: SSD_KERNEL_AUTO lets the library choose between this kernel and those of ssd_fused_chunk_state_passing_fwd
  * (which it runs when the shape, element types, a `states` output or too small a workspace rule the chain kernel out:
  * it needs bf16 x / B, fp32 initial / final states, fp32 or bf16 out, no `states`, dstate 64 or 128, chunk 128 or
@@ -253,8 +254,8 @@ int ssd_query_path(const ssd_tensor *x, const ssd_tensor *B, const ssd_dims *dim
 
 /*
  * Which kernel family a fused call on plain tensors of these sizes would run where the row kernel does not take it
- * (ssd_query_fused_rows), and why: the library ranks its other fused kernels by an estimate of their duration (a fit to measured times, per compute unit) and this call returns the
- * ranking.  Assumed: bf16 x / B, fp32 dt / dA_cumsum / out / final_states, contiguous, no `states` output -- the
+ * (ssd_query_fused_rows), and why: the library ranks its other fused kernels by an estimate of their duration (a fit to measured
+ * times, per compute unit) and this call returns the ranking.  Assumed: bf16 x / B, fp32 dt / dA_cumsum / out / final_states, contiguous, no `states` output -- the
  * arguments every family covers.  has_workspace != 0 asks about ssd_fused_chunk_state_passing_fwd_ws with a
  * workspace of ssd_fused_workspace_bytes(dims) and SSD_KERNEL_AUTO, 0 about ssd_fused_chunk_state_passing_fwd; no seq_idx.
  * compute_units: of the device the call would run on; 0 = 256 (MI355X).  Pure host logic: touches no device and

@@ -371,7 +371,8 @@ int chain_decision(const Params &p, const ssd_dims *dims, const ssd_fused_opts *
                          opts->workspace_bytes >= need && !(out16 && r < 2);
     // with the scan's state half asked for, the chain kernel is the only one that computes it in the same launch
     if (have_ws && ssd::chain_supported(p) &&
-        (kernel != SSD_KERNEL_AUTO || p.y || (g_forced_split.load(std::memory_order_relaxed) == 0 && !rows_preferred(p, compute_units() > 0 ? compute_units() : 256, true) &&
+        (kernel != SSD_KERNEL_AUTO || p.y ||
+         (g_forced_split.load(std::memory_order_relaxed) == 0 && !rows_preferred(p, compute_units() > 0 ? compute_units() : 256, true) &&
           chain_preferred(p, compute_units(), packed_form(p))))) {
         *use = true;
         if (opts->used_workspace) *opts->used_workspace = 1;

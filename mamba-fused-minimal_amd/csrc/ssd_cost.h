@@ -143,8 +143,8 @@ inline double rows_us(const Problem &q, int kr)
 // first (8 x 2048 x 48 heads: 66 us, the others 57).  A workgroup reads the same few columns of x to the end, so long rows
 // depend on how those columns fall on the memory channels, and a third of the workgroups finish up to a fifth late.  Up to 5120
 // tokens the kernel is ahead wherever its estimate is (rows_margin), beyond that only with four slices at dstate 128 or with chunks
-// of 128, and there in groups of 16 slices and more: below, too few workgroups share a group's B (12 x 10730).  Inputs from memory, the faster of the others
-// against this kernel, us (slices):
+// of 128, and there in groups of 16 slices and more: below, too few workgroups share a group's B (12 x 10730).  Inputs from
+// memory, the faster of the others against this kernel, us (slices):
 //     8 x 2048 x 24 heads       48.4 /  35.9 (3)      4 x 8192 x 64                   143.5 / 132.7 (4)
 //     2 x 2048 x 80             49.0 /  34.9 (3)      4 x 8192 x 80                   175.7 / 177.1 (5)   (not taken)
 //     1 x 4096 x 80             53.9 /  46.3 (2)      1 x 8192 x 80                    70.9 /  85.9 (2)   (not taken)

@@ -8,8 +8,10 @@
 // 0.75e-7 where the fp32 instructions left 0.66 - 1.3e-7 (fp32, fp16 and odd sizes, fast and slow decays).  Where a sum is not finite
 // (an infinite input, or one too large for its parts, kLift) the fp32 instructions do the wave's tokens again.
 //
-// What bounds it: the vector instructions that split the operands -- 6 to 8 per element, about as many clocks as the matrix
-// instructions take, and the two hardly overlap on a SIMD --, and for small calls a wave's start and the adding up at the end.
+// What bounds it: the vector instructions, most of them the splitting of operands.  Of a SIMD's 37.8 K clocks at 2 x 2048 x 24 heads,
+// fp32, they issue for 21.8 K, the matrix unit is busy for 9.2 K and the waves' waits overlap with little of either; fp16, 2 x 3001 x 24:
+// 30.4 K and 11.5 K of 51.8 K (hardware counters).  For small calls it is a wave's start and the adding up at the end: 2 x 1900 x 15 x 48 x
+// 96 in chunks of 64 has 1.8 waves a SIMD, vector instructions for 8.4 K and matrix instructions for 1.5 K of 23.4 K clocks.
 // Chunk states, fp32 matrix instructions / this: fp16, 2 x 3001 tokens x 24 heads x 64 x 128 31.5 / 24.3 us, 8 x 3001 x 48 188 / 120;
 // fp32, 2 x 2048 x 24 20.4 / 18.6; 1024 x 8 x 64 x 64 8.6 / 6.3.  A lane loads A consecutive headdim elements of eight tokens' x
 // rows and S consecutive dstate elements of their B rows, and its eight tokens of one row or column *are* the operand layout: lane i
@@ -18,10 +20,10 @@
 // vectors.  No LDS on the way in, no barrier in the loop, whole rows per load; the accumulators of one lane are S consecutive
 // columns, so rows leave as vectors as well.
 //
-// Tiles and chunks too small to repay the splitting (PARTS, generic_way in ssd_cost.h) and the walk over a sequence's chunks (FUSED: one chunk, or
-// a 16-bit out without room for chunk states) keep the fp32 matrix instructions, the walk because with the parts beside the
-// running state a 64 x 64 tile leaves one wave a SIMD: fp32 instructions / parts (fp16, 8 x 3000 x 48 x 64 x 128 234 / 242 us,
-// 8 x 102 x 76 x 128 x 128 47 / 64, 8 x 2000 x 60 x 40 x 40 in chunks of 100 114 / 134).
+// Tiles and chunks too small to repay the splitting (PARTS, generic_way in ssd_cost.h) and the walk over a sequence's chunks
+// (FUSED: one chunk, or a 16-bit out without room for chunk states) keep the fp32 matrix instructions, the walk because with the
+// parts beside the running state a 64 x 64 tile leaves one wave a SIMD: fp32 instructions / parts (fp16, 8 x 3000 x 48 x 64 x 128
+// 234 / 242 us, 8 x 102 x 76 x 128 x 128 47 / 64, 8 x 2000 x 60 x 40 x 40 in chunks of 100 114 / 134).
 //
 // One workgroup owns a (16 A) x (16 S) tile of one (batch, head) and chunk; its SPLIT = 4 waves take a quarter of the
 // chunk's tokens each and add up through LDS, after which wave v holds accumulator q = v of every instruction.  In
@@ -511,7 +513,8 @@ hipError_t launch_generic(const Params &p_in, bool fused, hipStream_t s)
     const int64_t n_cu = p.n_cu > 0 ? p.n_cu : 256;
     if (!fused) {
         const int64_t tiles = (int64_t)p.batch * p.nheads * p.C * ((p.headdim + 63) / 64) * ((p.dstate + 63) / 64);
-        const cost::GenericWay w = cost::generic_way(p.Q, generic::per_lane(p.headdim, 4), generic::per_lane(p.dstate, 4), p.dt_in == DT_F32 ? 3 : p.dt_in == DT_F16 ? 2 : 1,
+        const int b_parts = p.dt_in == DT_F32 ? 3 : p.dt_in == DT_F16 ? 2 : 1;
+        const cost::GenericWay w = cost::generic_way(p.Q, generic::per_lane(p.headdim, 4), generic::per_lane(p.dstate, 4), b_parts,
                                                      p.dstate, (double)tiles / n_cu);
         k.split = w.quarters ? generic::kWaves : 1;
         k.parts = w.parts;

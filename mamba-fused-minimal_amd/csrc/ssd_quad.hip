@@ -92,8 +92,9 @@ __global__ void __launch_bounds__(256, 2) quad_kernel(const Params p)
     char *stage = lds + kRing * NT * 1024 + 4 * wave_lds<NT, SPC>() + wave * kStage;
 
     // Workgroup -> (batch, group) and four of its state tiles; where a group's tiles are no multiple of four (chunk states
-    // only), the last workgroup's waves without a tile compute the last one again and store nothing.  Consecutive workgroups sit on the same XCD (workgroups are dealt round-robin over the p.n_xcd XCDs), so
-    // a batch's B is fetched from HBM by one or two L2 slices only.
+    // only), the last workgroup's waves without a tile compute the last one again and store nothing.  Consecutive workgroups sit
+    // on the same XCD (workgroups are dealt round-robin over the p.n_xcd XCDs), so a batch's B is fetched from HBM by one or two
+    // L2 slices only.
     const int n_pt = p.headdim >> 5, tiles = (p.nheads / p.ngroups) * n_pt, wpg = (tiles + 3) >> 2;
     const int n_wg = p.batch * p.ngroups * wpg, n_seg = CO ? p.n_seg : 1;
     const int per_xcd = (n_wg * n_seg + p.n_xcd - 1) / p.n_xcd;          // workgroups per XCD

@@ -20,8 +20,10 @@
 // Measured (inputs from memory, before / with this kernel): 8 x 2048 x 24 heads 48.4 / 35.3 us, 2048 x 80 heads 29.0 / 26.2,
 // 8 x 2048 x 24 in chunks of 128 64.9 / 42.7.  What bounds it: the rows of x that a workgroup reads are narrow (160 bytes of a
 // 10 KB token row with five slices), and it reads the same columns to the end: 4.0 - 4.6 TB/s of the 5.5 that wider, moving
-// requests reach (the loads alone 84 us of 177 at 4 x 8192 x 80), and a workgroup on a busy memory channel finishes last.  With
-// two slices it is the vector-memory path of the compute unit: 64 KB of B for 16 KB of x, at 25 clocks a KB, 50 a stored KB.
+// requests reach (the loads alone 84 us of 177 at 4 x 8192 x 80), and a workgroup on a busy memory channel finishes last.  No unit of a
+// compute unit is full: at 8 x 2048 x 24 (three slices) the matrix unit is busy a fifth of the launch, vector instructions issue for a
+// third, LDS instructions for a sixth, and the waves spend 43 % of their time in waits (hardware counters).  With two slices a
+// workgroup loads 64 KB of B for 16 KB of x: at 2048 x 80, on the 160 compute units that have one, the same shares are a fifth, a third, a sixth and 45 %.
 //
 // Reference semantics: kernels/ssd_chunk_state.py:97-173, kernels/ssd_state_passing.py:27-84,
 // kernels/fused_globalbar.py:16-198 (same math, one launch).

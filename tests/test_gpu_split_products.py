@@ -39,7 +39,8 @@ def test_error_is_that_of_fp32_sums(ops, dtype, L, Q, P, N, H):
         x, B = make(1, L, H, P), make(1, L, 1, N)
         got = ops._chunk_state_fwd(B.cuda(), x.cuda(), dt.cuda(), dA.cuda())
         want = _exact(x, B, dt, dA, Q)
-        # weights and products rounded to fp32 (exp's argument included: |dA| up to 7), L sums of them
+        # weights and products rounded to fp32 (exp's argument included: |dA| up to 7), L sums of them; too wide to see a product of
+        # parts left out, which is test_every_product_of_parts_counts
         bound = torch.matmul(x.double().abs().permute(0, 2, 3, 1), B.double().abs().transpose(1, 2).contiguous()).amax()
         err = (got.double().cpu() - want)
         assert float(err.norm() / want.norm()) < 4e-6 and float(err.abs().amax()) <= 2e-5 * float(bound)
